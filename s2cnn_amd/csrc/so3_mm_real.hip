@@ -1,5 +1,5 @@
 // Block-diagonal REAL products over the (2l+1)x(2l+1) blocks of an SO(3) spectrum held in the real
-// basis (see so3_real_basis.hip), on the fp32 matrix cores of gfx950 (v_mfma_f32_32x32x2_f32).
+// basis (see so3_real_basis.hip), on the bf16 matrix cores of gfx950 with float32 operands and results.
 //
 // The spectrum of a real signal on SO(3) obeys x[l,-m,-n] = (-1)^(m-n) conj(x[l,m,n]); a fixed unitary
 // change of basis per degree turns every such block into a real matrix, and the complex product
@@ -12,31 +12,52 @@
 // with tensors stored as [l, spectral row, spectral col, feature row, feature col] (the layout of the
 // complex product without the trailing pair).  As there, an operand is an L x L grid of dense feature
 // blocks in which either the contraction index ("K-contiguous") or the free index ("MN-contiguous") is
-// the fast one, and each tile sits in LDS in the orientation it has in memory.
+// the fast one.
 //
-// One MFMA 32x32x2 takes two contraction steps, one per half-wave; a lane reads four consecutive steps
-// at once (k = 8s + 4h .. +3) and feeds them to four consecutive MFMAs.
+// Arithmetic: every operand value is cut into three bf16 parts and six of the nine part products are summed in float32
+// (split_bf16.h).  At nl = 32, batch 16, 64 -> 64 features a product took 2.25 .. 2.35 ms with v_mfma_f32_32x32x2_f32 (77 % of
+// the float32 matrix peak) and takes 1.40 / 1.43 / 1.50 ms now (gradx, fwd, grady): 1.15 PFLOP/s of bf16 instructions, the
+// rate that a large library product in bf16 reaches on this card (its clock falls with the power the matrix cores draw), so
+// what bounds it is energy.  Errors against 64 bits fall as well (relative 2-norm 1.02e-6 -> 8.9e-7 at that size, 3.5e-7 ->
+// 2.9e-7 at 6 degrees): the products are exact and six roundings take the place of sixteen.
 //
-// Tiling.  A workgroup (4 waves) owns TM x TN = (64 NRB) x (64 NCB) outputs (NCB = 2, or 1 when the 128 x 128 tiles
+// Tiling.  A workgroup (4 waves) owns 128 x TN = 128 x (64 NCB) outputs (NCB = 2, or 1 when the 128 x 128 tiles
 // of a small problem would leave CUs without work); wave (wm, wn) takes row
 // blocks wm + 2i and column blocks wn + 2j (interleaved, so ragged tiles still split evenly).  The grid
-// lists exactly the tiles of all degrees, heaviest degree first.
-#include <type_traits>
+// lists exactly the tiles of all degrees, heaviest degree first; inside a degree in bands of 8 tile rows, and 32 consecutive
+// tiles go to one XCD, so that they share 8 + 4 operand panels in its L2 instead of fetching one panel per tile (22 degrees,
+// batch 32, 100 -> 100: 3 to 6 %; 32 degrees, 64 -> 64: 2 %; 16 and 64 tiles measured the same).
+//
+// Tried and not kept: three workgroups per CU (168 registers): 0 to 2 % slower.
 #include "common.h"
+#include "split_bf16.h"
 
 namespace {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
+using s2cnn::v16f;
+using s2cnn::SplitTile;
 
 constexpr int NRB = 2;            // 32-row blocks per wave
 constexpr int TM = 64 * NRB;
 constexpr int BSTR = 64, WSTR = 32;
 constexpr int TK = 32;            // contraction steps per LDS stage
 constexpr int NT = 256;
-constexpr int KC_LD = TK + 4;     // leading dim of a K-contiguous LDS tile: 144 B rows
+constexpr int BAND = 8;           // tiles are listed in bands of 8 rows of tiles, column after column
+constexpr int XCD_RUN = 32;       // consecutive tiles of the list that one XCD takes
 constexpr int SMALL_GRID = 512;   // workgroups that fill the chip (2 per CU)
+constexpr int SLICES_GRID = 256;  // fewer 128 x 64 tiles than this: the kernel for small problems
+constexpr int SLICES_WIDE = 400;  // as many 32 x 64 tiles: two blocks per wave of it
+constexpr unsigned OUTSIDE = 0x80000000u;   // a byte offset behind the end of every buffer: such loads return 0
 
 enum Mode { FWD = 0, GRADX = 1, GRADY = 2 };
+// How the contraction index (the flattened pair block, feature; KI features per block) is walked:
+//   DIVIDES  KI a multiple of 8 and KI, TK divide one another: an octet of steps never straddles a block and every stage
+//            starts at the same place inside a block, so a thread's offsets are fixed and a stage advances by a
+//            wave-uniform step
+//   WALK     any KI: every thread follows its own position (block, feature), in granules of GR steps (GR = 4, 2 or 1 divides
+//            KI, so a granule lies in one block)
+//   FAR      the same for operands whose degrees exceed 32-bit byte offsets
+enum Walk { DIVIDES = 0, WALK = 1, FAR = 2 };
 
 struct MmParams {
   const float* A;
@@ -54,334 +75,265 @@ template <> struct Cfg<FWD>   { static constexpr bool A_KC = true,  B_KC = false
 template <> struct Cfg<GRADX> { static constexpr bool A_KC = true,  B_KC = true,  A_MNMAJ = true,  B_MNMAJ = false, C_RMAJ = true;  };
 template <> struct Cfg<GRADY> { static constexpr bool A_KC = false, B_KC = false, A_MNMAJ = false, B_MNMAJ = false, C_RMAJ = false; };
 
-template <bool KC, int EXT> struct TileShape {
-  static constexpr int LD = KC ? KC_LD : EXT;
-  static constexpr int ELEMS = KC ? EXT * KC_LD : TK * EXT;
-};
-
 template <int VEC> struct VecT { typedef float type; };
 template <> struct VecT<2> { typedef float2 type; };
 template <> struct VecT<4> { typedef float4 type; };
 
-// One operand's tile loader: global -> registers -> LDS.  EXT = tile extent along the free index,
-// VEC = floats per access.  The contraction index is the flattened pair (block kb, feature kin): a stage
-// takes the next TK values of it whatever the block size, so small blocks (a batch of 16 in grad y) fill
-// whole stages and odd block sizes pad only the very last stage.  load() fetches the current stage and
-// steps to the next one.
-//
-// FAST: the block size KI along the contraction and the stage length TK divide one another, so every stage
-// starts at the same position inside a block for every thread.  Then the per-thread offsets are fixed at
-// init, the stage advances by a wave-uniform step (scalar arithmetic), rows outside the matrix are clamped
-// to a valid row (their products land in accumulators that are never stored) and only a ragged LAST stage
-// (TK a multiple of KI, odd number of blocks) is masked: the loop body is loads and LDS writes, nothing else.
-//
-// FAST = 2: KI >= TK but not a multiple of it (100 features), KI a multiple of VEC.  A stage then starts anywhere inside
-// a block and may run over ONE block boundary.  Where the stage starts is still uniform (scalar offset, scalar
-// bookkeeping); a thread only has to know whether ITS contraction steps lie behind the boundary, which is one compare
-// with a uniform value and the (uniform) distance between the end of a block and the start of the next added to its
-// offset: the same loop body as FAST = 1 plus a compare, a select and an add per slot.
-template <bool KC, bool MNMAJ, int EXT, int VEC, int FAST>
-struct TileLoader {
-  static constexpr int NSLOT = EXT * TK / (NT * VEC);
-  static constexpr int LD = TileShape<KC, EXT>::LD;
-  static constexpr int KSTEP = NT * VEC / EXT;     // MN-contiguous: contraction steps between slots
+// One operand's loader.  A thread owns NMN rows (ROWSTEP apart) of 8 contraction steps, starting at step k0 and ADV further on with
+// every load(): an octet of a row is what a lane feeds to the matrix instruction, and what one 16-byte LDS store takes,
+// whichever index is the fast one in memory.  VEC = floats per global access, along the contraction (K-contiguous) or along
+// the rows (MN-contiguous).  Rows outside the matrix and steps behind the last block are loaded from OUTSIDE, that is as
+// zeros.
+template <bool KC, bool MNMAJ, int NMN, int ROWSTEP, int VEC, int HOW, int GR, int ADV>
+struct Loader {
+  static_assert(NMN >= 1 && (KC || VEC == 1 || (VEC <= NMN && ROWSTEP == 1)) && (HOW != DIVIDES || ADV == TK), "no such loader");
   typedef typename VecT<VEC>::type vec_t;
-  static_assert(NSLOT >= 1 && NSLOT <= 32, "tile does not fit the workgroup");
 
-  const float* base;    // start of degree l
-  int off[KC ? NSLOT : 1];
-  unsigned valid_mn;    // bit q: slot q's row is inside the matrix (KC) / bit 0 (MN-contiguous)
-  int kb, kin;          // block and feature of this thread's first contraction step in the current stage
-  int lds_off;
-  int blk_k_stride;
-  int MNI, KI, L;
-  vec_t reg[NSLOT];
-  // FAST only
-  unsigned foff[FAST ? NSLOT : 1];   // per-slot BYTE offset: row/column block, row inside it, position inside the stage
-  __amdgpu_buffer_rsrc_t rsrc;  // the operand of this degree as a buffer: scalar base, per-slot offsets in VGPRs
-  unsigned soff;                // uniform: byte offset of the current stage (scalar offset of the loads)
-  int sub, nsub, step_in, step_cross;
-  int stage_i, last_ragged;     // last_ragged: index of the one masked stage, or -1
-  unsigned tail_ok;             // bit q: slot q lies inside the matrix in that stage
-  // FAST = 2 only
-  int kin_s;                    // uniform: position inside its block at which the current stage starts
-  int kk0;                      // this thread's first contraction step inside a stage
-  unsigned cross_bytes;         // uniform: what a step behind the block boundary adds to the offset
+  float reg[NMN][8];
+  const float* base;
+  __amdgpu_buffer_rsrc_t rsrc;
+  unsigned off[NMN];            // offset of the row (DIVIDES: and of the octet): bytes, FAR: floats; OUTSIDE for no row
+  int MNI, KI, L, blk_k_stride;
+  int kb, kin, adv_b, adv_k;    // WALK, FAR: block and feature of this thread's first step; what a stage adds to them
+  unsigned soff, step_in, step_cross;   // DIVIDES: uniform byte offset of the stage and its increments
+  int sub, nsub, stage_i, last_ragged;
+  bool tail_ok;
 
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ vec_t buffer_load(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned so) {
-    if constexpr (VEC == 4) {
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)so, 0);
-      return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    } else if constexpr (VEC == 2) {
-      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)so, 0);
-      return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
-    } else {
-      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)so, 0));
-    }
-  }
-
-  __device__ __forceinline__ void init(const float* base_l, int L_, int MNI_, int KI_, int tile0) {
+  __device__ __forceinline__ void init(const float* base_l, int L_, int MNI_, int KI_, int row0, int k0) {
     base = base_l; MNI = MNI_; KI = KI_; L = L_;
-    const int t = threadIdx.x;
     const int blk_elems = MNI * KI;
     const int blk_mn_stride = (MNMAJ ? L : 1) * blk_elems;
     blk_k_stride = (MNMAJ ? 1 : L) * blk_elems;
-    if (FAST) {
-      const int unit = KC ? 1 : MNI;                       // stride of one contraction step inside a block
-      const int K = L * KI, nstage = (K + TK - 1) / TK, ktail = K - (nstage - 1) * TK;
-      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base_l), 0, 4 * L * L * MNI * KI, 0x00020000);
+    const int unit = KC ? 1 : MNI;                       // stride of one contraction step inside a block
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base_l), 0, HOW == FAR ? 0 : 4 * L * L * MNI * KI, 0x00020000);
+    kb = k0 / KI;
+    kin = k0 - kb * KI;
+    const int K = L * KI, nstage = (K + TK - 1) / TK, ktail = K - (nstage - 1) * TK;
+#pragma unroll
+    for (int q = 0; q < NMN; ++q) {
+      const int row = row0 + q * ROWSTEP;
+      const int mb = row / MNI, mi = row - mb * MNI;
+      unsigned o = (unsigned)(mb * blk_mn_stride + mi * (KC ? KI : 1));
+      if (HOW == DIVIDES) o += (unsigned)((KI >= TK ? 0 : kb) * blk_k_stride + kin * unit);
+      off[q] = row >= L * MNI ? OUTSIDE : HOW == FAR ? o : 4u * o;
+    }
+    if (HOW == DIVIDES) {
       soff = 0; sub = 0; stage_i = 0;
-      if (FAST == 2) { nsub = 1; step_in = TK * unit; step_cross = 0; kin_s = 0; cross_bytes = 4u * (unsigned)(blk_k_stride - KI * unit); }
-      else if (KI >= TK) { nsub = KI / TK; step_in = TK * unit; step_cross = blk_k_stride - (KI - TK) * unit; }
-      else { nsub = 1; step_in = 0; step_cross = (TK / KI) * blk_k_stride; }
+      if (KI >= TK) { nsub = KI / TK; step_in = 4u * TK * unit; step_cross = 4u * (unsigned)(blk_k_stride - (KI - TK) * unit); }
+      else { nsub = 1; step_in = 0; step_cross = 4u * (unsigned)(TK / KI * blk_k_stride); }
       last_ragged = ktail < TK ? nstage - 1 : -1;
-      tail_ok = 0;
-      const int last = L * MNI - 1;
-      if (KC) {
-        constexpr int TPR = TK / VEC;
-        const int kk = (t % TPR) * VEC, r0 = t / TPR;
-        const int kbl = KI >= TK ? 0 : kk / KI, kin = kk - kbl * KI;
-        lds_off = r0 * LD + kk;
-        kk0 = kk;
-#pragma unroll
-        for (int q = 0; q < NSLOT; ++q) {
-          int row = tile0 + r0 + q * (NT / TPR);
-          row = row > last ? last : row;
-          const int mb = row / MNI, mi = row - mb * MNI;
-          foff[q] = 4u * (unsigned)(mb * blk_mn_stride + mi * KI + kbl * blk_k_stride + kin);
-          if (kk < ktail) tail_ok |= 1u << q;
-        }
-      } else {
-        constexpr int TPR = EXT / VEC;
-        int mn = tile0 + (t % TPR) * VEC;
-        mn = mn > last ? 0 : mn;
-        const int kk = t / TPR;
-        lds_off = kk * LD + (t % TPR) * VEC;
-        kk0 = kk;
-        const int mb = mn / MNI, mi = mn - mb * MNI;
-#pragma unroll
-        for (int q = 0; q < NSLOT; ++q) {
-          const int k = kk + q * KSTEP;
-          const int kbl = KI >= TK ? 0 : k / KI, kin = k - kbl * KI;
-          foff[q] = 4u * (unsigned)(mb * blk_mn_stride + mi + kbl * blk_k_stride + kin * MNI);
-          if (k < ktail) tail_ok |= 1u << q;
-        }
-      }
-      return;
-    }
-    valid_mn = 0;
-    int kk;
-    if (KC) {
-      constexpr int TPR = TK / VEC;
-      kk = (t % TPR) * VEC;
-      const int r0 = t / TPR;
-      lds_off = r0 * LD + kk;
-#pragma unroll
-      for (int q = 0; q < NSLOT; ++q) {
-        const int row = tile0 + r0 + q * (NT / TPR);
-        const int mb = row / MNI, mi = row - mb * MNI;
-        off[q] = mb * blk_mn_stride + mi * KI;
-        if (row < L * MNI) valid_mn |= 1u << q;
-      }
+      tail_ok = k0 < ktail;
     } else {
-      constexpr int TPR = EXT / VEC;
-      const int mn = tile0 + (t % TPR) * VEC;
-      kk = t / TPR;
-      lds_off = kk * LD + (t % TPR) * VEC;
-      const int mb = mn / MNI, mi = mn - mb * MNI;
-      off[0] = mb * blk_mn_stride + mi;
-      if (mn < L * MNI) valid_mn = 1u;
+      adv_b = ADV / KI;
+      adv_k = ADV - adv_b * KI;
     }
-    kb = kk / KI;
-    kin = kk - kb * KI;
   }
 
-  // clamped address + select instead of a predicated load: all loads of a stage are in flight together
+  __device__ __forceinline__ vec_t fetch(unsigned o, unsigned so) const {
+    if constexpr (HOW == FAR) {
+      static_assert(HOW != FAR || VEC == 1, "operands beyond 32-bit byte offsets are read one float at a time");
+      return o == OUTSIDE ? 0.f : base[o];
+    } else if constexpr (VEC == 4) {
+      typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)o, (int)so, 0);
+      return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+    } else if constexpr (VEC == 2) {
+      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)o, (int)so, 0);
+      return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
+    } else {
+      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)o, (int)so, 0));
+    }
+  }
+
+  // the values of access (row q, step e): K-contiguous VEC steps of one row, MN-contiguous one step of VEC rows
+  __device__ __forceinline__ void put(int q, int e, vec_t v) {
+    if constexpr (VEC == 1) reg[q][e] = v;
+    else if constexpr (KC && VEC == 2) { reg[q][e] = v.x; reg[q][e + 1] = v.y; }
+    else if constexpr (KC && VEC == 4) { reg[q][e] = v.x; reg[q][e + 1] = v.y; reg[q][e + 2] = v.z; reg[q][e + 3] = v.w; }
+    else { reg[q][e] = v.x; reg[q + 1][e] = v.y; }
+  }
+
+  // fetches the current stage and steps to the next one
   __device__ __forceinline__ void load() {
-    if (FAST == 2) {
-      const int room = KI - kin_s;                     // contraction steps of this stage that still lie in the current block
-      if (stage_i == last_ragged) {
+    constexpr int QS = KC ? 1 : VEC, ES = KC ? VEC : 1;
+    if (HOW == DIVIDES) {
+      const bool ok = stage_i != last_ragged || tail_ok;
 #pragma unroll
-        for (int q = 0; q < NSLOT; ++q) {
-          const int k = KC ? kk0 : kk0 + q * KSTEP;
-          const vec_t v = buffer_load(rsrc, foff[q] + (k >= room ? cross_bytes : 0u), soff);
-          reg[q] = ((tail_ok >> q) & 1u) ? v : vec_t{};
-        }
-      } else {
+      for (int q = 0; q < NMN; q += QS) {
+        const unsigned o = ok ? off[q] : OUTSIDE;
 #pragma unroll
-        for (int q = 0; q < NSLOT; ++q) {
-          const int k = KC ? kk0 : kk0 + q * KSTEP;    // KC: a thread's VEC steps never straddle a block (KI is a multiple of VEC)
-          reg[q] = buffer_load(rsrc, foff[q] + (k >= room ? cross_bytes : 0u), soff);
-        }
+        for (int e = 0; e < 8; e += ES)
+          put(q, e, KC ? fetch(o + 4u * e, soff) : fetch(o, soff + 4u * (unsigned)(e * MNI)));
       }
       ++stage_i;
-      kin_s += TK;
-      soff += 4u * (unsigned)step_in;
-      if (kin_s >= KI) { kin_s -= KI; soff += cross_bytes; }
+      if (++sub == nsub) { sub = 0; soff += step_cross; }
+      else soff += step_in;
       return;
     }
-    if (FAST) {
-      if (stage_i == last_ragged) {
+    const unsigned scale = HOW == FAR ? 1u : 4u, unit = scale * (unsigned)(KC ? 1 : MNI), bstride = scale * (unsigned)blk_k_stride;
+    const unsigned cross = bstride - (unsigned)KI * unit;      // from behind the end of a block to the start of the next
+    int k = kin, b = kb;
+    unsigned o = (unsigned)b * bstride + (unsigned)k * unit;
 #pragma unroll
-        for (int q = 0; q < NSLOT; ++q) {
-          const bool ok = (tail_ok >> q) & 1u;
-          const vec_t v = buffer_load(rsrc, foff[q], soff);
-          reg[q] = ok ? v : vec_t{};
-        }
-      } else {
+    for (int g = 0; g < 8; g += GR) {
 #pragma unroll
-        for (int q = 0; q < NSLOT; ++q) reg[q] = buffer_load(rsrc, foff[q], soff);
+      for (int q = 0; q < NMN; q += QS) {
+        const unsigned at = b < L && (HOW != FAR || off[q] != OUTSIDE) ? off[q] + o : OUTSIDE;   // OUTSIDE + o is outside as well
+#pragma unroll
+        for (int e = 0; e < GR; e += ES)
+          put(q, g + e, KC ? fetch(at + 4u * e, 0) : fetch(at, e * unit));
       }
-      ++stage_i;
-      if (++sub == nsub) { sub = 0; soff += 4u * (unsigned)step_cross; }
-      else soff += 4u * (unsigned)step_in;
-      return;
+      k += GR;
+      o += (unsigned)GR * unit;
+      if (k >= KI) { k = 0; ++b; o += cross; }                // KI is a multiple of GR
     }
-    if (KC) {
-      const bool kvalid = kb < L;
-      const int koff = kb * blk_k_stride + kin;
-#pragma unroll
-      for (int q = 0; q < NSLOT; ++q) {
-        const bool ok = kvalid && ((valid_mn >> q) & 1u);
-        const vec_t v = *reinterpret_cast<const vec_t*>(base + (ok ? off[q] + koff : 0));
-        reg[q] = ok ? v : vec_t{};
-      }
-    } else {
-      int b = kb, k = kin;
-#pragma unroll
-      for (int q = 0; q < NSLOT; ++q) {
-        const bool ok = valid_mn && b < L;
-        const vec_t v = *reinterpret_cast<const vec_t*>(base + (ok ? b * blk_k_stride + off[0] + k * MNI : 0));
-        reg[q] = ok ? v : vec_t{};
-        k += KSTEP;
-        if (KI >= KSTEP) { if (k >= KI) { k -= KI; ++b; } }
-        else { const int w = k / KI; b += w; k -= w * KI; }
-      }
-    }
-    kin += TK;
-    if (KI >= TK) { if (kin >= KI) { kin -= KI; ++kb; } }
-    else { const int w = kin / KI; kb += w; kin -= w * KI; }
-  }
-
-  __device__ __forceinline__ void store(float* tile) const {
-    constexpr int QSTEP = KC ? NT * VEC / TK : KSTEP;   // rows (KC) or k-rows between slots
-#pragma unroll
-    for (int q = 0; q < NSLOT; ++q)
-      *reinterpret_cast<vec_t*>(tile + lds_off + q * QSTEP * LD) = reg[q];
+    kin += adv_k;
+    kb += adv_b;
+    if (kin >= KI) { kin -= KI; ++kb; }
   }
 };
 
-// the four consecutive contraction steps k0 .. k0+3 of tile row/col `idx`
-template <bool KC, int LD>
-__device__ __forceinline__ float4 fetch_operand(const float* tile, int idx, int k0) {
-  if (KC) {
-    return *reinterpret_cast<const float4*>(tile + idx * LD + k0);
-  } else {
-    const float* q = tile + k0 * LD + idx;
-    return make_float4(q[0], q[LD], q[2 * LD], q[3 * LD]);
-  }
-}
+// The loader of a workgroup's tile of EXT rows and TK steps: K-contiguous, TK / 8 threads on a row; MN-contiguous, neighbouring
+// threads on neighbouring rows.
+template <bool KC, bool MNMAJ, int EXT, int VEC, int HOW, int GR>
+struct TileLoader : Loader<KC, MNMAJ, EXT * TK / (NT * 8), KC ? NT / (TK / 8) : 1, VEC, HOW, GR, TK> {
+  static constexpr int NMN = EXT * TK / (NT * 8), ROWSTEP = KC ? NT / (TK / 8) : 1;
+  int row0, octet;
 
-template <typename C_, int NCB, int NI, int NJ>
-__device__ __forceinline__ void stage_mma(const float* As, const float* Bs, v16f (&acc)[NRB][NCB], int arow, int bcol, int h) {
-  constexpr int TN = 64 * NCB;
-  constexpr int ALD = TileShape<C_::A_KC, TM>::LD, BLD = TileShape<C_::B_KC, TN>::LD;
-  constexpr int NS = TK / 8;
-  float4 a[2][NI], b[2][NJ];
-#pragma unroll
-  for (int i = 0; i < NI; ++i) a[0][i] = fetch_operand<C_::A_KC, ALD>(As, arow + BSTR * i, 4 * h);
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) b[0][j] = fetch_operand<C_::B_KC, BLD>(Bs, bcol + BSTR * j, 4 * h);
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int cur = s & 1, nxt = cur ^ 1;
-    if (s + 1 < NS) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) a[nxt][i] = fetch_operand<C_::A_KC, ALD>(As, arow + BSTR * i, 8 * (s + 1) + 4 * h);
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) b[nxt][j] = fetch_operand<C_::B_KC, BLD>(Bs, bcol + BSTR * j, 8 * (s + 1) + 4 * h);
-    }
-    __builtin_amdgcn_sched_barrier(0);   // keep the LDS reads of the next step ahead of this step's MFMAs
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const float av = t == 0 ? a[cur][i].x : t == 1 ? a[cur][i].y : t == 2 ? a[cur][i].z : a[cur][i].w;
-          const float bv = t == 0 ? b[cur][j].x : t == 1 ? b[cur][j].y : t == 2 ? b[cur][j].z : b[cur][j].w;
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc[i][j], 0, 0, 0);
-        }
+  __device__ __forceinline__ void init(const float* base_l, int L, int MNI, int KI, int tile0) {
+    const int t = threadIdx.x;
+    octet = KC ? t % (TK / 8) : t / (EXT / NMN);
+    row0 = KC ? t / (TK / 8) : (t % (EXT / NMN)) * NMN;
+    Loader<KC, MNMAJ, NMN, ROWSTEP, VEC, HOW, GR, TK>::init(base_l, L, MNI, KI, tile0 + row0, 8 * octet);
   }
-}
 
-// Double-buffered LDS: while the matrix cores consume stage s from one buffer, the operands of stage s+1
-// (fetched during stage s-1) are written to the other and the global loads of stage s+2 are issued; one
-// barrier per stage.
-template <typename C_, int NCB, int NI, int NJ, typename LA, typename LB>
-__device__ __forceinline__ void contract(LA& la, LB& lb, float* As, float* Bs, v16f (&acc)[NRB][NCB],
-                                         int nstage, int arow, int bcol, int h) {
-  constexpr int TN = 64 * NCB;
-  constexpr int AEL = TileShape<C_::A_KC, TM>::ELEMS, BEL = TileShape<C_::B_KC, TN>::ELEMS;
-  la.load();
-  lb.load();
-  la.store(As);
-  lb.store(Bs);
-  if (nstage > 1) {
-    la.load();
-    lb.load();
+  __device__ __forceinline__ void store(SplitTile<EXT, TK>& tile) const {
+#pragma unroll
+    for (int q = 0; q < NMN; ++q) tile.put(row0 + q * ROWSTEP, octet, this->reg[q]);
   }
-  __syncthreads();
-  for (int stage = 0; stage < nstage; ++stage) {
-    const int cur = stage & 1;
-    if (stage + 1 < nstage) {
-      la.store(As + (cur ^ 1) * AEL);       // that buffer was last read in stage - 1, which every wave has left
-      lb.store(Bs + (cur ^ 1) * BEL);
-      if (stage + 2 < nstage) {
-        la.load();
-        lb.load();
-      }
-    }
-    if (NI > 0 && NJ > 0)
-      stage_mma<C_, NCB, (NI > 0 ? NI : 1), (NJ > 0 ? NJ : 1)>(As + cur * AEL, Bs + cur * BEL, acc, arow, bcol, h);
-    __syncthreads();
-  }
-}
+};
 
-__host__ __device__ inline void tile_counts(int L, int RI, int CI, int TN, int& tm, int& tn, int& slots) {
+__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
+
+__host__ __device__ inline void tile_counts(int L, int RI, int CI, int TM, int TN, int& tm, int& tn, int& slots) {
   tm = s2cnn::ceil_div(L * RI, TM);
   tn = s2cnn::ceil_div(L * CI, TN);
   slots = tm * tn;
 }
 
-template <int MODE, int VA, int VB, int FAST, int NCB>
-__global__ __launch_bounds__(NT) void so3_block_mm_real_kernel(MmParams p) {
+// The tile again with the float32 matrix instruction, operands straight from memory: for tiles in which a result is not
+// finite.  The parts of an infinity, and of a value that rounds to one in bf16, are not its sum (inf - inf); here such
+// values take part as they are, so overflow, infinities and NaN come out as in any float32 product.
+template <typename C_, int NI, int NJ, int STEP>
+__device__ __forceinline__ void contract_float32(const MmParams& p, const float* A, const float* B, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h) {
+  const int K = L * p.KI;
+  size_t ao[NI], bo[NJ];
+  bool aok[NI], bok[NJ];
+  const size_t ablk = (size_t)p.RI * p.KI, bblk = (size_t)p.CI * p.KI;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = row0 + STEP * i, rb = row / p.RI, ri = row - rb * p.RI;
+    aok[i] = row < L * p.RI;
+    ao[i] = (C_::A_MNMAJ ? (size_t)rb * L : (size_t)rb) * ablk + (size_t)ri * (C_::A_KC ? p.KI : 1);
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int col = col0 + STEP * j, cb = col / p.CI, ci = col - cb * p.CI;
+    bok[j] = col < L * p.CI;
+    bo[j] = (C_::B_MNMAJ ? (size_t)cb * L : (size_t)cb) * bblk + (size_t)ci * (C_::B_KC ? p.KI : 1);
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  int kb = h / p.KI, kin = h - kb * p.KI;
+  for (int k0 = 0; k0 < K; k0 += 2) {
+    const bool ok = k0 + h < K;
+    const size_t ka = (C_::A_MNMAJ ? (size_t)kb : (size_t)kb * L) * ablk + (size_t)kin * (C_::A_KC ? 1 : p.RI);
+    const size_t kbo = (C_::B_MNMAJ ? (size_t)kb : (size_t)kb * L) * bblk + (size_t)kin * (C_::B_KC ? 1 : p.CI);
+    float a[NI], b[NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) a[i] = ok && aok[i] ? A[ao[i] + ka] : 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) b[j] = ok && bok[j] ? B[bo[j] + kbo] : 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    kin += 2;
+    while (kin >= p.KI) { kin -= p.KI; ++kb; }
+  }
+}
+
+// One LDS buffer: the operands of a stage are split and written while the loads of the next stage are issued, a barrier,
+// the matrix instructions, a barrier.  The other workgroup of the CU fills the matrix cores meanwhile.
+template <int NCB, bool FULL, typename LA, typename LB>
+__device__ __forceinline__ void contract(LA& la, LB& lb, SplitTile<TM, TK>& As, SplitTile<64 * NCB, TK>& Bs, v16f (&acc)[NRB][NCB],
+                                         int nstage, int arow, int bcol, int h, int ni, int nj) {
+  la.load();
+  lb.load();
+  for (int stage = 0; stage < nstage; ++stage) {
+    la.store(As);
+    lb.store(Bs);
+    if (stage + 1 < nstage) {
+      la.load();
+      lb.load();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < TK / 16; ++s) {
+      s2cnn::SplitFragment a[NRB], b[NCB];
+#pragma unroll
+      for (int i = 0; i < NRB; ++i) a[i] = As.get(arow + BSTR * i, 2 * s + h);
+#pragma unroll
+      for (int j = 0; j < NCB; ++j) b[j] = Bs.get(bcol + BSTR * j, 2 * s + h);
+      if (FULL) {
+        s2cnn::split_mma<NRB, NCB>(a, b, acc);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NRB; ++i)
+#pragma unroll
+          for (int j = 0; j < NCB; ++j)
+            if (i < ni && j < nj) s2cnn::split_mma_one(a[i], b[j], acc[i][j]);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+template <int MODE, int VA, int VB, int HOW, int GR, int NCB>
+__global__ __launch_bounds__(NT, 2) void so3_block_mm_real_kernel(MmParams p) {
   typedef Cfg<MODE> C_;
   constexpr int TN = 64 * NCB;
 
-  __shared__ __attribute__((aligned(16))) float As[2 * TileShape<C_::A_KC, TM>::ELEMS];
-  __shared__ __attribute__((aligned(16))) float Bs[2 * TileShape<C_::B_KC, TN>::ELEMS];
+  __shared__ SplitTile<TM, TK> As;
+  __shared__ SplitTile<TN, TK> Bs;
 
   int t = blockIdx.x;
+  constexpr int ROUND = 8 * XCD_RUN;
+  if (t < (int)gridDim.x / ROUND * ROUND) t = t / ROUND * ROUND + t % 8 * XCD_RUN + t % ROUND / 8;
   int l = p.nl - 1, tm = 0, tn = 0, slots = 0;
   for (;; --l) {
-    tile_counts(2 * l + 1, p.RI, p.CI, TN, tm, tn, slots);
+    tile_counts(2 * l + 1, p.RI, p.CI, TM, TN, tm, tn, slots);
     if (t < slots || l == 0) break;
     t -= slots;
   }
-  const int tile_nq = t / tm;
   const int L = 2 * l + 1;
-  const int tile_m = (t % tm) * TM;
-  const int tile_n = tile_nq * TN;
+  const int band = t / (BAND * tn), bm = tm - band * BAND < BAND ? tm - band * BAND : BAND, tb = t - band * BAND * tn;
+  const int tile_m = (band * BAND + tb % bm) * TM;
+  const int tile_n = tb / bm * TN;
   const size_t L0 = (size_t)l * (4 * l * l - 1) / 3;
   const int M = L * p.RI, N = L * p.CI;
+  const float* A = p.A + L0 * p.RI * p.KI;
+  const float* B = p.B + L0 * p.CI * p.KI;
 
-  TileLoader<C_::A_KC, C_::A_MNMAJ, TM, VA, FAST> la;
-  TileLoader<C_::B_KC, C_::B_MNMAJ, TN, VB, FAST> lb;
-  la.init(p.A + L0 * p.RI * p.KI, L, p.RI, p.KI, tile_m);
-  lb.init(p.B + L0 * p.CI * p.KI, L, p.CI, p.KI, tile_n);
+  TileLoader<C_::A_KC, C_::A_MNMAJ, TM, VA, HOW, GR> la;
+  TileLoader<C_::B_KC, C_::B_MNMAJ, TN, VB, HOW, GR> lb;
+  la.init(A, L, p.RI, p.KI, tile_m);
+  lb.init(B, L, p.CI, p.KI, tile_n);
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -400,31 +352,21 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_kernel(MmParams p) {
   int ni = remr <= 0 ? 0 : (remr + BSTR - 1) / BSTR, nj = remc <= 0 ? 0 : (remc + BSTR - 1) / BSTR;
   ni = ni > NRB ? NRB : ni;
   nj = nj > NCB ? NCB : nj;
-  if (ni == 0 || nj == 0) ni = nj = 0;
 
   const int nstage = s2cnn::ceil_div(L * p.KI, TK);
-#define S2CNN_CONTRACT(I, J) contract<C_, NCB, I, J>(la, lb, As, Bs, acc, nstage, wrow + r32, wcol + r32, h)
-  if (nj == NCB) {
-    switch (ni) {
-      case 4: if (NRB >= 4) { S2CNN_CONTRACT((NRB >= 4 ? 4 : 1), NCB); } break;
-      case 3: if (NRB >= 3) { S2CNN_CONTRACT((NRB >= 3 ? 3 : 1), NCB); } break;
-      case 2: if (NRB >= 2) { S2CNN_CONTRACT((NRB >= 2 ? 2 : 1), NCB); } break;
-      case 1: S2CNN_CONTRACT(1, NCB); break;
-      default: S2CNN_CONTRACT(0, 0); break;
-    }
-  } else if (nj == 0) {
-    S2CNN_CONTRACT(0, 0);
-  } else if constexpr (NCB > 1) {
-    switch (ni) {
-      case 4: if (NRB >= 4) { S2CNN_CONTRACT((NRB >= 4 ? 4 : 1), 1); } break;
-      case 3: if (NRB >= 3) { S2CNN_CONTRACT((NRB >= 3 ? 3 : 1), 1); } break;
-      case 2: if (NRB >= 2) { S2CNN_CONTRACT((NRB >= 2 ? 2 : 1), 1); } break;
-      default: S2CNN_CONTRACT(1, 1); break;
-    }
-  }
-#undef S2CNN_CONTRACT
+  if (ni == NRB && nj == NCB) contract<NCB, true>(la, lb, As, Bs, acc, nstage, wrow + r32, wcol + r32, h, ni, nj);
+  else contract<NCB, false>(la, lb, As, Bs, acc, nstage, wrow + r32, wcol + r32, h, ni, nj);
 
   // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32 of its 32x32 block.
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < NRB; ++i)
+#pragma unroll
+    for (int j = 0; j < NCB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) finite = finite && is_finite(acc[i][j][v]);
+  if (!__all(finite)) contract_float32<C_, NRB, NCB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);
+
   float* Cl = p.C + L0 * p.RI * p.CI;
   const int blk_elems = p.RI * p.CI;
 #pragma unroll
@@ -436,26 +378,136 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_kernel(MmParams p) {
     for (int i = 0; i < NRB; ++i) {
       if (i >= ni) continue;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = tile_m + wrow + BSTR * i + 8 * (v / 4) + 4 * h + (v % 4);
-        if (row < M) {
-          const int rb = row / p.RI, ri = row - rb * p.RI;
-          const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
-          Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = acc[i][j][v];
+      for (int g = 0; g < 4; ++g) {
+        const int row0 = tile_m + wrow + BSTR * i + 8 * g + 4 * h;
+        int rb = row0 / p.RI, ri = row0 - rb * p.RI;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          if (row0 + v < M) {
+            const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
+            Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = acc[i][j][4 * g + v];
+          }
+          if (++ri == p.RI) { ri = 0; ++rb; }
         }
       }
     }
   }
 }
 
-int total_slots(int nl, int RI, int CI, int TN) {
+// Small problems: too few 128 x 64 tiles to fill the chip, so that what counts is how many loads are in flight and how few
+// steps follow one another.  A workgroup owns 32 x (32 NJ) outputs and its four waves take every
+// fourth 16 steps of the contraction; a lane loads the octets it feeds to the matrix instruction straight from memory
+// (no LDS, no barriers, the next octets in flight meanwhile) and the four partial sums meet in LDS at the end.
+// us of fwd / gradx / grady, tiles of the other kernel -> this one (the float32 kernel before): 6 degrees, batch 32, 20 -> 40:
+// 14 / 21 / 20 -> 5.7 / 5.8 / 6.4 (15 / 22 / 19); the same with batch 1: 12 / 20 / 6 -> 4.7 / 5.5 / 4.0 (10 / 13 / 8); 8 degrees, batch 2,
+// 50 -> 50: 37 / 36 / 8 -> 9 / 9 / 9 (23 / 24 / 9).  From 256 tiles of 128 x 64 on it is the slower one: 24 degrees, batch 4, 30 -> 30
+// (440 tiles) 72 / 69 -> 74 / 82; around the line (10 to 40 stages, 230 to 360 tiles) the two are within 10 % of one another.  Two
+// blocks per wave pay from 400 tiles of 32 x 64 (422: 30.4 -> 28.4, 794: 47 -> 36; 353: 38 -> 44).
+template <int MODE, int VA, int VB, int HOW, int GR, int NJ>
+__global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p) {
+  typedef Cfg<MODE> C_;
+  constexpr int NW = NT / 64, TMS = 32, TNS = 32 * NJ, ADV = 16 * NW;
+  __shared__ float part[NW][NJ][16][64];
+
+  int t = blockIdx.x;
+  int l = p.nl - 1, tm = 0, tn = 0, slots = 0;
+  for (;; --l) {
+    tile_counts(2 * l + 1, p.RI, p.CI, TMS, TNS, tm, tn, slots);
+    if (t < slots || l == 0) break;
+    t -= slots;
+  }
+  const int L = 2 * l + 1;
+  const int tile_m = t % tm * TMS, tile_n = t / tm * TNS;
+  const size_t L0 = (size_t)l * (4 * l * l - 1) / 3;
+  const int M = L * p.RI, N = L * p.CI;
+  const float* A = p.A + L0 * p.RI * p.KI;
+  const float* B = p.B + L0 * p.CI * p.KI;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r32 = lane & 31, h = lane >> 5;
+
+  Loader<C_::A_KC, C_::A_MNMAJ, 1, 1, VA, HOW, GR, ADV> la;
+  Loader<C_::B_KC, C_::B_MNMAJ, NJ, 32, VB, HOW, GR, ADV> lb;
+  la.init(A, L, p.RI, p.KI, tile_m + r32, 16 * wave + 8 * h);
+  lb.init(B, L, p.CI, p.KI, tile_n + r32, 16 * wave + 8 * h);
+
+  v16f acc[1][NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[0][j][v] = 0.f;
+
+  const int nstep = s2cnn::ceil_div(L * p.KI, ADV);      // the same for all waves: steps behind the end are zeros
+  la.load();
+  lb.load();
+  for (int step = 0; step < nstep; ++step) {
+    s2cnn::SplitFragment a[1], b[NJ];
+    a[0] = s2cnn::split_octet(la.reg[0]);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) b[j] = s2cnn::split_octet(lb.reg[j]);
+    if (step + 1 < nstep) {
+      la.load();
+      lb.load();
+    }
+    s2cnn::split_mma<1, NJ>(a, b, acc);
+  }
+
+  // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32; wave w adds up and stores v = 4w .. 4w+3.
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[wave][j][v][lane] = acc[0][j][v];
+  __syncthreads();
+  float sum[NJ][4];
+  bool finite = true;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float s = part[0][j][4 * wave + v][lane];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) s += part[w][j][4 * wave + v][lane];
+      sum[j][v] = s;
+      finite = finite && is_finite(s);
+    }
+  if (!__all(finite)) {
+    contract_float32<C_, 1, NJ, 32>(p, A, B, acc, L, tile_m + r32, tile_n + r32, h);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (v / 4 == wave) sum[j][v % 4] = acc[0][j][v];
+  }
+
+  float* Cl = p.C + L0 * p.RI * p.CI;
+  const int blk_elems = p.RI * p.CI;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int col = tile_n + 32 * j + r32;
+    if (col >= N) continue;
+    const int cb = col / p.CI, ci = col - cb * p.CI;
+    const int row0 = tile_m + 8 * wave + 4 * h;
+    int rb = row0 / p.RI, ri = row0 - rb * p.RI;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (row0 + v < M) {
+        const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
+        Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = sum[j][v];
+      }
+      if (++ri == p.RI) { ri = 0; ++rb; }
+    }
+  }
+}
+
+long total_slots(int nl, int RI, int CI, int TM, int TN) {
   long n = 0;
   for (int l = 0; l < nl; ++l) {
     int tm, tn, slots;
-    tile_counts(2 * l + 1, RI, CI, TN, tm, tn, slots);
+    tile_counts(2 * l + 1, RI, CI, TM, TN, tm, tn, slots);
     n += slots;
   }
-  return n > 0x7fffffffL ? -1 : (int)n;
+  return n > 0x7fffffffL ? -1 : n;
 }
 
 inline bool aligned4(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
@@ -467,44 +519,64 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
   const long Lmax = 2L * nl - 1;
   if (Lmax * Lmax * RI * KI >= (1L << 31) || Lmax * Lmax * CI * KI >= (1L << 31)) return S2CNN_EINVAL;
   if (!aligned4(a) || !aligned4(b) || !aligned4(c)) return S2CNN_EALIGN;
-  // 128 x 128 tiles unless they are too few to give every CU its two workgroups: then 128 x 64
-  const bool narrow = total_slots(nl, RI, CI, 128) < SMALL_GRID;
-  const int grid = total_slots(nl, RI, CI, narrow ? 64 : 128);
+  // beyond the small problems: 128 x 128 tiles unless they are too few to give every CU its two workgroups: then 128 x 64
+  const bool narrow = total_slots(nl, RI, CI, TM, 128) < SMALL_GRID;
+  const int grid = (int)total_slots(nl, RI, CI, TM, narrow ? 64 : 128);
   if (grid < 1) return S2CNN_EINVAL;
   MmParams p{a, b, c, nl, RI, CI, KI};
   typedef Cfg<MODE> C_;
-  // four (two) floats per access need the fast index of the operand to be a multiple of 4 (2) and a 16-byte (8-byte) base
-  const int afast = C_::A_KC ? KI : RI, bfast = C_::B_KC ? KI : CI;
-  const bool a4 = afast % 4 == 0 && s2cnn::aligned16(a);
-  const bool b4 = bfast % 4 == 0 && s2cnn::aligned16(b);
-  const bool a2 = a4 || (afast % 2 == 0 && s2cnn::aligned8(a));
-  const bool b2 = b4 || (bfast % 2 == 0 && s2cnn::aligned8(b));
+  // Wide accesses need the fast index of the operand to be a multiple of the width and a base aligned to it.  Along the
+  // contraction (K-contiguous operands) the width is also the granule of the walk.
+  const auto width = [](int fast, const float* q) { return fast % 4 == 0 && s2cnn::aligned16(q) ? 4 : fast % 2 == 0 && s2cnn::aligned8(q) ? 2 : 1; };
+  const int wa = width(C_::A_KC ? KI : RI, a), wb = width(C_::B_KC ? KI : CI, b);
+  const bool a2 = wa >= 2, b2 = wb >= 2;
+  const bool near = Lmax * Lmax * RI * KI < (1L << 29) && Lmax * Lmax * CI * KI < (1L << 29);   // 32-bit byte offsets below OUTSIDE
+  const bool divides = near && (C_::A_KC ? wa == 4 : a2) && (C_::B_KC ? wb == 4 : b2) && KI % 8 == 0 && (KI % TK == 0 || TK % KI == 0);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // the fast loaders address a degree with 32-bit byte offsets
-  const bool small = Lmax * Lmax * RI * KI < (1L << 30) && Lmax * Lmax * CI * KI < (1L << 30);
-  const bool divides = (KI % TK == 0 || TK % KI == 0) && small;                 // block size and K stage divide one another
-  const bool crosses = !divides && KI > TK && small;                           // 100 features: stages that run over a block boundary
-  const bool fast = a4 && b4 && divides;
-  const bool fast2 = a4 && b4 && crosses && KI % 4 == 0;
-  // the same two loaders with 8-byte accesses: even sizes that are no multiples of four (50, 70 features)
-  const bool fast_v2 = !fast && a2 && b2 && divides && KI % 2 == 0;
-  const bool fast2_v2 = !fast2 && a2 && b2 && crosses && KI % 2 == 0;
-#define S2CNN_LAUNCH(VA, VB, FAST)                                                                                    \
-  do {                                                                                                                \
-    if (narrow) hipLaunchKernelGGL((so3_block_mm_real_kernel<MODE, VA, VB, FAST, 1>), dim3(grid), dim3(NT), 0, st, p); \
-    else hipLaunchKernelGGL((so3_block_mm_real_kernel<MODE, VA, VB, FAST, 2>), dim3(grid), dim3(NT), 0, st, p);        \
+  const long tiles64 = total_slots(nl, RI, CI, TM, 64);
+  if (near && tiles64 > 0 && tiles64 < SLICES_GRID) {
+    const long tiles = total_slots(nl, RI, CI, 32, 64);
+    const bool two = tiles >= SLICES_WIDE;
+    const int g = (int)(two ? tiles : total_slots(nl, RI, CI, 32, 32));
+#define S2CNN_SLICES(V, GR)                                                                                                                              \
+  do {                                                                                                                                                   \
+    if (two) hipLaunchKernelGGL((so3_block_mm_real_slices_kernel<MODE, (C_::A_KC ? V : 1), (C_::B_KC ? V : 1), WALK, GR, 2>), dim3(g), dim3(NT), 0, st, p); \
+    else hipLaunchKernelGGL((so3_block_mm_real_slices_kernel<MODE, (C_::A_KC ? V : 1), (C_::B_KC ? V : 1), WALK, GR, 1>), dim3(g), dim3(NT), 0, st, p);     \
   } while (0)
-  if (fast) S2CNN_LAUNCH(4, 4, 1);
-  else if (fast2) S2CNN_LAUNCH(4, 4, 2);
-  else if (fast_v2) S2CNN_LAUNCH(2, 2, 1);
-  else if (fast2_v2) S2CNN_LAUNCH(2, 2, 2);
-  else if (a4 && b4) S2CNN_LAUNCH(4, 4, 0);
-  else if (a4 && b2) S2CNN_LAUNCH(4, 2, 0);
-  else if (a2 && b4) S2CNN_LAUNCH(2, 4, 0);
-  else if (a2 && b2) S2CNN_LAUNCH(2, 2, 0);      // even feature counts (50, 70, 350 in the reference's shape network)
-  else if (a4) S2CNN_LAUNCH(4, 1, 0);
-  else if (b4) S2CNN_LAUNCH(1, 4, 0);
-  else S2CNN_LAUNCH(1, 1, 0);
+    const int w = !C_::A_KC ? (KI % 4 == 0 ? 4 : 1) : C_::B_KC && wb < wa ? wb : wa;
+    if (w == 4) S2CNN_SLICES(4, 4);
+    else if (w == 2 && C_::A_KC) S2CNN_SLICES(2, (C_::A_KC ? 2 : 1));
+    else S2CNN_SLICES(1, 1);
+#undef S2CNN_SLICES
+    return s2cnn::launch_status();
+  }
+  // a 64-column tile of an MN-contiguous operand has one column per thread
+#define S2CNN_LAUNCH(VA, VB, HOW, GR)                                                                                                    \
+  do {                                                                                                                                   \
+    if (narrow) hipLaunchKernelGGL((so3_block_mm_real_kernel<MODE, VA, (C_::B_KC ? VB : 1), HOW, GR, 1>), dim3(grid), dim3(NT), 0, st, p); \
+    else hipLaunchKernelGGL((so3_block_mm_real_kernel<MODE, VA, VB, HOW, GR, 2>), dim3(grid), dim3(NT), 0, st, p);                        \
+  } while (0)
+  if (!near) S2CNN_LAUNCH(1, 1, FAR, 1);
+  else if (divides) S2CNN_LAUNCH((C_::A_KC ? 4 : 2), (C_::B_KC ? 4 : 2), DIVIDES, 8);
+  else if constexpr (MODE == FWD) {
+    if (wa == 4) { if (b2) S2CNN_LAUNCH(4, 2, WALK, 4); else S2CNN_LAUNCH(4, 1, WALK, 4); }
+    else if (wa == 2) { if (b2) S2CNN_LAUNCH(2, 2, WALK, 2); else S2CNN_LAUNCH(2, 1, WALK, 2); }
+    else { if (b2) S2CNN_LAUNCH(1, 2, WALK, 1); else S2CNN_LAUNCH(1, 1, WALK, 1); }
+  } else if constexpr (MODE == GRADX) {
+    if (wa == 4 && wb == 4) S2CNN_LAUNCH(4, 4, WALK, 4);
+    else if (a2 && b2) S2CNN_LAUNCH(2, 2, WALK, 2);
+    else S2CNN_LAUNCH(1, 1, WALK, 1);
+  } else if (KI % 4 == 0) {
+    if (a2 && b2) S2CNN_LAUNCH(2, 2, WALK, 4);
+    else if (a2) S2CNN_LAUNCH(2, 1, WALK, 4);
+    else if (b2) S2CNN_LAUNCH(1, 2, WALK, 4);
+    else S2CNN_LAUNCH(1, 1, WALK, 4);
+  } else {
+    if (a2 && b2) S2CNN_LAUNCH(2, 2, WALK, 1);
+    else if (a2) S2CNN_LAUNCH(2, 1, WALK, 1);
+    else if (b2) S2CNN_LAUNCH(1, 2, WALK, 1);
+    else S2CNN_LAUNCH(1, 1, WALK, 1);
+  }
 #undef S2CNN_LAUNCH
   return s2cnn::launch_status();
 }

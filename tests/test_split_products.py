@@ -1,0 +1,92 @@
+"""The block products on the bf16 matrix cores, every operand value cut into three bf16 parts: at the edges of their tiles and
+walks over the contraction, on operands that are not aligned, and on values that the parts do not represent."""
+import pytest
+import torch
+
+from oracle import cpu_path as O
+
+
+def product64(which, a, b, nl):
+    """The product of one degree after the other in float64: fwd (x, y), gradx (gz, y), grady (gz, x)."""
+    out, pos = [], 0
+    for l in range(nl):
+        L = 2 * l + 1
+        A = a[pos:pos + L * L].double().reshape(L, L, *a.shape[1:]).transpose(1, 2).reshape(L * a.shape[1], -1)      # (row, feature) x (col, feature)
+        B = b[pos:pos + L * L].double().reshape(L, L, *b.shape[1:])
+        if which == "grady":
+            B = B.transpose(1, 2).reshape(L * b.shape[1], -1)
+            Z = (A.t() @ B).reshape(L, a.shape[2], L, b.shape[2]).permute(0, 2, 3, 1)              # (n, j) x (p, k) as n, p, k, j
+        else:
+            B = B.permute(0, 3, 1, 2).reshape(L * b.shape[2], -1)                                  # (n, j) x (p, k)
+            Z = (A @ (B.t() if which == "fwd" else B)).reshape(L, a.shape[1], L, -1).transpose(1, 2)
+        out.append(Z.reshape(L * L, Z.shape[2], Z.shape[3]))
+        pos += L * L
+    return torch.cat(out)
+
+
+def unaligned(t):
+    """The same values behind a base that is aligned to 4 bytes only."""
+    buf = torch.empty(t.numel() + 1, device=t.device)
+    view = buf[1:].view(t.shape)
+    return view.copy_(t)
+
+
+# Errors: six roundings of 2^-24 per 16 contraction steps, of partial sums that grow with the root of the steps: about
+# 2^-24 sqrt(6 K / 32 / 3) of the result, and one rounding for short contractions.  Twice that is allowed, and one more
+# rounding: 2^-24 (1 + sqrt(K / 4)).
+def bound(K):
+    return 2.0 ** -24 * (1 + (K / 4) ** 0.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [
+    # small problems, 32 x 32 and 32 x 64 outputs: one row, one block and one more, one 16-step and one more
+    (1, 1, 1, 1), (1, 32, 16, 32), (1, 33, 17, 65), (3, 1, 7, 20), (6, 1, 20, 40), (7, 32, 100, 55), (2, 64, 65, 33),
+    # tiles of 128 x 64 and 128 x 128, contraction blocks that divide the stage (8, 16, 32) or are divided by it (64)
+    (16, 8, 40, 40), (12, 16, 64, 64), (10, 32, 96, 80),
+    # granules of 4, 2 and 1 steps, ragged rows, columns and last stages, in the tiles of both widths
+    (22, 3, 36, 20), (13, 11, 33, 45), (16, 9, 50, 70), (14, 13, 55, 41), (20, 7, 25, 60), (18, 30, 26, 38)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_real_product_edges(hip, nl, B, Fi, Fo, aligned):
+    import s2cnn_amd
+    print(f"split product nl={nl} B={B} Fi={Fi} Fo={Fo} aligned={aligned}", flush=True)
+    ns = O.nspec_so3(nl)
+    g = torch.Generator(device="cuda").manual_seed(nl)
+    x, y, gz = (torch.randn(ns, *s, device="cuda", generator=g) for s in ((B, Fi), (Fi, Fo), (B, Fo)))
+    if not aligned:
+        x, y, gz = unaligned(x), unaligned(y), unaligned(gz)
+    xg, yg = x.detach().requires_grad_(), y.detach().requires_grad_()
+    z = s2cnn_amd.so3_mm_real(xg, yg)
+    gx, gy = torch.autograd.grad(z, (xg, yg), gz)
+    L = 2 * nl - 1
+    for got, want, K in ((z, product64("fwd", x, y, nl), L * Fi), (gx, product64("gradx", gz, y, nl), L * Fo), (gy, product64("grady", gz, x, nl), L * B)):
+        assert ((got.double() - want).norm() / want.norm()).item() <= bound(K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(3, 5, 9, 7), (16, 8, 40, 40)])      # either kernel
+def test_real_product_of_values_without_bf16_parts(hip, nl, B, Fi, Fo):
+    """Infinities, NaN and values that round to infinity in bf16 give what float32 products give: where they take part
+    the result is the infinity, NaN or finite value of the exact sum, and elsewhere nothing changes."""
+    import s2cnn_amd
+    ns = O.nspec_so3(nl)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, y = torch.randn(ns, B, Fi, device="cuda", generator=g), torch.randn(ns, Fi, Fo, device="cuda", generator=g)
+    y[ns - 30:, :, 0] = 0.0
+    plain = product64("fwd", x, y, nl)
+    x[ns - 1, 0, 0] = float("inf")          # times zeros (NaN), times positive and negative values
+    x[ns - 7, 1, 1] = float("nan")
+    x[ns - 12, 2, 2] = 3.4e38 * 0.9999      # its first bf16 part is infinite
+    y = y * 0.125
+    want = product64("fwd", x, y, nl)
+    got = s2cnn_amd.so3_mm_real(x, y).double()
+    assert (~torch.isfinite(want)).any() and torch.isfinite(want).any()
+    overflow = want.abs() > 3.402823466e38
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[overflow], want[overflow].sign() * float("inf"))
+    ok = torch.isfinite(want) & ~overflow
+    # one huge product and terms that vanish beside it: the rounding of that product and of its sum, 2^-24 each
+    huge = ok & (want.abs() > 1e20)
+    assert huge.any() and ((got - want)[huge].abs() <= 2.0 ** -22 * want[huge].abs()).all()
+    same = ok & ~huge
+    assert ((got - plain * 0.125)[same].norm() / want[same].norm()).item() <= bound((2 * nl - 1) * Fi)
