@@ -1,5 +1,5 @@
-// Block-diagonal complex products over the (2l+1)x(2l+1) blocks of an SO(3) spectrum,
-// on the fp32 matrix cores of gfx950 (v_mfma_f32_32x32x2_f32).
+// Block-diagonal complex products over the (2l+1)x(2l+1) blocks of an SO(3) spectrum, on the bf16 matrix cores of gfx950 with
+// float32 operands and results.
 //
 // For one degree l (L = 2l+1) each of the three products is a complex GEMM whose three
 // index spaces are pairs (spectral index, feature index):
@@ -11,41 +11,30 @@
 // with tensors stored as [l, spectral row, spectral col, feature row, feature col, 2].
 // An operand is therefore an L x L grid of dense feature blocks; within a block either the
 // contraction index ("K-contiguous") or the free index ("MN-contiguous") is the fast one.
-// The kernel keeps each operand tile in LDS in the orientation it has in memory, so loads
-// from HBM are coalesced and nothing is transposed on the way.
-//
-// Complex arithmetic on a real matrix core, three real products per complex one (Gauss): with
-// b = br + i bi' (bi' = -bi where the operand is conjugated)
-//     P1 = sum ar br,   P2 = sum ai bi',   P3 = sum (ar + ai)(br + bi')
-//     re = P1 - P2,     im = P3 - P1 - P2.
-// One MFMA 32x32x2 takes two contraction steps, one per half-wave; a lane holds two consecutive complex
-// steps of its row / column (four floats), forms the two sums in registers and feeds six MFMAs: 1.5 per
-// complex multiply-add instead of the 2 of the direct form, at the price of a third accumulator per block.
-// The sums are formed in fp32 before the product, so the imaginary part carries a rounding error of the
-// size of |a||b| eps rather than of its own size: the same bound as any fp32 complex product.
-//
-// Tiling.  A workgroup (4 waves) owns 128 rows x 64 columns = 4 x 2 blocks of 32.  Wave (wm, wn)
-// takes row blocks wm, wm+2 and column block wn, so a ragged tile (fewer live blocks) still
-// splits evenly over the waves; blocks that lie wholly outside the matrix are skipped per wave.
-// The grid lists exactly the tiles of all degrees, heaviest degree first (no idle workgroups:
-// a workgroup that exits at once still waits for a full slot and stalls the in-order dispatch).
-#include <type_traits>
 #include "common.h"
+#include "split_bf16.h"
+#include "block_loader.h"
 
 namespace {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
+using namespace s2cnn::block;
+using s2cnn::SplitFragment;
+using s2cnn::SplitTile;
+using s2cnn::v16f;
 
-constexpr int NRB = 2;            // 32-row blocks per wave
-constexpr int NCB = 1;            // 32-column blocks per wave (three accumulators per block: 96 registers per wave)
-constexpr int TM = 64 * NRB;      // tile rows   (flattened (spectral, feature) index): 2 waves x NRB blocks
-constexpr int TN = 64 * NCB;      // tile cols
+constexpr int NB = 2;             // 32 x 32 blocks per wave in each direction
+constexpr int TM = 64 * NB;       // tile rows and columns (flattened (spectral, feature) index)
 constexpr int BSTR = 64, WSTR = 32;   // a wave's blocks are 64 apart, the two waves of a dimension offset by 32
 constexpr int TK = 16;            // complex contraction steps per LDS stage
-constexpr int NT = 256;           // threads: 4 waves
-constexpr int KC_LD = TK + 2;     // leading dim (complex) of a K-contiguous LDS tile: 144 B rows
+constexpr int GROUP = 256;        // threads that form one of the three real products
+constexpr int NT = 3 * GROUP;
+constexpr int BAND = 8;           // tiles are listed in bands of 8 rows of tiles, column after column
+constexpr int XCD_RUN = 32;       // consecutive tiles of the list that one XCD takes
+constexpr int NTS = 256;          // threads of a workgroup of the kernel for small problems
+constexpr int SMALL_TILES = 2048; // fewer 32 x 32 tiles than this: that kernel
 
 enum Mode { FWD = 0, GRADX = 1, GRADY = 2 };
+enum Kind { RE = 0, IM = 1, SUM = 2 };
 
 struct MmParams {
   const float2* A;
@@ -63,306 +52,393 @@ template <> struct Cfg<FWD>   { static constexpr bool A_KC = true,  B_KC = false
 template <> struct Cfg<GRADX> { static constexpr bool A_KC = true,  B_KC = true,  A_MNMAJ = true,  B_MNMAJ = false, C_RMAJ = true,  CONJ = false; };
 template <> struct Cfg<GRADY> { static constexpr bool A_KC = false, B_KC = false, A_MNMAJ = false, B_MNMAJ = false, C_RMAJ = false, CONJ = true;  };
 
-template <bool KC, int EXT> struct TileShape {
-  static constexpr int LD = KC ? KC_LD : EXT;             // LDS leading dimension (complex)
-  static constexpr int ELEMS = KC ? EXT * KC_LD : TK * EXT;
-};
+__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 
-// One operand's tile loader: global -> registers -> LDS.  EXT = tile extent along the free index,
-// VEC = complex numbers per access.
-template <bool KC, bool MNMAJ, int EXT, int VEC>
-struct TileLoader {
-  static constexpr int NSLOT = EXT * TK / (NT * VEC);
-  static constexpr int LD = TileShape<KC, EXT>::LD;
-  typedef typename std::conditional<VEC == 2, float4, float2>::type vec_t;
-  static_assert(NSLOT >= 1, "tile too small for the workgroup");
+__host__ __device__ inline int tile_counts(int L, int RI, int CI, int TMV, int TNV, int& tm, int& tn) {
+  tm = s2cnn::ceil_div(L * RI, TMV);
+  tn = s2cnn::ceil_div(L * CI, TNV);
+  return tm * tn;
+}
 
-  const float2* base;   // start of degree l
-  int off[KC ? NSLOT : 1];
-  unsigned valid_mn;    // bit q: slot q's row is inside the matrix (KC) / bit 0 (MN-contiguous)
-  int kk;               // KC: this thread's k inside the stage; else k of slot 0
-  int lds_off;          // LDS offset (complex) of slot 0
-  int blk_k_stride;     // elements between consecutive contraction blocks
-  int MNI, KI;
-  vec_t reg[NSLOT];
-
-  __device__ void init(const float2* base_l, int L, int MNI_, int KI_, int tile0) {
-    base = base_l; MNI = MNI_; KI = KI_;
-    const int t = threadIdx.x;
-    const int blk_elems = MNI * KI;
-    const int blk_mn_stride = (MNMAJ ? L : 1) * blk_elems;
-    blk_k_stride = (MNMAJ ? 1 : L) * blk_elems;
-    valid_mn = 0;
-    if (KC) {
-      constexpr int TPR = TK / VEC;          // threads per tile row
-      kk = (t % TPR) * VEC;
-      const int r0 = t / TPR;
-      lds_off = r0 * LD + kk;
-#pragma unroll
-      for (int q = 0; q < NSLOT; ++q) {
-        const int row = tile0 + r0 + q * (NT / TPR);
-        const int mb = row / MNI, mi = row - mb * MNI;
-        off[q] = mb * blk_mn_stride + mi * KI + kk;
-        if (row < L * MNI) valid_mn |= 1u << q;
-      }
-    } else {
-      constexpr int TPR = EXT / VEC;         // threads per k-row of the tile
-      const int mn = tile0 + (t % TPR) * VEC;
-      kk = t / TPR;
-      lds_off = kk * LD + (t % TPR) * VEC;
-      const int mb = mn / MNI, mi = mn - mb * MNI;
-      off[0] = mb * blk_mn_stride + mi;
-      if (mn < L * MNI) valid_mn = 1u;
-    }
+// degree and place in its list of tiles, heaviest degree first
+__device__ __forceinline__ int find_degree(const MmParams& p, int TMV, int TNV, int& t, int& tm, int& tn) {
+  int l = p.nl - 1;
+  for (;; --l) {
+    const int slots = tile_counts(2 * l + 1, p.RI, p.CI, TMV, TNV, tm, tn);
+    if (t < slots || l == 0) break;
+    t -= slots;
   }
+  return l;
+}
 
-  // clamped address + select instead of a predicated load: all loads of a stage are in flight together
-  __device__ void load(int kb, int k0) {
-    const float2* p = base + (size_t)kb * blk_k_stride;
-    if (KC) {
-      const bool kvalid = (k0 + kk) < KI;
+// what one of the three products takes from a complex operand: b carries the sign of the conjugation
+template <int KIND> __device__ __forceinline__ float part_of(float2 v) { return KIND == RE ? v.x : KIND == IM ? v.y : v.x + v.y; }
+template <bool CONJ> __device__ __forceinline__ float2 conj_of(float2 v) { return CONJ ? make_float2(v.x, -v.y) : v; }
+
+// A real product of a tile with the float32 matrix instruction, operands straight from memory: for tiles in which it is not
+// finite.  The parts of an infinity, and of a value that rounds to one in bf16, are not its sum (inf - inf); here such
+// values take part as they are, so overflow, infinities and NaN come out as in a float32 product of the same form.
+template <typename C_, int KIND, int NI, int NJ, int STEP>
+__device__ __forceinline__ void contract_float32(const MmParams& p, const float2* A, const float2* B, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h) {
+  const int K = L * p.KI;
+  size_t ao[NI], bo[NJ];
+  bool aok[NI], bok[NJ];
+  const size_t ablk = (size_t)p.RI * p.KI, bblk = (size_t)p.CI * p.KI;
 #pragma unroll
-      for (int q = 0; q < NSLOT; ++q) {
-        const bool ok = kvalid && ((valid_mn >> q) & 1u);
-        const vec_t v = *reinterpret_cast<const vec_t*>(p + (ok ? off[q] + k0 : 0));
-        reg[q] = ok ? v : vec_t{};
-      }
-    } else {
-      constexpr int KSTEP = NT * VEC / EXT;
-#pragma unroll
-      for (int q = 0; q < NSLOT; ++q) {
-        const int k = k0 + kk + q * KSTEP;
-        const bool ok = valid_mn && k < KI;
-        const vec_t v = *reinterpret_cast<const vec_t*>(p + (ok ? off[0] + k * MNI : 0));
-        reg[q] = ok ? v : vec_t{};
-      }
-    }
+  for (int i = 0; i < NI; ++i) {
+    const int row = row0 + STEP * i, rb = row / p.RI, ri = row - rb * p.RI;
+    aok[i] = row < L * p.RI;
+    ao[i] = (C_::A_MNMAJ ? (size_t)rb * L : (size_t)rb) * ablk + (size_t)ri * (C_::A_KC ? p.KI : 1);
   }
-
-  __device__ void store(float2* tile) const {
-    if (KC) {
-      constexpr int RSTEP = NT * VEC / TK;
 #pragma unroll
-      for (int q = 0; q < NSLOT; ++q)
-        *reinterpret_cast<vec_t*>(tile + lds_off + q * RSTEP * LD) = reg[q];
-    } else {
-      constexpr int KSTEP = NT * VEC / EXT;
-#pragma unroll
-      for (int q = 0; q < NSLOT; ++q)
-        *reinterpret_cast<vec_t*>(tile + lds_off + q * KSTEP * LD) = reg[q];
-    }
+  for (int j = 0; j < NJ; ++j) {
+    const int col = col0 + STEP * j, cb = col / p.CI, ci = col - cb * p.CI;
+    bok[j] = col < L * p.CI;
+    bo[j] = (C_::B_MNMAJ ? (size_t)cb * L : (size_t)cb) * bblk + (size_t)ci * (C_::B_KC ? p.KI : 1);
   }
-};
-
-// The four reals (re k0, im k0, re k0+1, im k0+1) of tile row/col `idx` and the lane's pair of
-// contraction steps k0 = 4s + 2h.
-template <bool KC, int LD>
-__device__ __forceinline__ float4 fetch_operand(const float2* tile, int idx, int k0) {
-  if (KC) {
-    return *reinterpret_cast<const float4*>(tile + idx * LD + k0);
-  } else {
-    const float2 a = tile[k0 * LD + idx];
-    const float2 b = tile[(k0 + 1) * LD + idx];
-    return make_float4(a.x, a.y, b.x, b.y);
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  int kb = h / p.KI, kin = h - kb * p.KI;
+  for (int k0 = 0; k0 < K; k0 += 2) {
+    const bool ok = k0 + h < K;
+    const size_t ka = (C_::A_MNMAJ ? (size_t)kb : (size_t)kb * L) * ablk + (size_t)kin * (C_::A_KC ? 1 : p.RI);
+    const size_t kbo = (C_::B_MNMAJ ? (size_t)kb : (size_t)kb * L) * bblk + (size_t)kin * (C_::B_KC ? 1 : p.CI);
+    float a[NI], b[NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) a[i] = ok && aok[i] ? part_of<KIND>(A[ao[i] + ka]) : 0.f;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) b[j] = ok && bok[j] ? part_of<KIND>(conj_of<C_::CONJ>(B[bo[j] + kbo])) : 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+    kin += 2;
+    while (kin >= p.KI) { kin -= p.KI; ++kb; }
   }
 }
 
-// the three accumulators of a 32x32 block of complex outputs
-struct Acc3 { v16f p1, p2, p3; };
+// One operand's tile in LDS: real parts, imaginary parts (with the sign of the conjugation), their sums, each in bf16 parts.
+struct OperandTile {
+  SplitTile<TM, TK> kind[3];
 
-// All matrix-core work of one LDS stage for a wave with NI live row blocks (rows arow + 64 i) and NJ
-// live column blocks (columns bcol + 64 j).  Operand registers are double buffered: the LDS reads of
-// step s+1 are issued before the MFMAs of step s.
-template <typename C_, int NI, int NJ>
-__device__ __forceinline__ void stage_mma(const float2* As, const float2* Bs, Acc3 (&acc)[NRB][NCB], int arow, int bcol, int h) {
-  constexpr int ALD = TileShape<C_::A_KC, TM>::LD, BLD = TileShape<C_::B_KC, TN>::LD;
-  float4 a[2][NI], b[2][NJ];
+  template <bool CONJ> __device__ __forceinline__ void put(int row, int octet, const float2 (&v)[8]) {
+    float x[8];
 #pragma unroll
-  for (int i = 0; i < NI; ++i) a[0][i] = fetch_operand<C_::A_KC, ALD>(As, arow + BSTR * i, 2 * h);
+    for (int e = 0; e < 8; ++e) x[e] = v[e].x;
+    kind[RE].put(row, octet, x);
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) b[0][j] = fetch_operand<C_::B_KC, BLD>(Bs, bcol + BSTR * j, 2 * h);
+    for (int e = 0; e < 8; ++e) x[e] = CONJ ? -v[e].y : v[e].y;
+    kind[IM].put(row, octet, x);
 #pragma unroll
-  for (int s = 0; s < TK / 4; ++s) {
-    const int cur = s & 1, nxt = cur ^ 1;
-    if (s + 1 < TK / 4) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) a[nxt][i] = fetch_operand<C_::A_KC, ALD>(As, arow + BSTR * i, 4 * (s + 1) + 2 * h);
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) b[nxt][j] = fetch_operand<C_::B_KC, BLD>(Bs, bcol + BSTR * j, 4 * (s + 1) + 2 * h);
-    }
-    __builtin_amdgcn_sched_barrier(0);   // keep the LDS reads of the next step ahead of this step's MFMAs
-    float2 asum[NI], bim[NJ], bsum[NJ];  // per contraction step of the lane's pair: ar + ai | bi' | br + bi'
-#pragma unroll
-    for (int i = 0; i < NI; ++i) asum[i] = make_float2(a[cur][i].x + a[cur][i].y, a[cur][i].z + a[cur][i].w);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const float4 v = b[cur][j];
-      bim[j] = C_::CONJ ? make_float2(-v.y, -v.w) : make_float2(v.y, v.w);
-      bsum[j] = make_float2(v.x + bim[j].x, v.z + bim[j].y);
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          const float ar = t == 0 ? a[cur][i].x : a[cur][i].z, ai = t == 0 ? a[cur][i].y : a[cur][i].w;
-          const float br = t == 0 ? b[cur][j].x : b[cur][j].z;
-          acc[i][j].p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(ar, br, acc[i][j].p1, 0, 0, 0);
-          acc[i][j].p2 = __builtin_amdgcn_mfma_f32_32x32x2f32(ai, t == 0 ? bim[j].x : bim[j].y, acc[i][j].p2, 0, 0, 0);
-          acc[i][j].p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(t == 0 ? asum[i].x : asum[i].y, t == 0 ? bsum[j].x : bsum[j].y,
-                                                              acc[i][j].p3, 0, 0, 0);
-        }
+    for (int e = 0; e < 8; ++e) x[e] = CONJ ? v[e].x - v[e].y : v[e].x + v[e].y;
+    kind[SUM].put(row, octet, x);
   }
-}
+};
 
-// The contraction loop of one tile.  LDS is double buffered: while the matrix cores consume stage s from one
-// buffer, the operands of stage s+1 (fetched during stage s-1) are written to the other and the global loads
-// of stage s+2 are issued; one barrier per stage.
-template <typename C_, int NI, int NJ, typename LA, typename LB>
-__device__ __forceinline__ void contract(LA& la, LB& lb, float2* As, float2* Bs, Acc3 (&acc)[NRB][NCB],
-                                         int nstage, int nkc, int arow, int bcol, int h) {
-  constexpr int AEL = TileShape<C_::A_KC, TM>::ELEMS, BEL = TileShape<C_::B_KC, TN>::ELEMS;
-  int kb = 0, kc = 0;
-  auto advance = [&]() { if (++kc == nkc) { kc = 0; ++kb; } };
-  la.load(0, 0);
-  lb.load(0, 0);
-  la.store(As);
-  lb.store(Bs);
-  advance();
-  if (nstage > 1) {
-    la.load(kb, kc * TK);
-    lb.load(kb, kc * TK);
-  }
+constexpr int CLD = TM;           // row pitch (floats) of the products on their way to the combination
+union Smem {
+  struct { OperandTile a, b; } stage[2];
+  float product[3][64][CLD];
+};
+
+// a thread without a share of the loads
+struct NoLoader {
+  __device__ __forceinline__ void load() {}
+};
+
+// The contraction loop of group G.  While the matrix cores take stage s from one buffer, the first two groups cut the operands
+// of stage s + 1 (group 0 those of A, group 1 those of B, fetched during stage s - 1) into the other; one barrier per stage.
+// Group 0 cuts first and multiplies second, group 1 the other way round: a SIMD holds one wave of each group, and one at most
+// has the vector unit to itself while the others feed the matrix cores.
+template <int G, bool FULL, bool CONJ, typename LD>
+__device__ __forceinline__ void contract(LD& ld, Smem& s, v16f (&acc)[NB][NB], int nstage, int row, int octet, int arow, int bcol, int h, int ni, int nj) {
+  auto put = [&](int buf) {
+    if constexpr (G == 0) s.stage[buf].a.template put<false>(row, octet, ld.reg[0]);
+    if constexpr (G == 1) s.stage[buf].b.template put<CONJ>(row, octet, ld.reg[0]);
+  };
+  auto mma = [&](int buf) {
+    SplitFragment a[NB], b[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) a[i] = s.stage[buf].a.kind[G].get(arow + BSTR * i, h);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) b[j] = s.stage[buf].b.kind[G].get(bcol + BSTR * j, h);
+    if (FULL) {
+      s2cnn::split_mma<NB, NB>(a, b, acc);
+    } else {
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          if (i < ni && j < nj) s2cnn::split_mma_one(a[i], b[j], acc[i][j]);
+    }
+  };
+  ld.load();
+  put(0);
+  if (nstage > 1) ld.load();
   __syncthreads();
   for (int stage = 0; stage < nstage; ++stage) {
     const int cur = stage & 1;
-    if (stage + 1 < nstage) {
-      la.store(As + (cur ^ 1) * AEL);       // that buffer was last read in stage - 1, which every wave has left
-      lb.store(Bs + (cur ^ 1) * BEL);
-      advance();
-      if (stage + 2 < nstage) {
-        la.load(kb, kc * TK);
-        lb.load(kb, kc * TK);
-      }
+    if (G != 0) mma(cur);
+    if (stage + 1 < nstage) {                  // the other buffer was last read in stage - 1, which every wave has left
+      put(cur ^ 1);
+      if (stage + 2 < nstage) ld.load();
     }
-    if (NI > 0 && NJ > 0)
-      stage_mma<C_, (NI > 0 ? NI : 1), (NJ > 0 ? NJ : 1)>(As + cur * AEL, Bs + cur * BEL, acc, arow, bcol, h);
+    if (G == 0) mma(cur);
     __syncthreads();
   }
 }
 
-__host__ __device__ inline void tile_counts(int L, int RI, int CI, int& tm, int& tn, int& slots) {
-  tm = s2cnn::ceil_div(L * RI, TM);
-  tn = s2cnn::ceil_div(L * CI, TN);
-  slots = tm * tn;   // every workgroup of the grid has a tile: idle workgroups stall the dispatcher
-}
-
-template <int MODE, int VEC>
-__global__ __launch_bounds__(NT, MODE == GRADX ? 2 : 3) void so3_block_mm_kernel(MmParams p) {   // grad x: two K-contiguous tiles leave LDS for two workgroups
+// Complex arithmetic on a real matrix core, three real products per complex one (Gauss): with
+// b = br + i bi' (bi' = -bi where the operand is conjugated)
+//     P1 = sum ar br,   P2 = sum ai bi',   P3 = sum (ar + ai)(br + bi')
+//     re = P1 - P2,     im = P3 - P1 - P2.
+// A workgroup of twelve waves owns 128 x 128 outputs; each of its three groups of four forms one of the real products of the
+// tile, operands cut into three bf16 parts once per tile and read by the group that needs them (the sums are formed in
+// float32 before they are cut, so the imaginary part carries a rounding error of the size of |a||b| eps rather than of its own
+// size: the bound of any float32 complex product).  The products meet in LDS at the end.
+//
+// Why three groups: a wave that forms all three products of 2 x 2 blocks needs 192 accumulator registers (one wave per SIMD), and
+// of 2 x 1 blocks reads 27 KB of LDS for 36 matrix instructions, more clocks than these take; a wave of a group reads 12 KB
+// for 24 and holds 64 accumulators, three waves per SIMD.  LDS: 1 728 of the 2 304 clocks of matrix instructions per stage.
+// One workgroup per CU (149 KB), tiles listed in bands and dealt to the XCDs in runs as in so3_mm_real.hip.
+//
+// Measured (us, fwd / gradx / grady; before: v_mfma_f32_32x32x2_f32 in tiles of 128 x 64, at 77 % of its peak):
+//   32 degrees, batch 16,  64 ->  64:  6849 / 6839 / 6553 -> 4312 / 4240 / 4294, 1.15 PFLOP/s of bf16 instructions, the rate that
+//                                      the real product reaches as well (energy: the clock falls with the power drawn)
+//   22 degrees, batch 32, 100 -> 100:  8190 / 8365 / 7246 -> 4670 / 4719 / 4592
+//   16 degrees, batch 16,  64 ->  64:   539 /  588 /  465 ->  366 /  363 /  300
+//   24 degrees, batch  4,  30 ->  30:   277 /  267 /  503 ->  154 /  153 /  127
+// Errors against 64 bits (relative 2-norm) at the first size 1.56e-6 / 1.56e-6 / 7.8e-7 -> 1.33e-6 / 1.33e-6 / 6.6e-7, smaller at all
+// sizes measured.
+template <int MODE, int VA, int VB, int HOW, int GA, int GB>
+__global__ __launch_bounds__(NT, 3) void so3_block_mm_kernel(MmParams p) {
   typedef Cfg<MODE> C_;
-  __shared__ __attribute__((aligned(16))) float2 As[2 * TileShape<C_::A_KC, TM>::ELEMS];
-  __shared__ __attribute__((aligned(16))) float2 Bs[2 * TileShape<C_::B_KC, TN>::ELEMS];
+  __shared__ __attribute__((aligned(16))) Smem s;
 
-  // ---- which tile: degrees in descending order so the heaviest tiles are dispatched first
   int t = blockIdx.x;
-  int l = p.nl - 1, tm = 0, tn = 0, slots = 0;
-  for (;; --l) {
-    tile_counts(2 * l + 1, p.RI, p.CI, tm, tn, slots);
-    if (t < slots || l == 0) break;
-    t -= slots;
-  }
-  const int r = t;                                  // row tiles run fastest within a degree
-  const int tile_nq = r / tm;
+  constexpr int ROUND = 8 * XCD_RUN;
+  if (t < (int)gridDim.x / ROUND * ROUND) t = t / ROUND * ROUND + t % 8 * XCD_RUN + t % ROUND / 8;
+  int tm = 0, tn = 0;
+  const int l = find_degree(p, TM, TM, t, tm, tn);
   const int L = 2 * l + 1;
-  const int tile_m = (r % tm) * TM;
-  const int tile_n = tile_nq * TN;
+  const int band = t / (BAND * tn), bm = tm - band * BAND < BAND ? tm - band * BAND : BAND, tb = t - band * BAND * tn;
+  const int tile_m = (band * BAND + tb % bm) * TM;
+  const int tile_n = tb / bm * TM;
   const size_t L0 = (size_t)l * (4 * l * l - 1) / 3;
   const int M = L * p.RI, N = L * p.CI;
-
-  TileLoader<C_::A_KC, C_::A_MNMAJ, TM, VEC> la;
-  TileLoader<C_::B_KC, C_::B_MNMAJ, TN, VEC> lb;
-  la.init(p.A + L0 * p.RI * p.KI, L, p.RI, p.KI, tile_m);
-  lb.init(p.B + L0 * p.CI * p.KI, L, p.CI, p.KI, tile_n);
+  const float2* A = p.A + L0 * p.RI * p.KI;
+  const float2* B = p.B + L0 * p.CI * p.KI;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = wave >> 2;
   const int r32 = lane & 31, h = lane >> 5;
-  const int wrow = (wave >> 1) * WSTR, wcol = (wave & 1) * WSTR;
+  const int wrow = ((wave >> 1) & 1) * WSTR, wcol = (wave & 1) * WSTR;
 
-  Acc3 acc[NRB][NCB];
+  v16f acc[NB][NB];
 #pragma unroll
-  for (int i = 0; i < NRB; ++i)
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < NCB; ++j)
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) { acc[i][j].p1[v] = 0.f; acc[i][j].p2[v] = 0.f; acc[i][j].p3[v] = 0.f; }
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
 
-  // live blocks of this wave: rows tile_m + wrow + 64 i < M, columns tile_n + wcol + 64 j < N (prefixes of i, j)
   const int remr = M - tile_m - wrow, remc = N - tile_n - wcol;
   int ni = remr <= 0 ? 0 : (remr + BSTR - 1) / BSTR, nj = remc <= 0 ? 0 : (remc + BSTR - 1) / BSTR;
-  ni = ni > NRB ? NRB : ni;
-  nj = nj > NCB ? NCB : nj;
-  if (ni == 0 || nj == 0) ni = nj = 0;
-
-  const int nkc = s2cnn::ceil_div(p.KI, TK);
-  const int nstage = L * nkc;
-  // one specialised copy of the whole contraction loop per count of live blocks (wave-uniform choice)
-#define S2CNN_CONTRACT(I, J) contract<C_, I, J>(la, lb, As, Bs, acc, nstage, nkc, wrow + r32, wcol + r32, h)
-  if (nj == NCB) {
-    switch (ni) {
-      case 4: if (NRB >= 4) { S2CNN_CONTRACT((NRB >= 4 ? 4 : 1), NCB); } break;
-      case 3: if (NRB >= 3) { S2CNN_CONTRACT((NRB >= 3 ? 3 : 1), NCB); } break;
-      case 2: if (NRB >= 2) { S2CNN_CONTRACT((NRB >= 2 ? 2 : 1), NCB); } break;
-      case 1: S2CNN_CONTRACT(1, NCB); break;
-      default: S2CNN_CONTRACT(0, 0); break;
-    }
-  } else if (nj == 0) {
-    S2CNN_CONTRACT(0, 0);
-  } else if constexpr (NCB > 1) {  // one live column block of two
-    switch (ni) {
-      case 4: if (NRB >= 4) { S2CNN_CONTRACT((NRB >= 4 ? 4 : 1), 1); } break;
-      case 3: if (NRB >= 3) { S2CNN_CONTRACT((NRB >= 3 ? 3 : 1), 1); } break;
-      case 2: if (NRB >= 2) { S2CNN_CONTRACT((NRB >= 2 ? 2 : 1), 1); } break;
-      default: S2CNN_CONTRACT(1, 1); break;
-    }
+  ni = ni > NB ? NB : ni;
+  nj = nj > NB ? NB : nj;
+  const bool full = ni == NB && nj == NB;
+  const int nstage = s2cnn::ceil_div(L * p.KI, TK);
+  const int u = threadIdx.x & (GROUP - 1);
+  const auto finite = [&]() {
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) ok = ok && is_finite(acc[i][j][v]);
+    return __all(ok);
+  };
+#define S2CNN_GROUP(G, LDR)                                                                                                       \
+  do {                                                                                                                            \
+    if (full) contract<G, true, C_::CONJ>(LDR, s, acc, nstage, row, octet, wrow + r32, wcol + r32, h, ni, nj);                     \
+    else contract<G, false, C_::CONJ>(LDR, s, acc, nstage, row, octet, wrow + r32, wcol + r32, h, ni, nj);                         \
+    if (!finite()) contract_float32<C_, G, NB, NB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);            \
+  } while (0)
+  if (group == 0) {            // K-contiguous: two threads on a row; MN-contiguous: neighbouring threads on neighbouring rows
+    const int row = C_::A_KC ? u >> 1 : u & (TM - 1), octet = C_::A_KC ? u & 1 : u / TM;
+    Loader<float2, C_::A_KC, C_::A_MNMAJ, 1, 1, VA, HOW, GA, TK> ld;
+    ld.init(A, L, p.RI, p.KI, tile_m + row, 8 * octet);
+    S2CNN_GROUP(0, ld);
+  } else if (group == 1) {
+    const int row = C_::B_KC ? u >> 1 : u & (TM - 1), octet = C_::B_KC ? u & 1 : u / TM;
+    Loader<float2, C_::B_KC, C_::B_MNMAJ, 1, 1, VB, HOW, GB, TK> ld;
+    ld.init(B, L, p.CI, p.KI, tile_n + row, 8 * octet);
+    S2CNN_GROUP(1, ld);
+  } else {
+    const int row = 0, octet = 0;
+    NoLoader ld;
+    S2CNN_GROUP(2, ld);
   }
-#undef S2CNN_CONTRACT
+#undef S2CNN_GROUP
 
-  // ---- write the sub-tile.  Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4
-  // and column r32 of its 32x32 block.
+  // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32 of its 32x32 block.  64 rows of the tile at a
+  // time; a thread stores every sixth row of one column.
   float2* Cl = p.C + L0 * p.RI * p.CI;
   const int blk_elems = p.RI * p.CI;
+  const int ct = threadIdx.x % TM, col = tile_n + ct;
+  const int cb = col / p.CI, ci = col - cb * p.CI;
 #pragma unroll
-  for (int j = 0; j < NCB; ++j) {
-    const int col = tile_n + wcol + BSTR * j + r32;
-    if (j >= nj || col >= N) continue;
-    const int cb = col / p.CI, ci = col - cb * p.CI;
+  for (int i = 0; i < NB; ++i) {
+    if (i) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NRB; ++i) {
-      if (i >= ni) continue;
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = tile_m + wrow + BSTR * i + 8 * (v / 4) + 4 * h + (v % 4);
-        if (row < M) {
-          const int rb = row / p.RI, ri = row - rb * p.RI;
-          const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
-          const float p1 = acc[i][j].p1[v], p2 = acc[i][j].p2[v];
-          Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = make_float2(p1 - p2, acc[i][j].p3[v] - p1 - p2);
-        }
+      for (int v = 0; v < 16; ++v)
+        s.product[group][wrow + 8 * (v / 4) + 4 * h + v % 4][wcol + BSTR * j + r32] = acc[i][j][v];
+    __syncthreads();
+    if (col < N) {
+      for (int r = threadIdx.x / TM; r < 64; r += NT / TM) {
+        const int row = tile_m + BSTR * i + r;
+        if (row >= M) break;
+        const int rb = row / p.RI, ri = row - rb * p.RI;
+        const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
+        const float p1 = s.product[RE][r][ct], p2 = s.product[IM][r][ct];
+        Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = make_float2(p1 - p2, s.product[SUM][r][ct] - p1 - p2);
       }
     }
   }
 }
 
-int total_slots(int nl, int RI, int CI) {
+__device__ __forceinline__ uint4 flip_signs(uint4 v) { return make_uint4(v.x ^ 0x80008000u, v.y ^ 0x80008000u, v.z ^ 0x80008000u, v.w ^ 0x80008000u); }
+__device__ __forceinline__ s2cnn::v8bf negated(s2cnn::v8bf v) {
+  return __builtin_bit_cast(s2cnn::v8bf, flip_signs(__builtin_bit_cast(uint4, v)));
+}
+
+// Small problems: too few 128 x 128 tiles to fill the chip.  A workgroup owns 32 x 32 outputs, its four waves take every
+// fourth 16 steps of the contraction; a lane loads the octets it feeds to the matrix instruction straight from memory (no LDS,
+// no barriers, the next octets in flight meanwhile) and the four partial sums meet in LDS at the end.  What bounds it is the
+// cutting of operands that each wave has to itself, so the four products of the direct form take the place of three with
+// sums that would have to be cut as well (and the errors halve).
+// us of fwd / gradx / grady, float32 kernel before -> tiles of 128 x 128 -> this one: 6 degrees, batch 32, 20 -> 40: 49 / 66 / 49 -> 30 / 48 / 40
+// -> 12 / 12 / 11; 13 degrees, batch 11, 33 -> 45: 178 / 151 / 109 -> 96 / 134 / 65 -> 70 / 91 / 72.  The line, in 32 x 32 tiles: 1 792 (32
+// degrees, batch 1, 32 -> 32) 190 us in tiles of 128, 144 here; 2 460 (24 degrees, batch 4, 30 -> 30) 154 and 165; 2 720 24.7 and 26;
+// 3 174 59 and 69; 4 148 equal; 5 712 366 and 466.
+template <int MODE, int VA, int VB, int HOW, int GR>
+__global__ __launch_bounds__(NTS) void so3_block_mm_slices_kernel(MmParams p) {
+  typedef Cfg<MODE> C_;
+  constexpr int NW = NTS / 64, T = 32, ADV = 16 * NW;
+  __shared__ float part[NW][2][16][64];
+
+  int t = blockIdx.x, tm = 0, tn = 0;
+  const int l = find_degree(p, T, T, t, tm, tn);
+  const int L = 2 * l + 1;
+  const int tile_m = t % tm * T, tile_n = t / tm * T;
+  const size_t L0 = (size_t)l * (4 * l * l - 1) / 3;
+  const int M = L * p.RI, N = L * p.CI;
+  const float2* A = p.A + L0 * p.RI * p.KI;
+  const float2* B = p.B + L0 * p.CI * p.KI;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r32 = lane & 31, h = lane >> 5;
+
+  Loader<float2, C_::A_KC, C_::A_MNMAJ, 1, 1, VA, HOW, GR, ADV> la;
+  Loader<float2, C_::B_KC, C_::B_MNMAJ, 1, 1, VB, HOW, GR, ADV> lb;
+  la.init(A, L, p.RI, p.KI, tile_m + r32, 16 * wave + 8 * h);
+  lb.init(B, L, p.CI, p.KI, tile_n + r32, 16 * wave + 8 * h);
+
+  v16f re, im;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) { re[v] = 0.f; im[v] = 0.f; }
+  const auto split = [](const float2 (&v)[8], SplitFragment& r, SplitFragment& i) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = v[e].x;
+    r = s2cnn::split_octet(x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = v[e].y;
+    i = s2cnn::split_octet(x);
+  };
+  const int nstep = s2cnn::ceil_div(L * p.KI, ADV);      // the same for all waves: steps behind the end are zeros
+  la.load();
+  lb.load();
+  for (int step = 0; step < nstep; ++step) {
+    SplitFragment ar, ai, br, bi;
+    split(la.reg[0], ar, ai);
+    split(lb.reg[0], br, bi);
+    if (step + 1 < nstep) {
+      la.load();
+      lb.load();
+    }
+    const SplitFragment bn{negated(bi.h), negated(bi.m), negated(bi.l)};
+    // conjugated b: re = ar br + ai bi, im = ai br - ar bi; else re = ar br - ai bi, im = ai br + ar bi
+#define S2CNN_PARTS(PA, PB)                                                                                           \
+    re = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ar.PA, br.PB, re, 0, 0, 0);                                          \
+    im = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ai.PA, br.PB, im, 0, 0, 0);                                          \
+    re = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ai.PA, C_::CONJ ? bi.PB : bn.PB, re, 0, 0, 0);                       \
+    im = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ar.PA, C_::CONJ ? bn.PB : bi.PB, im, 0, 0, 0);
+    S2CNN_PARTS(l, h)
+    S2CNN_PARTS(h, l)
+    S2CNN_PARTS(m, m)
+    S2CNN_PARTS(m, h)
+    S2CNN_PARTS(h, m)
+    S2CNN_PARTS(h, h)
+#undef S2CNN_PARTS
+  }
+
+  // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32; wave w adds up and stores v = 4w .. 4w+3.
+#pragma unroll
+  for (int v = 0; v < 16; ++v) { part[wave][0][v][lane] = re[v]; part[wave][1][v][lane] = im[v]; }
+  __syncthreads();
+  float2 sum[4];
+  bool finite = true;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float2 z = make_float2(part[0][0][4 * wave + v][lane], part[0][1][4 * wave + v][lane]);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) { z.x += part[w][0][4 * wave + v][lane]; z.y += part[w][1][4 * wave + v][lane]; }
+    sum[v] = z;
+    finite = finite && is_finite(z.x) && is_finite(z.y);
+  }
+  if (!__all(finite)) {
+    v16f p1[1][1], p2[1][1], p3[1][1];
+    contract_float32<C_, RE, 1, 1, 32>(p, A, B, p1, L, tile_m + r32, tile_n + r32, h);
+    contract_float32<C_, IM, 1, 1, 32>(p, A, B, p2, L, tile_m + r32, tile_n + r32, h);
+    contract_float32<C_, SUM, 1, 1, 32>(p, A, B, p3, L, tile_m + r32, tile_n + r32, h);
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      if (v / 4 == wave) sum[v % 4] = make_float2(p1[0][0][v] - p2[0][0][v], p3[0][0][v] - p1[0][0][v] - p2[0][0][v]);
+  }
+
+  float2* Cl = p.C + L0 * p.RI * p.CI;
+  const int col = tile_n + r32;
+  if (col >= N) return;
+  const int cb = col / p.CI, ci = col - cb * p.CI;
+  const int row0 = tile_m + 8 * wave + 4 * h;
+  int rb = row0 / p.RI, ri = row0 - rb * p.RI;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    if (row0 + v < M) {
+      const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
+      Cl[(size_t)blk * (p.RI * p.CI) + ri * p.CI + ci] = sum[v];
+    }
+    if (++ri == p.RI) { ri = 0; ++rb; }
+  }
+}
+
+long total_slots(int nl, int RI, int CI, int TMV, int TNV) {
   long n = 0;
   for (int l = 0; l < nl; ++l) {
-    int tm, tn, slots;
-    tile_counts(2 * l + 1, RI, CI, tm, tn, slots);
-    n += slots;
+    int tm, tn;
+    n += tile_counts(2 * l + 1, RI, CI, TMV, TNV, tm, tn);
   }
-  return n > 0x7fffffffL ? -1 : (int)n;
+  return n > 0x7fffffffL ? -1 : n;
 }
 
 template <int MODE>
@@ -373,20 +449,33 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
   const long Lmax = 2L * nl - 1;
   if (Lmax * Lmax * RI * KI >= (1L << 31) || Lmax * Lmax * CI * KI >= (1L << 31)) return S2CNN_EINVAL;
   if (!s2cnn::aligned8(a) || !s2cnn::aligned8(b) || !s2cnn::aligned8(c)) return S2CNN_EALIGN;
-  const int grid = total_slots(nl, RI, CI);
-  if (grid < 1) return S2CNN_EINVAL;
+  const long grid = total_slots(nl, RI, CI, TM, TM), small = total_slots(nl, RI, CI, 32, 32);
+  if (total_slots(nl, RI, CI, 128, 64) < 1) return S2CNN_EINVAL;      // a grid beyond 2^31 - 1
   MmParams p{reinterpret_cast<const float2*>(a), reinterpret_cast<const float2*>(b),
              reinterpret_cast<float2*>(c), nl, RI, CI, KI};
   typedef Cfg<MODE> C_;
-  // two complex numbers per access need the fast index of each operand to be even and 16-byte bases
-  const bool a_even = C_::A_KC ? (KI % 2 == 0) : (RI % 2 == 0);
-  const bool b_even = C_::B_KC ? (KI % 2 == 0) : (CI % 2 == 0);
-  const bool vec2 = a_even && b_even && s2cnn::aligned16(a) && s2cnn::aligned16(b);
+  // two complex numbers per access need a K-contiguous operand of even length and a 16-byte base
+  const bool pairs = KI % 2 == 0 && (!C_::A_KC || s2cnn::aligned16(a)) && (!C_::B_KC || s2cnn::aligned16(b));
+  const bool near = Lmax * Lmax * RI * KI < (1L << 28) && Lmax * Lmax * CI * KI < (1L << 28);   // byte offsets below OUTSIDE
+  const bool divides = near && pairs && KI % 8 == 0 && (KI % TK == 0 || TK % KI == 0);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (vec2)
-    hipLaunchKernelGGL((so3_block_mm_kernel<MODE, 2>), dim3(grid), dim3(NT), 0, st, p);
-  else
-    hipLaunchKernelGGL((so3_block_mm_kernel<MODE, 1>), dim3(grid), dim3(NT), 0, st, p);
+#define S2CNN_LAUNCH(V, HOW, GR) \
+  hipLaunchKernelGGL((so3_block_mm_kernel<MODE, (C_::A_KC ? V : 1), (C_::B_KC ? V : 1), HOW, GR, GR>), dim3((unsigned)grid), dim3(NT), 0, st, p)
+#define S2CNN_SLICES(V, GR) \
+  hipLaunchKernelGGL((so3_block_mm_slices_kernel<MODE, (C_::A_KC ? V : 1), (C_::B_KC ? V : 1), WALK, GR>), dim3((unsigned)small), dim3(NTS), 0, st, p)
+  if (near && small > 0 && small < SMALL_TILES) {
+    if (pairs && KI % 4 == 0) S2CNN_SLICES(2, 4);
+    else if (pairs) S2CNN_SLICES(2, 2);
+    else S2CNN_SLICES(1, 1);
+    return s2cnn::launch_status();
+  }
+  if (!near) S2CNN_LAUNCH(1, FAR, 1);
+  else if (divides) S2CNN_LAUNCH(2, DIVIDES, 8);
+  else if (pairs && KI % 4 == 0) S2CNN_LAUNCH(2, WALK, 4);
+  else if (pairs) S2CNN_LAUNCH(2, WALK, 2);
+  else S2CNN_LAUNCH(1, WALK, 1);
+#undef S2CNN_LAUNCH
+#undef S2CNN_SLICES
   return s2cnn::launch_status();
 }
 

@@ -31,9 +31,11 @@
 // Tried and not kept: three workgroups per CU (168 registers): 0 to 2 % slower.
 #include "common.h"
 #include "split_bf16.h"
+#include "block_loader.h"
 
 namespace {
 
+using namespace s2cnn::block;
 using s2cnn::v16f;
 using s2cnn::SplitTile;
 
@@ -47,18 +49,8 @@ constexpr int XCD_RUN = 32;       // consecutive tiles of the list that one XCD 
 constexpr int SMALL_GRID = 512;   // workgroups that fill the chip (2 per CU)
 constexpr int SLICES_GRID = 256;  // fewer 128 x 64 tiles than this: the kernel for small problems
 constexpr int SLICES_WIDE = 400;  // as many 32 x 64 tiles: two blocks per wave of it
-constexpr unsigned OUTSIDE = 0x80000000u;   // a byte offset behind the end of every buffer: such loads return 0
 
 enum Mode { FWD = 0, GRADX = 1, GRADY = 2 };
-// How the contraction index (the flattened pair block, feature; KI features per block) is walked:
-//   DIVIDES  KI a multiple of 8 and KI, TK divide one another: an octet of steps never straddles a block and every stage
-//            starts at the same place inside a block, so a thread's offsets are fixed and a stage advances by a
-//            wave-uniform step
-//   WALK     any KI: every thread follows its own position (block, feature), in granules of GR steps (GR = 4, 2 or 1 divides
-//            KI, so a granule lies in one block)
-//   FAR      the same for operands whose degrees exceed 32-bit byte offsets
-enum Walk { DIVIDES = 0, WALK = 1, FAR = 2 };
-
 struct MmParams {
   const float* A;
   const float* B;
@@ -75,129 +67,10 @@ template <> struct Cfg<FWD>   { static constexpr bool A_KC = true,  B_KC = false
 template <> struct Cfg<GRADX> { static constexpr bool A_KC = true,  B_KC = true,  A_MNMAJ = true,  B_MNMAJ = false, C_RMAJ = true;  };
 template <> struct Cfg<GRADY> { static constexpr bool A_KC = false, B_KC = false, A_MNMAJ = false, B_MNMAJ = false, C_RMAJ = false; };
 
-template <int VEC> struct VecT { typedef float type; };
-template <> struct VecT<2> { typedef float2 type; };
-template <> struct VecT<4> { typedef float4 type; };
-
-// One operand's loader.  A thread owns NMN rows (ROWSTEP apart) of 8 contraction steps, starting at step k0 and ADV further on with
-// every load(): an octet of a row is what a lane feeds to the matrix instruction, and what one 16-byte LDS store takes,
-// whichever index is the fast one in memory.  VEC = floats per global access, along the contraction (K-contiguous) or along
-// the rows (MN-contiguous).  Rows outside the matrix and steps behind the last block are loaded from OUTSIDE, that is as
-// zeros.
-template <bool KC, bool MNMAJ, int NMN, int ROWSTEP, int VEC, int HOW, int GR, int ADV>
-struct Loader {
-  static_assert(NMN >= 1 && (KC || VEC == 1 || (VEC <= NMN && ROWSTEP == 1)) && (HOW != DIVIDES || ADV == TK), "no such loader");
-  typedef typename VecT<VEC>::type vec_t;
-
-  float reg[NMN][8];
-  const float* base;
-  __amdgpu_buffer_rsrc_t rsrc;
-  unsigned off[NMN];            // offset of the row (DIVIDES: and of the octet): bytes, FAR: floats; OUTSIDE for no row
-  int MNI, KI, L, blk_k_stride;
-  int kb, kin, adv_b, adv_k;    // WALK, FAR: block and feature of this thread's first step; what a stage adds to them
-  unsigned soff, step_in, step_cross;   // DIVIDES: uniform byte offset of the stage and its increments
-  int sub, nsub, stage_i, last_ragged;
-  bool tail_ok;
-
-  __device__ __forceinline__ void init(const float* base_l, int L_, int MNI_, int KI_, int row0, int k0) {
-    base = base_l; MNI = MNI_; KI = KI_; L = L_;
-    const int blk_elems = MNI * KI;
-    const int blk_mn_stride = (MNMAJ ? L : 1) * blk_elems;
-    blk_k_stride = (MNMAJ ? 1 : L) * blk_elems;
-    const int unit = KC ? 1 : MNI;                       // stride of one contraction step inside a block
-    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base_l), 0, HOW == FAR ? 0 : 4 * L * L * MNI * KI, 0x00020000);
-    kb = k0 / KI;
-    kin = k0 - kb * KI;
-    const int K = L * KI, nstage = (K + TK - 1) / TK, ktail = K - (nstage - 1) * TK;
-#pragma unroll
-    for (int q = 0; q < NMN; ++q) {
-      const int row = row0 + q * ROWSTEP;
-      const int mb = row / MNI, mi = row - mb * MNI;
-      unsigned o = (unsigned)(mb * blk_mn_stride + mi * (KC ? KI : 1));
-      if (HOW == DIVIDES) o += (unsigned)((KI >= TK ? 0 : kb) * blk_k_stride + kin * unit);
-      off[q] = row >= L * MNI ? OUTSIDE : HOW == FAR ? o : 4u * o;
-    }
-    if (HOW == DIVIDES) {
-      soff = 0; sub = 0; stage_i = 0;
-      if (KI >= TK) { nsub = KI / TK; step_in = 4u * TK * unit; step_cross = 4u * (unsigned)(blk_k_stride - (KI - TK) * unit); }
-      else { nsub = 1; step_in = 0; step_cross = 4u * (unsigned)(TK / KI * blk_k_stride); }
-      last_ragged = ktail < TK ? nstage - 1 : -1;
-      tail_ok = k0 < ktail;
-    } else {
-      adv_b = ADV / KI;
-      adv_k = ADV - adv_b * KI;
-    }
-  }
-
-  __device__ __forceinline__ vec_t fetch(unsigned o, unsigned so) const {
-    if constexpr (HOW == FAR) {
-      static_assert(HOW != FAR || VEC == 1, "operands beyond 32-bit byte offsets are read one float at a time");
-      return o == OUTSIDE ? 0.f : base[o];
-    } else if constexpr (VEC == 4) {
-      typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)o, (int)so, 0);
-      return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    } else if constexpr (VEC == 2) {
-      typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)o, (int)so, 0);
-      return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
-    } else {
-      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)o, (int)so, 0));
-    }
-  }
-
-  // the values of access (row q, step e): K-contiguous VEC steps of one row, MN-contiguous one step of VEC rows
-  __device__ __forceinline__ void put(int q, int e, vec_t v) {
-    if constexpr (VEC == 1) reg[q][e] = v;
-    else if constexpr (KC && VEC == 2) { reg[q][e] = v.x; reg[q][e + 1] = v.y; }
-    else if constexpr (KC && VEC == 4) { reg[q][e] = v.x; reg[q][e + 1] = v.y; reg[q][e + 2] = v.z; reg[q][e + 3] = v.w; }
-    else { reg[q][e] = v.x; reg[q + 1][e] = v.y; }
-  }
-
-  // fetches the current stage and steps to the next one
-  __device__ __forceinline__ void load() {
-    constexpr int QS = KC ? 1 : VEC, ES = KC ? VEC : 1;
-    if (HOW == DIVIDES) {
-      const bool ok = stage_i != last_ragged || tail_ok;
-#pragma unroll
-      for (int q = 0; q < NMN; q += QS) {
-        const unsigned o = ok ? off[q] : OUTSIDE;
-#pragma unroll
-        for (int e = 0; e < 8; e += ES)
-          put(q, e, KC ? fetch(o + 4u * e, soff) : fetch(o, soff + 4u * (unsigned)(e * MNI)));
-      }
-      ++stage_i;
-      if (++sub == nsub) { sub = 0; soff += step_cross; }
-      else soff += step_in;
-      return;
-    }
-    const unsigned scale = HOW == FAR ? 1u : 4u, unit = scale * (unsigned)(KC ? 1 : MNI), bstride = scale * (unsigned)blk_k_stride;
-    const unsigned cross = bstride - (unsigned)KI * unit;      // from behind the end of a block to the start of the next
-    int k = kin, b = kb;
-    unsigned o = (unsigned)b * bstride + (unsigned)k * unit;
-#pragma unroll
-    for (int g = 0; g < 8; g += GR) {
-#pragma unroll
-      for (int q = 0; q < NMN; q += QS) {
-        const unsigned at = b < L && (HOW != FAR || off[q] != OUTSIDE) ? off[q] + o : OUTSIDE;   // OUTSIDE + o is outside as well
-#pragma unroll
-        for (int e = 0; e < GR; e += ES)
-          put(q, g + e, KC ? fetch(at + 4u * e, 0) : fetch(at, e * unit));
-      }
-      k += GR;
-      o += (unsigned)GR * unit;
-      if (k >= KI) { k = 0; ++b; o += cross; }                // KI is a multiple of GR
-    }
-    kin += adv_k;
-    kb += adv_b;
-    if (kin >= KI) { kin -= KI; ++kb; }
-  }
-};
-
 // The loader of a workgroup's tile of EXT rows and TK steps: K-contiguous, TK / 8 threads on a row; MN-contiguous, neighbouring
 // threads on neighbouring rows.
 template <bool KC, bool MNMAJ, int EXT, int VEC, int HOW, int GR>
-struct TileLoader : Loader<KC, MNMAJ, EXT * TK / (NT * 8), KC ? NT / (TK / 8) : 1, VEC, HOW, GR, TK> {
+struct TileLoader : Loader<float, KC, MNMAJ, EXT * TK / (NT * 8), KC ? NT / (TK / 8) : 1, VEC, HOW, GR, TK> {
   static constexpr int NMN = EXT * TK / (NT * 8), ROWSTEP = KC ? NT / (TK / 8) : 1;
   int row0, octet;
 
@@ -205,7 +78,7 @@ struct TileLoader : Loader<KC, MNMAJ, EXT * TK / (NT * 8), KC ? NT / (TK / 8) : 
     const int t = threadIdx.x;
     octet = KC ? t % (TK / 8) : t / (EXT / NMN);
     row0 = KC ? t / (TK / 8) : (t % (EXT / NMN)) * NMN;
-    Loader<KC, MNMAJ, NMN, ROWSTEP, VEC, HOW, GR, TK>::init(base_l, L, MNI, KI, tile0 + row0, 8 * octet);
+    Loader<float, KC, MNMAJ, NMN, ROWSTEP, VEC, HOW, GR, TK>::init(base_l, L, MNI, KI, tile0 + row0, 8 * octet);
   }
 
   __device__ __forceinline__ void store(SplitTile<EXT, TK>& tile) const {
@@ -427,8 +300,8 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r32 = lane & 31, h = lane >> 5;
 
-  Loader<C_::A_KC, C_::A_MNMAJ, 1, 1, VA, HOW, GR, ADV> la;
-  Loader<C_::B_KC, C_::B_MNMAJ, NJ, 32, VB, HOW, GR, ADV> lb;
+  Loader<float, C_::A_KC, C_::A_MNMAJ, 1, 1, VA, HOW, GR, ADV> la;
+  Loader<float, C_::B_KC, C_::B_MNMAJ, NJ, 32, VB, HOW, GR, ADV> lb;
   la.init(A, L, p.RI, p.KI, tile_m + r32, 16 * wave + 8 * h);
   lb.init(B, L, p.CI, p.KI, tile_n + r32, 16 * wave + 8 * h);
 

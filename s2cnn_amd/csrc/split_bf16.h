@@ -44,9 +44,9 @@ __device__ __forceinline__ SplitFragment split_octet(const float (&x)[8]) {
 // The parts of EXT rows x TK contraction steps in LDS: per part and octet of steps one 16-byte slot per row.  A lane's operand
 // of the matrix instruction is one slot.  Two slots of padding per octet and the exchange of neighbouring slots in every
 // other group of eight rows keep the stores (four octets of neighbouring rows, or every other row of one octet) and the
-// loads (neighbouring rows of one octet) of eight lanes in different banks.
+// loads (neighbouring rows of one octet) of eight lanes in different banks; with two octets (TK = 16: four rows of both) four.
 template <int EXT, int TK> struct SplitTile {
-  static constexpr int LD = EXT + 2;
+  static constexpr int LD = EXT + (TK == 16 ? 4 : 2);
   uint4 part[3][TK / 8][LD];
 
   static __device__ __forceinline__ int slot(int row) { return row ^ ((row >> 3) & 1); }

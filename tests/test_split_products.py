@@ -63,6 +63,70 @@ def test_real_product_edges(hip, nl, B, Fi, Fo, aligned):
         assert ((got.double() - want).norm() / want.norm()).item() <= bound(K)
 
 
+def product64_complex(which, a, b, nl):
+    """The same of complex operands [..., 2]: x conj(y), gz y, x conj(gz)."""
+    (ar, ai), (br, bi) = a.unbind(-1), b.unbind(-1)
+    ai, bi = -ai if which == "grady" else ai, -bi if which == "fwd" else bi
+    return torch.stack((product64(which, ar, br, nl) - product64(which, ai, bi, nl),
+                        product64(which, ai, br, nl) + product64(which, ar, bi, nl)), -1)
+
+
+# The three real products of the Gauss form carry sqrt(2) times the error of a real product of the same length relative to the
+# complex result (variances K + K of the real part, 4 K + K + K of the imaginary one, over 4 K), the sums of operands one more rounding.
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [
+    # 32 x 32 outputs: one row, one block and one more, one 16-step and one more
+    (1, 1, 1, 1), (1, 32, 16, 32), (1, 33, 17, 65), (3, 1, 7, 20), (6, 1, 20, 40), (7, 32, 100, 55), (2, 64, 65, 33),
+    # tiles of 128 x 128, contraction blocks that divide the stage (8, 16) or are divided by it (64), that neither
+    (16, 8, 40, 40), (12, 16, 64, 64), (10, 32, 96, 80),
+    # granules of 4, 2 and 1 steps, ragged rows, columns and last stages
+    (22, 3, 36, 20), (16, 9, 50, 70), (14, 13, 55, 41), (20, 7, 25, 60), (18, 30, 26, 38)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_complex_product_edges(hip, nl, B, Fi, Fo, aligned):
+    import s2cnn_amd
+    print(f"complex split product nl={nl} B={B} Fi={Fi} Fo={Fo} aligned={aligned}", flush=True)
+    ns = O.nspec_so3(nl)
+    g = torch.Generator(device="cuda").manual_seed(nl)
+    x, y, gz = (torch.randn(ns, *s, 2, device="cuda", generator=g) for s in ((B, Fi), (Fi, Fo), (B, Fo)))
+    if not aligned:                       # to 8 bytes, the least that the library takes
+        x, y, gz = (torch.empty(t.numel() + 2, device="cuda")[2:].view(t.shape).copy_(t) for t in (x, y, gz))
+    xg, yg = x.detach().requires_grad_(), y.detach().requires_grad_()
+    z = s2cnn_amd.so3_mm(xg, yg)
+    gx, gy = torch.autograd.grad(z, (xg, yg), gz)
+    L = 2 * nl - 1
+    for got, want, K in ((z, product64_complex("fwd", x, y, nl), L * Fi), (gx, product64_complex("gradx", gz, y, nl), L * Fo),
+                         (gy, product64_complex("grady", gz, x, nl), L * B)):
+        assert ((got.double() - want).norm() / want.norm()).item() <= 2 * bound(K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(3, 5, 9, 7), (16, 8, 40, 40)])      # either kernel
+def test_complex_product_of_values_without_bf16_parts(hip, nl, B, Fi, Fo):
+    """Results into which infinities, NaN or values that round to infinity in bf16 go are not finite where a float32 product is
+    not, finite where it is, and the others are what they are without them."""
+    import s2cnn_amd
+    ns = O.nspec_so3(nl)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, y = torch.randn(ns, B, Fi, 2, device="cuda", generator=g), torch.randn(ns, Fi, Fo, 2, device="cuda", generator=g) * 0.0625
+    plain = product64_complex("fwd", x, y, nl)
+    x[ns - 1, 0, 0, 0] = float("inf")
+    x[ns - 7, 1, 1, 1] = float("nan")
+    x[ns - 12, 2, 2, 0] = 3.4e38 * 0.9999   # its first bf16 part is infinite; its products are in range
+    want = product64_complex("fwd", x, y, nl)
+    got = s2cnn_amd.so3_mm(x, y).double()
+    broken = ~torch.isfinite(want).all(-1)
+    assert broken.any() and not torch.isfinite(got[broken]).all(-1).any()
+    assert torch.isfinite(got[~broken]).all()
+    # one huge product beside terms that vanish: three products of its size, rounded, and two sums of them: 2^-24 each, of a size
+    # of up to |a||b| where the result may be a part of that
+    huge = ~broken & (want.abs() > 1e20).any(-1)
+    assert huge.any()
+    size = want[huge].norm(dim=-1, keepdim=True)
+    assert ((got - want)[huge].abs() <= 2.0 ** -21 * size).all()
+    same = ~broken & ~huge
+    assert ((got - plain)[same].norm() / want[same].norm()).item() <= 2 * bound((2 * nl - 1) * Fi)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("nl,B,Fi,Fo", [(3, 5, 9, 7), (16, 8, 40, 40)])      # either kernel
 def test_real_product_of_values_without_bf16_parts(hip, nl, B, Fi, Fo):
