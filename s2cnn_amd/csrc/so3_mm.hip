@@ -52,8 +52,6 @@ template <> struct Cfg<FWD>   { static constexpr bool A_KC = true,  B_KC = false
 template <> struct Cfg<GRADX> { static constexpr bool A_KC = true,  B_KC = true,  A_MNMAJ = true,  B_MNMAJ = false, C_RMAJ = true,  CONJ = false; };
 template <> struct Cfg<GRADY> { static constexpr bool A_KC = false, B_KC = false, A_MNMAJ = false, B_MNMAJ = false, C_RMAJ = false, CONJ = true;  };
 
-__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
-
 __host__ __device__ inline int tile_counts(int L, int RI, int CI, int TMV, int TNV, int& tm, int& tn) {
   tm = s2cnn::ceil_div(L * RI, TMV);
   tn = s2cnn::ceil_div(L * CI, TNV);
@@ -75,9 +73,9 @@ __device__ __forceinline__ int find_degree(const MmParams& p, int TMV, int TNV, 
 template <int KIND> __device__ __forceinline__ float part_of(float2 v) { return KIND == RE ? v.x : KIND == IM ? v.y : v.x + v.y; }
 template <bool CONJ> __device__ __forceinline__ float2 conj_of(float2 v) { return CONJ ? make_float2(v.x, -v.y) : v; }
 
-// A real product of a tile with the float32 matrix instruction, operands straight from memory: for tiles in which it is not
-// finite.  The parts of an infinity, and of a value that rounds to one in bf16, are not its sum (inf - inf); here such
-// values take part as they are, so overflow, infinities and NaN come out as in a float32 product of the same form.
+// A real product of a tile with the float32 matrix instruction, operands straight from memory: for tiles in which the sums of
+// the parts do not hold.  Here infinities, values that round to one in bf16 and tiny values take part as they are, so
+// overflow, infinities and NaN come out as in a float32 product of the same form.
 template <typename C_, int KIND, int NI, int NJ, int STEP>
 __device__ __forceinline__ void contract_float32(const MmParams& p, const float2* A, const float2* B, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h) {
   const int K = L * p.KI;
@@ -254,21 +252,21 @@ __global__ __launch_bounds__(NT, 3) void so3_block_mm_kernel(MmParams p) {
   const bool full = ni == NB && nj == NB;
   const int nstage = s2cnn::ceil_div(L * p.KI, TK);
   const int u = threadIdx.x & (GROUP - 1);
-  const auto finite = [&]() {
+  const auto holds = [&]() {
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) ok = ok && is_finite(acc[i][j][v]);
+        for (int v = 0; v < 16; ++v) ok = ok && s2cnn::sum_holds(acc[i][j][v]);
     return __all(ok);
   };
 #define S2CNN_GROUP(G, LDR)                                                                                                       \
   do {                                                                                                                            \
     if (full) contract<G, true, C_::CONJ>(LDR, s, acc, nstage, row, octet, wrow + r32, wcol + r32, h, ni, nj);                     \
     else contract<G, false, C_::CONJ>(LDR, s, acc, nstage, row, octet, wrow + r32, wcol + r32, h, ni, nj);                         \
-    if (!finite()) contract_float32<C_, G, NB, NB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);            \
+    if (!holds()) contract_float32<C_, G, NB, NB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);            \
   } while (0)
   if (group == 0) {            // K-contiguous: two threads on a row; MN-contiguous: neighbouring threads on neighbouring rows
     const int row = C_::A_KC ? u >> 1 : u & (TM - 1), octet = C_::A_KC ? u & 1 : u / TM;
@@ -397,16 +395,16 @@ __global__ __launch_bounds__(NTS) void so3_block_mm_slices_kernel(MmParams p) {
   for (int v = 0; v < 16; ++v) { part[wave][0][v][lane] = re[v]; part[wave][1][v][lane] = im[v]; }
   __syncthreads();
   float2 sum[4];
-  bool finite = true;
+  bool holds = true;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     float2 z = make_float2(part[0][0][4 * wave + v][lane], part[0][1][4 * wave + v][lane]);
 #pragma unroll
     for (int w = 1; w < NW; ++w) { z.x += part[w][0][4 * wave + v][lane]; z.y += part[w][1][4 * wave + v][lane]; }
     sum[v] = z;
-    finite = finite && is_finite(z.x) && is_finite(z.y);
+    holds = holds && s2cnn::sum_holds(z.x) && s2cnn::sum_holds(z.y);
   }
-  if (!__all(finite)) {
+  if (!__all(holds)) {
     v16f p1[1][1], p2[1][1], p3[1][1];
     contract_float32<C_, RE, 1, 1, 32>(p, A, B, p1, L, tile_m + r32, tile_n + r32, h);
     contract_float32<C_, IM, 1, 1, 32>(p, A, B, p2, L, tile_m + r32, tile_n + r32, h);

@@ -87,17 +87,15 @@ struct TileLoader : Loader<float, KC, MNMAJ, EXT * TK / (NT * 8), KC ? NT / (TK 
   }
 };
 
-__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
-
 __host__ __device__ inline void tile_counts(int L, int RI, int CI, int TM, int TN, int& tm, int& tn, int& slots) {
   tm = s2cnn::ceil_div(L * RI, TM);
   tn = s2cnn::ceil_div(L * CI, TN);
   slots = tm * tn;
 }
 
-// The tile again with the float32 matrix instruction, operands straight from memory: for tiles in which a result is not
-// finite.  The parts of an infinity, and of a value that rounds to one in bf16, are not its sum (inf - inf); here such
-// values take part as they are, so overflow, infinities and NaN come out as in any float32 product.
+// The tile again with the float32 matrix instruction, operands straight from memory: for tiles in which a sum of the parts does
+// not hold.  Here infinities, values that round to one in bf16 and tiny values take part as they are, so overflow,
+// infinities and NaN come out as in any float32 product.
 template <typename C_, int NI, int NJ, int STEP>
 __device__ __forceinline__ void contract_float32(const MmParams& p, const float* A, const float* B, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h) {
   const int K = L * p.KI;
@@ -231,14 +229,14 @@ __global__ __launch_bounds__(NT, 2) void so3_block_mm_real_kernel(MmParams p) {
   else contract<NCB, false>(la, lb, As, Bs, acc, nstage, wrow + r32, wcol + r32, h, ni, nj);
 
   // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32 of its 32x32 block.
-  bool finite = true;
+  bool holds = true;
 #pragma unroll
   for (int i = 0; i < NRB; ++i)
 #pragma unroll
     for (int j = 0; j < NCB; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) finite = finite && is_finite(acc[i][j][v]);
-  if (!__all(finite)) contract_float32<C_, NRB, NCB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);
+      for (int v = 0; v < 16; ++v) holds = holds && s2cnn::sum_holds(acc[i][j][v]);
+  if (!__all(holds)) contract_float32<C_, NRB, NCB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);
 
   float* Cl = p.C + L0 * p.RI * p.CI;
   const int blk_elems = p.RI * p.CI;
@@ -333,7 +331,7 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
     for (int v = 0; v < 16; ++v) part[wave][j][v][lane] = acc[0][j][v];
   __syncthreads();
   float sum[NJ][4];
-  bool finite = true;
+  bool holds = true;
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -342,9 +340,9 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
 #pragma unroll
       for (int w = 1; w < NW; ++w) s += part[w][j][4 * wave + v][lane];
       sum[j][v] = s;
-      finite = finite && is_finite(s);
+      holds = holds && s2cnn::sum_holds(s);
     }
-  if (!__all(finite)) {
+  if (!__all(holds)) {
     contract_float32<C_, 1, NJ, 32>(p, A, B, acc, L, tile_m + r32, tile_n + r32, h);
 #pragma unroll
     for (int j = 0; j < NJ; ++j)

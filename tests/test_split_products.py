@@ -154,3 +154,19 @@ def test_real_product_of_values_without_bf16_parts(hip, nl, B, Fi, Fo):
     assert huge.any() and ((got - want)[huge].abs() <= 2.0 ** -22 * want[huge].abs()).all()
     same = ok & ~huge
     assert ((got - plain * 0.125)[same].norm() / want[same].norm()).item() <= bound((2 * nl - 1) * Fi)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(3, 5, 9, 7), (16, 8, 40, 40)])      # either kernel
+@pytest.mark.parametrize("complex_", [False, True])
+def test_product_of_tiny_values(hip, nl, B, Fi, Fo, complex_):
+    """Operands whose low bf16 parts are subnormal give the accuracy of float32 products: one rounding per step, twice what
+    the sums of 16 steps are allowed."""
+    import s2cnn_amd
+    ns, pair = O.nspec_so3(nl), (2,) if complex_ else ()
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(ns, B, Fi, *pair, device="cuda", generator=g) * 2.0 ** -118
+    y = torch.randn(ns, Fi, Fo, *pair, device="cuda", generator=g)
+    want = (product64_complex if complex_ else product64)("fwd", x, y, nl)
+    got = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(x, y)
+    assert ((got.double() - want).norm() / want.norm()).item() <= 4 * bound((2 * nl - 1) * Fi)
