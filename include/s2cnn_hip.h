@@ -96,7 +96,7 @@ int s2cnn_so3_mm_real_grady(const float *gz, const float *x, float *gy,
  * [len(grid), nspec] matrix (so3_ft.py:8-24).  For the grid points A_i that share beta_i,
  * conj D^l_{mn} = d^l_{mn}(beta_i) exp(-i(m alpha_a + n gamma_a)), hence
  *     y[l,m,n] = sum_i d^l_{mn}(beta_i) G_i[m,n],    G_i[m,n] = sum_{a in A_i} x_a exp(-i(m alpha_a + n gamma_a)):
- * a small GEMM (caller's library) for G, then the pass below, linear in the size of y.  Real x only.
+ * a product with a small matrix for G, then the pass below, linear in the size of y.  Real x only.
  *   G    [nbeta, (2b-1) * b, 2, ncols]   row (m + b-1) * b + n, m in -(b-1)..b-1, n in 0..b-1; (re, im) planes
  *   dtab [nbeta, nspec(b)]               d^l_{mn}(beta_i), degree-major then m then n
  *   y    [nspec(b), ncols]               in the real basis of s2cnn_so3_spectrum_to_real
@@ -108,6 +108,28 @@ int s2cnn_so3_mm_real_grady(const float *gz, const float *x, float *gy,
 int s2cnn_so3_rft_expand_real(const float *G, const float *dtab, float *y, int b, int nbeta, long ncols, void *stream);
 int s2cnn_so3_rft_expand(const float *G, const float *dtab, float *y, int b, int nbeta, long ncols, void *stream);
 int s2cnn_so3_rft_expand_real_grad(const float *gy, const float *dtab, float *gG, int b, int nbeta, long ncols, void *stream);
+/* Both steps from the samples, for any ncols:
+ *   x    [ncols, npts]                   samples, one row per column of y
+ *   idx  [nbeta, P]                      position of group member p in a row of x; -1: no such member (E is zero there)
+ *   E    [nbeta, P, R]                   cos, -sin of m alpha + n gamma, R = (2b-1) * b * 2 in the order of G
+ * rft           : y from scale * x, in the real basis or (complex_out; ncols a multiple of 4) as complex pairs
+ *   Et   [nbeta, R, P]                   the same, for the adjoint
+ * rft_real_grad : gx from gy (real basis), the adjoint; every point must be a member of one group
+ * workspace     : s2cnn_so3_rft_workspace() bytes, 16-byte aligned.
+ */
+size_t s2cnn_so3_rft_workspace(int b, int nbeta, long ncols);
+int s2cnn_so3_rft(const float *x, const int *idx, const float *E, const float *dtab, float *y, void *workspace, size_t workspace_bytes,
+                  int b, int nbeta, int P, int npts, long ncols, float scale, int complex_out, void *stream);
+int s2cnn_so3_rft_real_grad(const float *gy, const int *idx, const float *Et, const float *dtab, float *gx, void *workspace,
+                            size_t workspace_bytes, int b, int nbeta, int P, int npts, long ncols, float scale, void *stream);
+/* The product alone (kernel spectra of the S^2 layers: nbeta = 1, idx = NULL, E [npts, l * m] in the real basis):
+ *   planes      : out[i, r, c] = scale * sum_p E[i, p, r] x[c, idx[i, p]], rows of out ld apart (idx = NULL: p itself)
+ *   planes_grad : gx[c, idx[i, p]] = scale * sum_r Et[i, r, p] g[i, r, c]
+ */
+int s2cnn_rft_planes(const float *x, const int *idx, const float *E, float *out, int nbeta, int P, int R, int npts, long ncols, long ld,
+                     float scale, void *stream);
+int s2cnn_rft_planes_grad(const float *g, const int *idx, const float *Et, float *gx, int nbeta, int P, int R, int npts, long ncols, long ld,
+                          float scale, void *stream);
 
 /* ---- S^2 x S^2 -> SO(3) spectral outer products -------------------------------------
  * x  [nl^2, nbatch, f_in , 2]
@@ -372,6 +394,14 @@ size_t s2cnn_s2_synthesis_workspace(int b_in, int b_out, long nbatch, int comple
 int s2cnn_s2_synthesis(const float *xhat, const float *table, float *out,
                        void *workspace, size_t workspace_bytes,
                        int b_in, int b_out, long nbatch, int complex_out, void *stream);
+/* The analysis of a real signal with its spectrum in the real basis, out [b_out^2, nbatch]: sqrt2 Re (m > 0), Re (m = 0),
+ * sqrt2 Im of the entry -m (m < 0); workspace as for s2cnn_s2_analysis.  grad: its gradient, g [b_out^2, nbatch] -> gx, with the
+ * same table.  Where real_basis_available(b_grid, b_spec) says so.
+ */
+int s2cnn_s2_real_basis_available(int b_grid, int b_spec);
+int s2cnn_s2_analysis_real_basis(const float *x, const float *table, float *out, void *workspace, size_t workspace_bytes,
+                                 int b_in, int b_out, long nbatch, void *stream);
+int s2cnn_s2_analysis_real_basis_grad(const float *g, const float *table, float *gx, int b_in, int b_out, long nbatch, void *stream);
 
 /* ---- Haar integral over SO(3) -------------------------------------------------------
  * x [n, 2b, 2b, 2b], w [2b] -> out [n]:  out[z] = sum_beta w[beta] sum_{alpha,gamma} x[z,...]

@@ -14,7 +14,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "csrc", "libs2cnn_hip.so")
 
 _c_float_p = ctypes.c_void_p
-_int, _long, _size_t, _vp = ctypes.c_int, ctypes.c_long, ctypes.c_size_t, ctypes.c_void_p
+_int, _long, _float, _size_t, _vp = ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_size_t, ctypes.c_void_p
 
 _MM_SIG = [_c_float_p, _c_float_p, _c_float_p, _int, _int, _int, _int, _vp]
 _FT_SIG = [_c_float_p, _c_float_p, _c_float_p, _vp, _size_t, _int, _int, _long, _int, _vp]
@@ -36,6 +36,11 @@ SIGNATURES = {
     "s2cnn_so3_rft_expand_real": (_int, [_c_float_p, _c_float_p, _c_float_p, _int, _int, _long, _vp]),
     "s2cnn_so3_rft_expand": (_int, [_c_float_p, _c_float_p, _c_float_p, _int, _int, _long, _vp]),
     "s2cnn_so3_rft_expand_real_grad": (_int, [_c_float_p, _c_float_p, _c_float_p, _int, _int, _long, _vp]),
+    "s2cnn_so3_rft_workspace": (_size_t, [_int, _int, _long]),
+    "s2cnn_so3_rft": (_int, [_c_float_p, _vp, _c_float_p, _c_float_p, _c_float_p, _vp, _size_t, _int, _int, _int, _int, _long, _float, _int, _vp]),
+    "s2cnn_so3_rft_real_grad": (_int, [_c_float_p, _vp, _c_float_p, _c_float_p, _c_float_p, _vp, _size_t, _int, _int, _int, _int, _long, _float, _vp]),
+    "s2cnn_rft_planes": (_int, [_c_float_p, _vp, _c_float_p, _c_float_p, _int, _int, _int, _int, _long, _long, _float, _vp]),
+    "s2cnn_rft_planes_grad": (_int, [_c_float_p, _vp, _c_float_p, _c_float_p, _int, _int, _int, _int, _long, _long, _float, _vp]),
     "s2cnn_s2_mm_fwd": (_int, _MM_SIG),
     "s2cnn_s2_mm_gradx": (_int, _MM_SIG),
     "s2cnn_s2_mm_grady": (_int, _MM_SIG),
@@ -73,6 +78,9 @@ SIGNATURES = {
     "s2cnn_so3_pack_table": (_int, [_c_float_p, _c_float_p, _int, _int, _int, _vp]),
     "s2cnn_s2_analysis_workspace": (_size_t, _WS_SIG),
     "s2cnn_s2_analysis": (_int, _FT_SIG),
+    "s2cnn_s2_real_basis_available": (_int, [_int, _int]),
+    "s2cnn_s2_analysis_real_basis": (_int, [_c_float_p, _c_float_p, _c_float_p, _vp, _size_t, _int, _int, _long, _vp]),
+    "s2cnn_s2_analysis_real_basis_grad": (_int, [_c_float_p, _c_float_p, _c_float_p, _int, _int, _long, _vp]),
     "s2cnn_s2_synthesis_workspace": (_size_t, _WS_SIG),
     "s2cnn_s2_synthesis": (_int, _FT_SIG),
     "s2cnn_so3_integrate": (_int, [_c_float_p, _c_float_p, _c_float_p, _int, _long, _vp]),

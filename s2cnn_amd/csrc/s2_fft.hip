@@ -145,6 +145,59 @@ extern "C" size_t s2cnn_s2_analysis_workspace(int b_in, int b_out, long nbatch, 
 }
 extern "C" size_t s2cnn_s2_synthesis_workspace(int b_in, int b_out, long nbatch, int) { return ws_bytes(b_out, b_in, nbatch); }
 
+namespace {
+// one kernel, one workgroup per signal; REAL: the spectrum comes out in the real basis
+template <bool REAL>
+int real_analysis(const s2_real::Plan& plan, const float* x, const float* table, float* out, void* workspace, size_t workspace_bytes, int n2, int nb,
+                  long nbatch, hipStream_t st) {
+  // few signals: split along beta, partial spectra in the workspace, added up in a fixed order
+  int nsplit = s2_real::splits_for(n2, plan.rb, nbatch);
+  const size_t nout = (size_t)nb * nb * nbatch;
+  if (nsplit > 1 && nsplit * nout * sizeof(float2) > workspace_bytes)      // a workspace sized for the two-kernel path only:
+    nsplit = (int)(workspace_bytes / (nout * sizeof(float2)));              // as many splits as it holds
+  if (nsplit < 2) nsplit = 1;
+  const auto launch = [&](auto kernel, float* dst) {
+    if (plan.lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nbatch, nsplit), dim3(s2_real::NT), plan.lds, st, x, table, dst, n2, nb, nbatch, plan.rb);
+  };
+  if (nsplit == 1) {
+    launch(s2_real::analysis_kernel<REAL>, out);
+  } else {
+    launch(s2_real::analysis_kernel<false>, static_cast<float*>(workspace));
+    hipLaunchKernelGGL(s2_real::reduce_splits<REAL>, dim3((unsigned)((nout + 255) / 256 < 1024 ? (nout + 255) / 256 : 1024)), dim3(256), 0, st,
+                       static_cast<const float2*>(workspace), out, (long)nout, nsplit, nbatch);
+  }
+  return s2cnn::launch_status();
+}
+
+template <bool REAL>
+int real_synthesis(const s2_real::Plan& plan, const float* xhat, const float* table, float* out, int n2, int nb, long nbatch, hipStream_t st) {
+  if (plan.lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)s2_real::synthesis_kernel<REAL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds);
+  hipLaunchKernelGGL(s2_real::synthesis_kernel<REAL>, dim3((unsigned)nbatch, s2_real::splits_for(n2, 64, nbatch)), dim3(s2_real::NT), plan.lds, st, xhat,
+                     table, out, n2, nb, nbatch);
+  return s2cnn::launch_status();
+}
+}  // namespace
+
+extern "C" int s2cnn_s2_real_basis_available(int b_grid, int b_spec) {
+  return sizes_ok(b_grid, b_spec, 1) && s2_real::plan_fwd(2 * b_grid, b_spec).rb > 0 && s2_real::plan_inv(2 * b_grid, b_spec).rb > 0 ? 1 : 0;
+}
+
+extern "C" int s2cnn_s2_analysis_real_basis(const float* x, const float* table, float* out, void* workspace, size_t workspace_bytes, int b_in, int b_out,
+                                            long nbatch, void* stream) {
+  s2cnn::clear_stale_error();
+  if (!x || !table || !out || !sizes_ok(b_in, b_out, nbatch) || !s2cnn_s2_real_basis_available(b_in, b_out)) return S2CNN_EINVAL;
+  if (!workspace || workspace_bytes < ws_bytes(b_in, b_out, nbatch) || !s2cnn::aligned8(workspace)) return S2CNN_EWORKSPACE;
+  return real_analysis<true>(s2_real::plan_fwd(2 * b_in, b_out), x, table, out, workspace, workspace_bytes, 2 * b_in, b_out, nbatch,
+                             static_cast<hipStream_t>(stream));
+}
+
+extern "C" int s2cnn_s2_analysis_real_basis_grad(const float* g, const float* table, float* gx, int b_in, int b_out, long nbatch, void* stream) {
+  s2cnn::clear_stale_error();
+  if (!g || !table || !gx || !sizes_ok(b_in, b_out, nbatch) || !s2cnn_s2_real_basis_available(b_in, b_out)) return S2CNN_EINVAL;
+  return real_synthesis<true>(s2_real::plan_inv(2 * b_in, b_out), g, table, gx, 2 * b_in, b_out, nbatch, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int s2cnn_s2_analysis(const float* x, const float* table, float* out, void* workspace, size_t workspace_bytes,
                                  int b_in, int b_out, long nbatch, int complex_in, void* stream) {
   s2cnn::clear_stale_error();
@@ -155,22 +208,7 @@ extern "C" int s2cnn_s2_analysis(const float* x, const float* table, float* out,
   const int n2 = 2 * b_in, nb = b_out;
   if (!complex_in) {   // real signals, b_out <= 32: one kernel, one workgroup per signal
     const s2_real::Plan plan = s2_real::plan_fwd(n2, nb);
-    if (plan.rb > 0) {
-      if (plan.lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)s2_real::analysis_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds);
-      // few signals: split along beta, partial spectra in the workspace, added up in a fixed order
-      int nsplit = s2_real::splits_for(n2, plan.rb, nbatch);
-      const size_t nout = (size_t)nb * nb * nbatch;
-      if (nsplit > 1 && nsplit * nout * sizeof(float2) > workspace_bytes)      // a workspace sized for the two-kernel path only:
-        nsplit = (int)(workspace_bytes / (nout * sizeof(float2)));              // as many splits as it holds
-      if (nsplit < 2) nsplit = 1;
-      float2* dst = nsplit > 1 ? static_cast<float2*>(workspace) : reinterpret_cast<float2*>(out);
-      hipLaunchKernelGGL(s2_real::analysis_kernel, dim3((unsigned)nbatch, nsplit), dim3(s2_real::NT), plan.lds, st, x, table,
-                         dst, n2, nb, nbatch, plan.rb);
-      if (nsplit > 1)
-        hipLaunchKernelGGL(s2_real::reduce_splits, dim3((unsigned)((nout + 255) / 256 < 1024 ? (nout + 255) / 256 : 1024)), dim3(256), 0, st,
-                           dst, reinterpret_cast<float2*>(out), (long)nout, nsplit);
-      return s2cnn::launch_status();
-    }
+    if (plan.rb > 0) return real_analysis<false>(plan, x, table, out, workspace, workspace_bytes, n2, nb, nbatch, st);
   }
   float2* X = static_cast<float2*>(workspace);
   const size_t lds = sizeof(float) * (2 * n2 + (complex_in ? 2 : 1) * n2);
@@ -194,12 +232,7 @@ extern "C" int s2cnn_s2_synthesis(const float* xhat, const float* table, float* 
   const int n2 = 2 * b_out, nb = b_in;
   if (!complex_out) {
     const s2_real::Plan plan = s2_real::plan_inv(n2, nb);
-    if (plan.rb > 0) {
-      if (plan.lds > 48 * 1024) (void)hipFuncSetAttribute((const void*)s2_real::synthesis_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)plan.lds);
-      hipLaunchKernelGGL(s2_real::synthesis_kernel, dim3((unsigned)nbatch, s2_real::splits_for(n2, 64, nbatch)), dim3(s2_real::NT), plan.lds, st,
-                         reinterpret_cast<const float2*>(xhat), table, out, n2, nb, nbatch);
-      return s2cnn::launch_status();
-    }
+    if (plan.rb > 0) return real_synthesis<false>(plan, xhat, table, out, n2, nb, nbatch, st);
   }
   const int MW = 2 * nb - 1;
   float2* S = static_cast<float2*>(workspace);

@@ -79,19 +79,33 @@ inline int splits_for(int n2, int RB, long nbatch) {
   return want < 1 ? 1 : (int)want;
 }
 
-// out[e][z] = sum over the splits of partial[s][e][z], in the order of s
-__global__ void reduce_splits(const float2* __restrict__ partial, float2* __restrict__ out, long n, int nsplit) {
+// Entry e = (l, m) of the spectrum of a real signal in the real basis: sqrt2 Re X[l,m] (m > 0), X[l,0], sqrt2 Im X[l,|m|] (m < 0), from
+// v = X[l,m] = (-1)^m conj X[l,-m]
+constexpr float SQRT2 = 1.41421356237309504880f;
+__device__ __forceinline__ float real_basis_entry(float2 v, int m) {
+  return m == 0 ? v.x : m > 0 ? SQRT2 * v.x : ((m & 1) ? SQRT2 : -SQRT2) * v.y;
+}
+
+// out[e][z] = sum over the splits of partial[s][e][z], in the order of s; REAL: in the real basis
+template <bool REAL>
+__global__ void reduce_splits(const float2* __restrict__ partial, float* __restrict__ out, long n, int nsplit, long nbatch) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     float2 v = partial[i];
     for (int s = 1; s < nsplit; ++s) { const float2 p = partial[(size_t)s * n + i]; v.x += p.x; v.y += p.y; }
-    out[i] = v;
+    if constexpr (REAL) {
+      const int e = (int)(i / nbatch), l = isqrt_floor(e);
+      out[i] = real_basis_entry(v, e - l * l - l);
+    } else {
+      reinterpret_cast<float2*>(out)[i] = v;
+    }
   }
 }
 
-// x [nbatch][n2][n2] -> out [nb^2][nbatch] complex;  T [n2][nb^2]
-// grid.y > 1: split blockIdx.y takes its share of the rows and writes out + blockIdx.y * nb^2 * nbatch (partial spectra)
+// x [nbatch][n2][n2] -> out [nb^2][nbatch], complex or (REAL) in the real basis;  T [n2][nb^2]
+// grid.y > 1: split blockIdx.y takes its share of the rows and writes out + blockIdx.y * nb^2 * nbatch (complex partial spectra)
+template <bool REAL>
 __global__ __launch_bounds__(NT) void analysis_kernel(const float* __restrict__ x, const float* __restrict__ T,
-                                                      float2* __restrict__ out, int n2, int nb, long nbatch, int RB) {
+                                                      float* __restrict__ out, int n2, int nb, long nbatch, int RB) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int h = n2 / 2, hg = h + 1, nbp = pad(nb, 2), nspec = nb * nb;
   float2* tab = reinterpret_cast<float2*>(smem);      // [hg][nbp]
@@ -102,7 +116,6 @@ __global__ __launch_bounds__(NT) void analysis_kernel(const float* __restrict__ 
   const float* xs = x + (size_t)z * n2 * n2;
   const int rps = rows_per_split(n2, RB, gridDim.y);
   const int rbeg = blockIdx.y * rps, rend = rbeg + rps < n2 ? rbeg + rps : n2;       // this workgroup's rows
-  out += (size_t)blockIdx.y * nspec * nbatch;
 
   for (int i = t; i < hg * nbp; i += NT) {
     const int j = i / nbp, k = i - j * nbp;
@@ -193,11 +206,17 @@ __global__ __launch_bounds__(NT) void analysis_kernel(const float* __restrict__ 
   }
 #pragma unroll
   for (int q = 0; q < 2; ++q)
-    if (eok[q]) out[(size_t)(t + q * NT) * nbatch + z] = acc[q];
+    if (eok[q]) {
+      const size_t o = (size_t)(t + q * NT) * nbatch + z;
+      if constexpr (REAL) out[o] = real_basis_entry(acc[q], em[q]);
+      else reinterpret_cast<float2*>(out)[(size_t)blockIdx.y * nspec * nbatch + o] = acc[q];
+    }
 }
 
-// xhat [nb^2][nbatch] complex -> y [nbatch][n2][n2];  T [n2][nb^2]; grid.y splits the rows
-__global__ __launch_bounds__(NT) void synthesis_kernel(const float2* __restrict__ xhat, const float* __restrict__ T,
+// xhat [nb^2][nbatch] complex -> y [nbatch][n2][n2];  T [n2][nb^2]; grid.y splits the rows.  REAL: xhat is the gradient with respect to
+// a spectrum in the real basis; what goes through the synthesis is its adjoint, sqrt2 (g[l,m] + i g[l,-m]) at m > 0 and 0 at m < 0
+template <bool REAL>
+__global__ __launch_bounds__(NT) void synthesis_kernel(const float* __restrict__ xhat, const float* __restrict__ T,
                                                        float* __restrict__ y, int n2, int nb, long nbatch) {
   extern __shared__ __attribute__((aligned(16))) float smem[];
   constexpr int RB = 64;
@@ -213,7 +232,15 @@ __global__ __launch_bounds__(NT) void synthesis_kernel(const float2* __restrict_
     const int k = i / hp, j = i - k * hp;
     tab[i] = j <= h ? dft_common::cs_entry(j, k, n2) : make_float2(0.f, 0.f);
   }
-  for (int e = t; e < nspec; e += NT) xh[e] = xhat[(size_t)e * nbatch + z];
+  for (int e = t; e < nspec; e += NT) {
+    if constexpr (REAL) {
+      const int l = isqrt_floor(e), m = e - l * l - l;
+      xh[e] = m < 0 ? make_float2(0.f, 0.f) : m == 0 ? make_float2(xhat[(size_t)e * nbatch + z], 0.f)
+                    : make_float2(SQRT2 * xhat[(size_t)e * nbatch + z], SQRT2 * xhat[(size_t)(e - 2 * m) * nbatch + z]);
+    } else {
+      xh[e] = reinterpret_cast<const float2*>(xhat)[(size_t)e * nbatch + z];
+    }
+  }
   __syncthreads();
   const int rps = rows_per_split(n2, RB, gridDim.y);
   const int rbeg = blockIdx.y * rps, rend = rbeg + rps < n2 ? rbeg + rps : n2;

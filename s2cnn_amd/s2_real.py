@@ -68,6 +68,58 @@ def s2_rft_real(x, b, grid):
     return out.view(-1, *sz[:-1])
 
 
+@lru_cache(maxsize=32)
+def _setup_s2_rft_plan(b, grid, device):
+    """The matrix of `_setup_s2_ft_real` and its transpose, for the product and its adjoint."""
+    F = _setup_s2_ft_real(b, grid, device)
+    return F, F.t().contiguous()
+
+
+class _KernelSpectrum(torch.autograd.Function):
+    """x [ncols, n_grid] -> [l * m, ncols], the product of scale * x with F [n_grid, l * m] and, as its gradient, the adjoint."""
+    @staticmethod
+    def forward(ctx, x, plan, scale):
+        F = plan[0]
+        _hip.require_gpu_f32(x)
+        x = x.contiguous()
+        ncols, npts = x.shape
+        ctx.plan, ctx.scale = plan, scale
+        y = x.new_empty((F.size(1), ncols))
+        _hip.call("s2cnn_rft_planes", _hip.ptr(x), None, _hip.ptr(F), _hip.ptr(y), 1, npts, F.size(1), npts, ncols, ncols, scale, _hip.stream_ptr())
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        return _KernelSpectrumAdjoint.apply(gy, ctx.plan, ctx.scale), None, None
+
+
+class _KernelSpectrumAdjoint(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, gy, plan, scale):
+        F, Ft = plan
+        _hip.require_gpu_f32(gy)
+        gy = gy.contiguous()
+        npts, ncols = F.size(0), gy.size(1)
+        ctx.plan, ctx.scale = plan, scale
+        gx = gy.new_empty((ncols, npts))
+        _hip.call("s2cnn_rft_planes_grad", _hip.ptr(gy), None, _hip.ptr(Ft), _hip.ptr(gx), 1, npts, F.size(1), npts, ncols, ncols, scale, _hip.stream_ptr())
+        return gx
+
+    @staticmethod
+    def backward(ctx, ggx):
+        return _KernelSpectrum.apply(ggx, ctx.plan, ctx.scale), None, None
+
+
+def scaled_kernel_spectrum(kernel, scale, b, grid):
+    """s2_rft_real(kernel * scale, b, grid) with the factor inside the transform: the kernel spectrum of the layer."""
+    if not (kernel.is_cuda and kernel.dtype == torch.float32 and kernel.numel() > 0) or torch.is_autocast_enabled():
+        return s2_rft_real(kernel * scale, b, grid)
+    plan = _setup_s2_rft_plan(b, grid if isinstance(grid, tuple) else tuple(grid), kernel.device)
+    assert kernel.size(-1) == plan[0].size(0)
+    sz = kernel.size()
+    return _KernelSpectrum.apply(kernel.reshape(-1, sz[-1]), plan, scale).view(-1, *sz[:-1])
+
+
 class _S2_mm_real(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, y):

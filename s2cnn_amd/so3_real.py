@@ -120,55 +120,61 @@ def _setup_so3_ft_real(b, grid, device):
 @lru_cache(maxsize=32)
 def _setup_so3_rft_plan(b, grid, device):
     """Factorised form of the matrix of `_setup_so3_ft_real` for grids with few distinct beta values
-    (wigner.so3_rft_plan); None where it does not apply."""
+    (wigner.so3_rft_plan): (idx, E, its transpose per beta, dtab) on the device; None where it does not apply."""
     plan = wigner.so3_rft_plan(b, grid)
     if plan is None:
         return None
     idx, E, dtab = plan
-    valid = torch.tensor(idx >= 0, device=device)
-    sel = np.flatnonzero(idx.reshape(-1) >= 0)       # positions of the grid points in the padded [nbeta * P] layout
-    return (torch.tensor(np.maximum(idx, 0), dtype=torch.long, device=device), valid,
+    return (torch.tensor(idx.astype(np.int32), device=device).contiguous(),
             torch.tensor(E.astype(np.float32), device=device).contiguous(),
-            torch.tensor(dtab.astype(np.float32), device=device).contiguous(),
-            torch.tensor(sel, dtype=torch.long, device=device),
-            torch.tensor(idx.reshape(-1)[sel], dtype=torch.long, device=device))
+            torch.tensor(E.astype(np.float32), device=device).transpose(1, 2).contiguous(),
+            torch.tensor(dtab.astype(np.float32), device=device).contiguous())
 
 
-class _SO3RftRealFactorised(torch.autograd.Function):
-    """x [ncols, n_grid] -> y [nspec, ncols]: plane coefficients per beta group by a batched GEMM, then the
-    expansion over the degrees (s2cnn_so3_rft_expand_real) and its adjoint."""
+class _KernelSpectrum(torch.autograd.Function):
+    """x [ncols, n_grid] -> y [nspec, ncols] (complex_out: [nspec, ncols, 2]), the spectrum of scale * x: plane coefficients
+    per beta group, then the expansion over the degrees.  Linear: its gradient is the adjoint, and the adjoint's is it."""
     @staticmethod
-    def forward(ctx, x2, b, plan, complex_out=False):
-        idx, valid, E, dtab = plan[:4]
-        _hip.require_gpu_f32(x2)
-        ncols = x2.size(0)
-        with torch.autocast(device_type="cuda", enabled=False):  # the expansion kernel reads G as float32
-            xg = x2.t()[idx] * valid.unsqueeze(-1)                # [nbeta, P, ncols]
-            G = torch.bmm(E.transpose(1, 2), xg).contiguous()    # [nbeta, R, ncols]
-        _hip.require_gpu_f32(G)
+    def forward(ctx, x, b, plan, scale, complex_out=False):
+        idx, E, _, dtab = plan
+        _hip.require_gpu_f32(x)
+        x = x.contiguous()
+        ncols, npts = x.shape
+        ctx.args = b, plan, scale, complex_out, npts
+        nbeta, npoint = idx.shape
         nspec = b * (4 * b * b - 1) // 3
-        y = x2.new_empty((nspec, ncols, 2) if complex_out else (nspec, ncols))
-        _hip.call("s2cnn_so3_rft_expand" if complex_out else "s2cnn_so3_rft_expand_real",
-                  _hip.ptr(G), _hip.ptr(dtab), _hip.ptr(y), b, idx.size(0), ncols, _hip.stream_ptr())
-        ctx.plan, ctx.b, ctx.n_grid, ctx.complex_out = plan, b, x2.size(1), complex_out
+        y = x.new_empty((nspec, ncols, 2) if complex_out else (nspec, ncols))
+        ws = _hip.workspace(_hip.lib().s2cnn_so3_rft_workspace(b, nbeta, ncols), x.device)
+        _hip.call("s2cnn_so3_rft", _hip.ptr(x), _hip.ptr(idx), _hip.ptr(E), _hip.ptr(dtab), _hip.ptr(y), _hip.ptr(ws), ws.numel(), b, nbeta,
+                  npoint, npts, ncols, scale, int(complex_out), _hip.stream_ptr())
         return y
 
     @staticmethod
     def backward(ctx, gy):
-        idx, valid, E, dtab, sel, idx_sel = ctx.plan
-        gy = gy.contiguous()
-        if ctx.complex_out:      # the adjoint of the change of basis, then the adjoint of the real-basis expansion
-            _hip.require_gpu_f32(gy)
-            gy = _convert("s2cnn_so3_spectrum_to_real", gy, gy.shape[:-1])
+        return _KernelSpectrumAdjoint.apply(gy, *ctx.args), None, None, None, None
+
+
+class _KernelSpectrumAdjoint(torch.autograd.Function):
+    """gy [nspec, ncols] (complex_out: [nspec, ncols, 2]) -> gx [ncols, npts]."""
+    @staticmethod
+    def forward(ctx, gy, b, plan, scale, complex_out, npts):
+        idx, _, Et, dtab = plan
+        ctx.args = b, plan, scale, complex_out
         _hip.require_gpu_f32(gy)
+        gy = gy.contiguous()
+        if complex_out:      # the adjoint of the change of basis, then the adjoint of the real-basis expansion
+            gy = _convert("s2cnn_so3_spectrum_to_real", gy, gy.shape[:-1])
         ncols = gy.size(1)
-        gG = gy.new_empty((idx.size(0), E.size(2), ncols))
-        _hip.call("s2cnn_so3_rft_expand_real_grad", _hip.ptr(gy), _hip.ptr(dtab), _hip.ptr(gG), ctx.b, idx.size(0), ncols, _hip.stream_ptr())
-        with torch.autocast(device_type="cuda", enabled=False):
-            gxg = torch.bmm(E, gG)                                # [nbeta, P, ncols]
-        gx = gy.new_zeros((ctx.n_grid, ncols))
-        gx.index_add_(0, idx_sel, gxg.reshape(-1, ncols).index_select(0, sel))   # no boolean masks: they would sync with the host
-        return gx.t(), None, None, None
+        nbeta, npoint = idx.shape
+        gx = gy.new_empty((ncols, npts))
+        ws = _hip.workspace(_hip.lib().s2cnn_so3_rft_workspace(b, nbeta, ncols), gy.device)
+        _hip.call("s2cnn_so3_rft_real_grad", _hip.ptr(gy), _hip.ptr(idx), _hip.ptr(Et), _hip.ptr(dtab), _hip.ptr(gx), _hip.ptr(ws), ws.numel(), b,
+                  nbeta, npoint, npts, ncols, scale, _hip.stream_ptr())
+        return gx
+
+    @staticmethod
+    def backward(ctx, ggx):
+        return _KernelSpectrum.apply(ggx, *ctx.args), None, None, None, None, None
 
 
 def so3_rft_complex(x, b, grid):
@@ -186,8 +192,20 @@ def so3_rft_complex(x, b, grid):
     if plan is None:
         return None
     assert sz[-1] == len(grid)
-    out = _SO3RftRealFactorised.apply(x.reshape(-1, sz[-1]), b, plan, True)
+    out = _KernelSpectrum.apply(x.reshape(-1, sz[-1]), b, plan, 1.0, True)
     return out.view(-1, *sz[:-1], 2)
+
+
+def scaled_kernel_spectrum(kernel, scale, b, grid):
+    """so3_rft_real(kernel * scale, b, grid) with the factor inside the transform: the kernel spectrum of the layer."""
+    sz = kernel.size()
+    plan = None
+    if kernel.is_cuda and kernel.dtype == torch.float32 and kernel.numel() > 0 and so3_rft_real.factorised:
+        plan = _setup_so3_rft_plan(b, grid if isinstance(grid, tuple) else tuple(grid), kernel.device)
+    if plan is None:
+        return so3_rft_real(kernel * scale, b, grid)
+    assert sz[-1] == len(grid)
+    return _KernelSpectrum.apply(kernel.reshape(-1, sz[-1]), b, plan, scale).view(-1, *sz[:-1])
 
 
 def so3_rft_real(x, b, grid):
@@ -202,7 +220,7 @@ def so3_rft_real(x, b, grid):
     plan = _setup_so3_rft_plan(b, tuple(grid), x.device) if fast else None
     if plan is not None:
         assert sz[-1] == len(grid)
-        out = _SO3RftRealFactorised.apply(x.reshape(-1, sz[-1]), b, plan)
+        out = _KernelSpectrum.apply(x.reshape(-1, sz[-1]), b, plan, 1.0)
         return out.view(-1, *sz[:-1])
     F = _setup_so3_ft_real(b, grid, x.device)  # [beta_alpha_gamma, l * m * n]
     assert x.size(-1) == F.size(0)

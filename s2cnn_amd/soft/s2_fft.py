@@ -127,6 +127,44 @@ class S2_fft_real(torch.autograd.Function):
         return s2_rifft(grad_output, for_grad=True, b_out=ctx.b_in), None
 
 
+class _S2FftRealBasis(torch.autograd.Function):
+    """S2_fft_real with the spectrum in the real basis of s2cnn_amd.s2_real, [l * m, ...]; used by S2Convolution."""
+    @staticmethod
+    def forward(ctx, x, b_out):  # pylint: disable=W
+        b_in, b_out, batch_size = _grid_args(x, b_out, False)
+        ctx.args = b_in, b_out, batch_size
+        _hip.require_gpu_f32(x)
+        x = x.contiguous()
+        nbatch = _count(batch_size)
+        out = x.new_empty((b_out ** 2, *batch_size))
+        if nbatch == 0:
+            return out
+        ws = _hip.workspace(_hip.lib().s2cnn_s2_analysis_workspace(b_in, b_out, nbatch, 0), x.device)
+        _hip.call("s2cnn_s2_analysis_real_basis", _hip.ptr(x), _hip.ptr(_setup_wigner(b_in, nl=b_out, weighted=True, device=x.device)), _hip.ptr(out),
+                  _hip.ptr(ws), ws.numel(), b_in, b_out, nbatch, _hip.stream_ptr())
+        return out
+
+    @staticmethod
+    def backward(ctx, g):  # pylint: disable=W
+        b_in, b_out, batch_size = ctx.args
+        _hip.require_gpu_f32(g)
+        g = g.contiguous()
+        nbatch = _count(batch_size)
+        gx = g.new_empty((*batch_size, 2 * b_in, 2 * b_in))
+        if nbatch > 0:
+            _hip.call("s2cnn_s2_analysis_real_basis_grad", _hip.ptr(g), _hip.ptr(_setup_wigner(b_in, nl=b_out, weighted=True, device=g.device)),
+                      _hip.ptr(gx), b_in, b_out, nbatch, _hip.stream_ptr())
+        return gx, None
+
+
+def s2_rfft_real_basis(x, b_out):
+    """s2_spectrum_to_real(S2_fft_real.apply(x, b_out)): one kernel where the library has it."""
+    if x.is_cuda and _hip.lib().s2cnn_s2_real_basis_available(x.size(-1) // 2, b_out):
+        return _S2FftRealBasis.apply(x, b_out)
+    from ..s2_real import s2_spectrum_to_real
+    return s2_spectrum_to_real(S2_fft_real.apply(x, b_out))
+
+
 class S2_ifft_real(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, b_out=None):  # pylint: disable=W

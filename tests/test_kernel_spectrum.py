@@ -1,0 +1,106 @@
+"""Kernel spectra of the layers (s2cnn_rft_planes, s2cnn_so3_rft and their adjoints) and the S^2 analysis that writes the real
+basis, against float64 products with the matrices of the transforms."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# Errors: products of K terms with six roundings of 2^-24 per 16 of them (about 2^-24 sqrt(K / 16) of the result), one rounding each
+# of the matrix, the d-values and the factor, three of the sums over betas and the change of basis; all in relative 2-norm.
+def bound(K):
+    return 2.0 ** -24 * (6 + (K / 4) ** 0.5)
+
+
+def rel(got, want):
+    return ((got.double().cpu() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("b,shape", [
+    (1, (1, 1)), (2, (1, 3)), (6, (20, 40)), (7, (3, 11)), (13, (33, 45)),          # split contraction, columns 1, 3, 800, 33, 1485
+    (20, (32, 64)), (11, (5, 205))])                                             # a block per wave, whole and ragged columns
+@pytest.mark.parametrize("kind", ["near", "equatorial", "point"])
+def test_so3_kernel_spectrum(hip, b, shape, kind):
+    import s2cnn_amd
+    from s2cnn_amd import wigner
+    from s2cnn_amd.so3_real import scaled_kernel_spectrum
+    grid = {"near": s2cnn_amd.so3_near_identity_grid(), "equatorial": s2cnn_amd.so3_equatorial_grid(n_alpha=2 * b, n_beta=2, n_gamma=3),
+            "point": ((0, 0, 0),)}[kind]
+    print(f"kernel spectrum b={b} shape={shape} grid={kind}", flush=True)
+    g = torch.Generator().manual_seed(b)
+    k = torch.randn(*shape, len(grid), generator=g)
+    F = torch.from_numpy(wigner.so3_ft_matrix_real(b, grid)) * 0.37
+    kg = k.cuda().requires_grad_()
+    y = scaled_kernel_spectrum(kg, 0.37, b, grid)
+    gy = torch.randn(y.shape, generator=g)
+    (gk,) = torch.autograd.grad(y, kg, gy.cuda())
+    flat = k.double().reshape(-1, len(grid))
+    assert rel(y.detach().reshape(F.size(1), -1), F.t() @ flat.t()) <= bound(len(grid))
+    want = (gy.double().reshape(F.size(1), -1).t() @ F.t()).reshape(k.shape)
+    # the sums over the spectrum cancel: the error is relative to |gy| |F|, as for any order of the sum
+    size = ((gy.double().reshape(F.size(1), -1).t() ** 2) @ (F.t() ** 2)).sum().sqrt()
+    assert ((gk.double().cpu() - want).norm() / size).item() <= bound(F.size(1))
+
+
+@pytest.mark.parametrize("b,shape", [(1, (1, 1)), (10, (1, 20)), (20, (3, 26)), (32, (6, 100)), (7, (64, 320))])
+def test_s2_kernel_spectrum(hip, b, shape):
+    import s2cnn_amd
+    from s2cnn_amd.s2_real import _setup_s2_ft_real, scaled_kernel_spectrum
+    for grid in (s2cnn_amd.s2_near_identity_grid(), s2cnn_amd.s2_equatorial_grid(max_beta=0, n_alpha=130, n_beta=1)):
+        g = torch.Generator().manual_seed(b)
+        k = torch.randn(*shape, len(grid), generator=g)
+        F = _setup_s2_ft_real(b, grid, torch.device("cpu")).double() * 0.37
+        kg = k.cuda().requires_grad_()
+        y = scaled_kernel_spectrum(kg, 0.37, b, grid)
+        gy = torch.randn(y.shape, generator=g)
+        (gk,) = torch.autograd.grad(y, kg, gy.cuda())
+        assert rel(y.detach().reshape(F.size(1), -1), F.t() @ k.double().reshape(-1, len(grid)).t()) <= bound(len(grid))
+        want = (gy.double().reshape(F.size(1), -1).t() @ F.t()).reshape(k.shape)
+        size = ((gy.double().reshape(F.size(1), -1).t() ** 2) @ (F.t() ** 2)).sum().sqrt()
+        assert ((gk.double().cpu() - want).norm() / size).item() <= bound(F.size(1))
+
+
+def test_kernel_spectrum_of_values_without_bf16_parts(hip):
+    """A column with an infinity or NaN is not finite; one with a value that rounds to infinity in bf16 and the others are."""
+    import s2cnn_amd
+    from s2cnn_amd import wigner
+    from s2cnn_amd.so3_real import scaled_kernel_spectrum
+    b, grid = 6, s2cnn_amd.so3_near_identity_grid()
+    k = torch.randn(5, 9, len(grid), generator=torch.Generator().manual_seed(0))
+    k[0, 0, 7], k[1, 1, 3], k[2, 2, 100] = float("inf"), float("nan"), 3.4e38 * 0.9999
+    y = scaled_kernel_spectrum(k.cuda(), 0.0625, b, grid).cpu().reshape(-1, 45)
+    finite = torch.isfinite(y).all(0)
+    assert finite.sum() == 43 and not finite[0] and not finite[10]
+    want = torch.from_numpy(wigner.so3_ft_matrix_real(b, grid)).t() @ k.double().reshape(45, -1)[finite].t() * 0.0625
+    err = (y[:, finite].double() - want).norm(dim=0) / want.norm(dim=0)
+    assert err.max().item() <= 4 * bound(len(grid))          # per column, with a quarter of the chip's columns as room
+
+
+def test_kernel_spectrum_gradient_of_the_gradient(hip):
+    """The transform is linear: the gradient of a function of its gradient is the transform again."""
+    import s2cnn_amd
+    from s2cnn_amd import s2_real, so3_real
+    for mod, grid in ((so3_real, s2cnn_amd.so3_near_identity_grid()), (s2_real, s2cnn_amd.s2_near_identity_grid())):
+        k = torch.randn(3, 5, len(grid), device="cuda", requires_grad=True)
+        y = mod.scaled_kernel_spectrum(k, 0.5, 5, grid)
+        gy = torch.randn_like(y).requires_grad_()
+        (gk,) = torch.autograd.grad(y, k, gy, create_graph=True)
+        v = torch.randn_like(gk)
+        (ggy,) = torch.autograd.grad(gk, gy, v)
+        assert torch.equal(ggy, mod.scaled_kernel_spectrum(v, 0.5, 5, grid))
+
+
+@pytest.mark.parametrize("b_in,b_out,batch", [(1, 1, 1), (3, 2, 5), (30, 10, 1), (30, 10, 33), (50, 20, 27), (64, 32, 7), (128, 32, 3)])
+def test_s2_analysis_in_the_real_basis(hip, b_in, b_out, batch):
+    """The map of the complex spectrum and, as its gradient, that of the composition: the same sums in the same order, one more
+    rounding of the factor."""
+    from s2cnn_amd.s2_real import s2_spectrum_to_real
+    from s2cnn_amd.soft.s2_fft import S2_fft_real, s2_rfft_real_basis
+    x = torch.randn(batch, 1, 2 * b_in, 2 * b_in, device="cuda", requires_grad=True)
+    want, got = s2_spectrum_to_real(S2_fft_real.apply(x, b_out)), s2_rfft_real_basis(x, b_out)
+    assert got.shape == want.shape
+    assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -22
+    g = torch.randn_like(want)
+    gw, gg = (torch.autograd.grad(y, x, g)[0] for y in (want, got))
+    assert ((gg - gw).norm() / gw.norm()).item() <= 2.0 ** -22
