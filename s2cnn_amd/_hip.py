@@ -168,17 +168,19 @@ def require_gpu_f32(*tensors):
             raise RuntimeError(
                 "s2cnn_amd runs float32 tensors on the GPU only (got %s on %s); there is no CPU path"
                 % (t.dtype, t.device))
-        if t.device.index != torch.cuda.current_device():
+        if t.device.index != torch._C._cuda_getDevice():
             raise RuntimeError("operand on %s but the current device is cuda:%d: call inside torch.cuda.device(%d)"
                                % (t.device, torch.cuda.current_device(), t.device.index))
 
 
 def stream_ptr():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current device's current stream (its handle alone: building a torch.cuda.Stream takes longer than a launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    """Address of a tensor's data, for the void * arguments of the library (ctypes takes the number as it is)."""
+    return t.data_ptr()
 
 
 def workspace(nbytes, device):
