@@ -19,7 +19,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from .soft.bn_relu import run_sequence
+from .soft.bn_relu import evaluate_sequence, run_sequence
 from . import (S2Convolution, SO3Convolution, s2_equatorial_grid, s2_near_identity_grid, so3_equatorial_grid, so3_integrate,
                so3_near_identity_grid)
 
@@ -82,7 +82,7 @@ class Shrec17Model(nn.Module):
         if self.fused_norm:
             x = run_sequence(self.sequential, x, head="integrate")    # [batch, feature]
         else:
-            x = so3_integrate(self.sequential(x))                     # [batch, feature, beta, alpha, gamma] -> [batch, feature]
+            x = so3_integrate(evaluate_sequence(self.sequential, x))  # [batch, feature, beta, alpha, gamma] -> [batch, feature]
         return F.log_softmax(self.out_layer(x), dim=1)
 
 
@@ -101,7 +101,7 @@ class Shrec17ModelOriginal(nn.Module):
         if self.fused_norm:
             x = run_sequence(self.sequential, x, head="max")          # [batch, feature]
         else:
-            x = self.sequential(x)
+            x = evaluate_sequence(self.sequential, x)
             x = x.view(x.size(0), x.size(1), -1).max(-1)[0]
         return F.log_softmax(self.out_layer(x), dim=1)
 

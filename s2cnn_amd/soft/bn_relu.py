@@ -16,8 +16,10 @@ parameters and buffers (running statistics, num_batches_tracked) stay those of t
 """
 import torch
 from torch import nn
+from torch.nn.modules import module as _nn_module
 
 from .. import _hip
+from .s2_conv import S2Convolution
 from .so3_conv import SO3Convolution
 from .so3_integrate import _setup_so3_integrate, so3_integrate
 from .so3_fft import (LoadAffineReLU, LoadBNReLUGrad, analysis_prologue_available, so3_rfft_real_basis,
@@ -229,3 +231,45 @@ def run_sequence(sequence, x, head=None):
     for m in mods[i:]:
         y = m(y)
     return finish(y)
+
+
+def _hooked(*mods):
+    """Whether a call of one of the modules does more than its forward."""
+    return (any(m._forward_hooks or m._forward_pre_hooks for m in mods)
+            or bool(_nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks))
+
+
+def _folds(conv, bn, act):
+    """A layer whose output a normalisation with fixed statistics and a ReLU follow, each module exactly what it says."""
+    return (type(conv) in (S2Convolution, SO3Convolution) and type(bn) is nn.BatchNorm3d and type(act) is nn.ReLU and conv.real_basis
+            and conv.activation is None and conv.nfeature_out == bn.num_features and not bn.training and bn.running_mean is not None
+            and bn.running_var is not None and not _hooked(conv, bn, act)
+            and all(t is None or (t.is_cuda and t.dtype == torch.float32)
+                    for t in (conv.kernel, conv.bias, bn.weight, bn.bias, bn.running_mean, bn.running_var)))
+
+
+def evaluate_sequence(sequence, x):
+    """`sequence(x)`, where no gradient is asked for with every BatchNorm3d in evaluation mode and ReLU that follow a spectral layer
+    folded into that layer: a (layer(x)) + b is the layer with its kernel times a and its bias times a plus b, and the ReLU is
+    applied where the last transform writes.  Same function; the two passes of the modules over the activations fall away."""
+    if (torch.is_grad_enabled() or torch.is_autocast_enabled() or type(sequence) is not nn.Sequential or _hooked(sequence)
+            or not x.is_cuda or x.dtype != torch.float32 or x.size(0) == 0):
+        return sequence(x)
+    mods = list(sequence)
+    i = 0
+    while i < len(mods):
+        if i + 2 < len(mods) and _folds(*mods[i:i + 3]):
+            conv, bn = mods[i], mods[i + 1]
+            a = torch.rsqrt(bn.running_var + bn.eps)
+            if bn.weight is not None:
+                a = a * bn.weight
+            shift = (conv.bias.reshape(-1) - bn.running_mean) * a
+            if bn.bias is not None:
+                shift = shift + bn.bias
+            zr = conv.product_spectrum(x, kernel=conv.kernel * a.view(1, -1, 1))
+            x = so3_rifft_real_basis(zr, bias=shift, relu=True)
+            i += 3
+        else:
+            x = mods[i](x)
+            i += 1
+    return x

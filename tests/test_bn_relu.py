@@ -281,3 +281,41 @@ def test_shape_network_with_fused_normalisation(hip):
     _, lb, _ = harness.train_steps("shrec17", batch=4, steps=4, warmup=0, lr=0.02, model=fused)
     print("plain", ["%.5f" % l for l in la], "fused", ["%.5f" % l for l in lb], flush=True)
     assert max(abs(a - b) for a, b in zip(la, lb)) < 2e-4 * abs(la[0])
+
+
+@pytest.mark.parametrize("affine", [True, False])
+@pytest.mark.parametrize("b_mid", [16, 7, 32])
+def test_normalisation_with_fixed_statistics_folded_into_the_layer(hip, affine, b_mid):
+    """evaluate_sequence against the modules one after the other, in evaluation mode without gradients: factors of both signs and
+    statistics away from 0 and 1; calls with a gradient, in training mode or with a hook run the modules.  The factor sits on the
+    kernel instead of the result: a rounding more per term of sums that take a few already."""
+    import s2cnn_amd
+    from torch import nn
+    torch.manual_seed(b_mid)
+    seq = nn.Sequential(s2cnn_amd.S2Convolution(2, 5, 34, b_mid, s2cnn_amd.s2_near_identity_grid()), nn.BatchNorm3d(5, affine=affine), nn.ReLU(),
+                        s2cnn_amd.SO3Convolution(5, 7, b_mid, 6, s2cnn_amd.so3_near_identity_grid()), nn.BatchNorm3d(7, affine=affine), nn.ReLU()).cuda().eval()
+    for bn in (seq[1], seq[4]):
+        bn.running_mean.normal_(0.3, 0.5)
+        bn.running_var.uniform_(0.2, 2.0)
+        if affine:
+            with torch.no_grad():
+                bn.weight.normal_()
+                bn.bias.normal_()
+    with torch.no_grad():
+        seq[0].bias.normal_()
+    x = torch.randn(3, 2, 68, 68, device="cuda")
+    with torch.no_grad():
+        want, got = seq(x), bn_relu.evaluate_sequence(seq, x)
+        assert not torch.equal(want, got) and _rel(got.double(), want.double()) < 2e-6
+        seen = []
+        handle = seq[1].register_forward_hook(lambda *a: seen.append(1))
+        hooked = bn_relu.evaluate_sequence(seq, x)
+        handle.remove()
+        assert seen and _rel(hooked.double(), want.double()) < 2e-6
+    xg = x.clone().requires_grad_()
+    assert torch.equal(bn_relu.evaluate_sequence(seq, xg), seq(xg))
+    seq.train()
+    with torch.no_grad():
+        n = int(seq[1].num_batches_tracked)
+        bn_relu.evaluate_sequence(seq, x)
+        assert int(seq[1].num_batches_tracked) == n + 1
