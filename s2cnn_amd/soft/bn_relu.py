@@ -16,6 +16,7 @@ parameters and buffers (running statistics, num_batches_tracked) stay those of t
 """
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 from torch.nn.modules import module as _nn_module
 
 from .. import _hip
@@ -251,8 +252,10 @@ def _folds(conv, bn, act):
 def evaluate_sequence(sequence, x):
     """`sequence(x)`, where no gradient is asked for with every BatchNorm3d in evaluation mode and ReLU that follow a spectral layer
     folded into that layer: a (layer(x)) + b is the layer with its kernel times a and its bias times a plus b, and the ReLU is
-    applied where the last transform writes.  Same function; the two passes of the modules over the activations fall away."""
-    if (torch.is_grad_enabled() or torch.is_autocast_enabled() or type(sequence) is not nn.Sequential or _hooked(sequence)
+    applied where the last transform writes.  Same function; the two passes of the modules over the activations fall away.
+    Tangents and batched parameters of a normalisation (forward mode, torch.func) pass the modules, not a layer's own functions."""
+    if (torch.is_grad_enabled() or torch.is_autocast_enabled() or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or type(sequence) is not nn.Sequential or _hooked(sequence)
             or not x.is_cuda or x.dtype != torch.float32 or x.size(0) == 0):
         return sequence(x)
     mods = list(sequence)

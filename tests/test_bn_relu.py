@@ -319,3 +319,19 @@ def test_normalisation_with_fixed_statistics_folded_into_the_layer(hip, affine, 
         n = int(seq[1].num_batches_tracked)
         bn_relu.evaluate_sequence(seq, x)
         assert int(seq[1].num_batches_tracked) == n + 1
+
+
+def test_tangents_of_a_normalisation_pass_the_modules(hip):
+    """Forward mode is on under no_grad as well: a tangent of the normalisation's shift has the modules run, the folded layer has none."""
+    import s2cnn_amd
+    from torch import nn
+    from torch.autograd import forward_ad
+    torch.manual_seed(0)
+    seq = nn.Sequential(s2cnn_amd.S2Convolution(2, 3, 8, 5, s2cnn_amd.s2_near_identity_grid()), nn.BatchNorm3d(3), nn.ReLU()).cuda().eval()
+    x = torch.randn(2, 2, 16, 16, device="cuda")
+    with torch.no_grad(), forward_ad.dual_level(), torch.backends.cudnn.flags(enabled=False):    # MIOpen's has no forward mode
+        shift = seq[1].bias.detach().clone()
+        del seq[1].bias
+        seq[1].bias = forward_ad.make_dual(shift, torch.ones_like(shift))
+        y, t = forward_ad.unpack_dual(bn_relu.evaluate_sequence(seq, x))
+    assert torch.equal(t, (y > 0).float())
