@@ -6,7 +6,7 @@ backward over one synthetic batch that is already resident in HBM.
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu] [--no-fft]
 
 Prints ONE JSON line.  `roofline` is for the dominant kernel (the block-diagonal spectral
-product so3_mm, bound by the fp32 matrix cores), timed with events on the launch stream inside
+product so3_mm, bound by the matrix cores), timed with events on the launch stream inside
 the timed steps; `so3_fft` reports the standalone SO(3) FFT round trip of benchmark config 2
 against HBM bandwidth; `cpu_baseline` is the CPU oracle timed on this host on a bounded sample.
 """
@@ -21,13 +21,13 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
-PEAK_FP32_MFMA_TFLOPS = 157.3   # MI355X dense fp32 matrix
+PEAK_PRODUCT_TFLOPS = 416.7   # 2500 / 6, MI355X dense bf16 matrix: a float32 product takes six bf16 ones (csrc/split_bf16.h)
 PEAK_HBM_GBS = 8000.0           # MI355X HBM3E
 # HBM-side bytes per launch of the three product kernels at this workload, from rocprofv3 --pmc FETCH_SIZE /
 # WRITE_SIZE scaled by a 1 GiB elementwise kernel of the same run (profiles/so3_mm_real_b32_B16_F64_hbm_traffic.md);
 # not re-measured at run time.
-MM_TRAFFIC_BYTES = {"s2cnn_so3_mm_real_fwd": 6.67e9 + 0.179e9, "s2cnn_so3_mm_real_gradx": 6.61e9 + 0.179e9,
-                    "s2cnn_so3_mm_real_grady": 5.04e9 + 0.716e9}
+MM_TRAFFIC_BYTES = {"s2cnn_so3_mm_real_fwd": 3.53e9 + 0.179e9, "s2cnn_so3_mm_real_gradx": 3.61e9 + 0.179e9,
+                    "s2cnn_so3_mm_real_grady": 2.35e9 + 0.716e9}
 
 
 def sum_of_squares(t):
@@ -117,7 +117,7 @@ def measure_rows(torch, dev, with_cpu):
             ent = {"ms": round(ms, 4), "bound": "hbm", "achieved_GBs": round(rate / 1e9, 1), "frac": round(rate / 1e9 / PEAK_HBM_GBS, 4)}
         else:
             ent = {"ms": round(ms, 4), "bound": "mfma", "achieved_TFLOPs": round(rate / 1e12, 2),
-                   "frac": round(rate / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4)}
+                   "frac": round(rate / 1e12 / PEAK_PRODUCT_TFLOPS, 4)}
         if cpu_t is not None:
             ent["cpu_s_full_size_estimate"] = round(cpu_t / cpu_frac, 3)
             ent["cpu_sample"] = note
@@ -234,8 +234,8 @@ def measure_so3_mm(torch, dev, reps=5):
     """Benchmark config 3: the complex block product alone, x [43680, 16, 64, 2], y [43680, 64, 64, 2] with entries
     N(0, 1/64), forward and the gradients with respect to x and y, each timed with events on the launch stream.  The kernels
     form a complex product from three real ones (6 flops per complex multiply-add on the matrix cores instead of 8), so
-    `frac` = EXECUTED flops over the fp32 matrix peak (what the roofline bounds); `algorithmic_frac` counts the 8 flops of
-    the textbook complex multiply-add and can exceed 1."""
+    `frac` = EXECUTED flops over the peak for products of three bf16 parts (what the roofline bounds); `algorithmic_frac` counts the 8 flops of
+    the textbook complex multiply-add."""
     import s2cnn_amd
     from s2cnn_amd import _hip
     nl, B, Fi, Fo = 32, 16, 64, 64
@@ -258,13 +258,13 @@ def measure_so3_mm(torch, dev, reps=5):
     pc = {k: sum(v) / len(v) for k, v in kt.summary().items()}
     fl = mm_flops(nl, B, Fi, Fo, real=False)
     out = {"workload": "so3_mm fwd + grad x + grad y, x [43680,16,64,2], y [43680,64,64,2] (benchmark config 3)", "bound": "mfma",
-           "flop_per_launch": fl, "executed_flop_per_launch": 0.75 * fl, "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s"}
+           "flop_per_launch": fl, "executed_flop_per_launch": 0.75 * fl, "peak": PEAK_PRODUCT_TFLOPS, "unit": "TFLOP/s"}
     total = 0.0
     for name in ("s2cnn_so3_mm_fwd", "s2cnn_so3_mm_gradx", "s2cnn_so3_mm_grady"):
         ach = fl / (pc[name] * 1e-3) / 1e12
         total += pc[name]
-        out[name] = {"ms": round(pc[name], 3), "achieved": round(0.75 * ach, 2), "frac": round(0.75 * ach / PEAK_FP32_MFMA_TFLOPS, 4),
-                     "algorithmic_tflops": round(ach, 2), "algorithmic_frac": round(ach / PEAK_FP32_MFMA_TFLOPS, 4)}
+        out[name] = {"ms": round(pc[name], 3), "achieved": round(0.75 * ach, 2), "frac": round(0.75 * ach / PEAK_PRODUCT_TFLOPS, 4),
+                     "algorithmic_tflops": round(ach, 2), "algorithmic_frac": round(ach / PEAK_PRODUCT_TFLOPS, 4)}
     out["ms_fwd_bwd"] = round(total, 3)
     del x, y, gz
     torch.cuda.empty_cache()
@@ -594,8 +594,8 @@ def main():
     flops_of = {n: mm_flops(b, B, F, F, real="_real_" in n) for n in mm_names}
     flops = flops_of[dominant]
     ach = flops / (per_call[dominant] * 1e-3) / 1e12
-    roofline = {"bound": "mfma", "kernel": dominant, "achieved": round(ach, 2), "peak": PEAK_FP32_MFMA_TFLOPS,
-                "unit": "TFLOP/s", "frac": round(ach / PEAK_FP32_MFMA_TFLOPS, 4),
+    roofline = {"bound": "mfma", "kernel": dominant, "achieved": round(ach, 2), "peak": PEAK_PRODUCT_TFLOPS,
+                "unit": "TFLOP/s", "frac": round(ach / PEAK_PRODUCT_TFLOPS, 4),
                 "traffic": MM_TRAFFIC_BYTES.get(dominant) if (B, F, b) == (16, 64, 32) else None,
                 "traffic_source": "profiles/so3_mm_real_b32_B16_F64_hbm_traffic.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of "
                                   "this workload; not re-measured in this run)",
