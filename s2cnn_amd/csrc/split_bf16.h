@@ -31,11 +31,11 @@ struct SplitFragment { v8bf h, m, l; };
 
 // Whether a sum of part products is what a float32 product gives.  It is not where it is not finite (the parts of an infinity,
 // and of a value that rounds to one in bf16, are not its sum), and where operands are so small that their low parts are
-// subnormal in bf16, which the matrix cores take as zero: below 2^-108 beside operands of order one (relative errors of the products
-// at 2^-112: 1.3 times those at 1, at 2^-116: 13 times).
+// subnormal in bf16, which the matrix cores take as zero: below 2^-108 (relative errors of the products at 2^-112: 1.3 times
+// those at 1, at 2^-116: 13 times).  The line at 2^-70 takes in such values beside partners of up to 2^38.
 __device__ __forceinline__ bool sum_holds(float v) {
   const float a = fabsf(v);
-  return a == 0.f || (a >= 0x1p-100f && a <= 3.402823466e38f);
+  return a == 0.f || (a >= 0x1p-70f && a <= 3.402823466e38f);
 }
 
 __device__ __forceinline__ void split_octet(const float (&x)[8], uint4& h, uint4& m, uint4& l) {

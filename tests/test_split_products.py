@@ -170,3 +170,18 @@ def test_product_of_tiny_values(hip, nl, B, Fi, Fo, complex_):
     want = (product64_complex if complex_ else product64)("fwd", x, y, nl)
     got = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(x, y)
     assert ((got.double() - want).norm() / want.norm()).item() <= 4 * bound((2 * nl - 1) * Fi)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(3, 5, 9, 7), (16, 8, 40, 40)])      # either kernel
+@pytest.mark.parametrize("complex_", [False, True])
+def test_product_of_tiny_values_and_large_partners(hip, nl, B, Fi, Fo, complex_):
+    """The same where the other operand is large, so that the sums themselves are far from subnormal."""
+    import s2cnn_amd
+    ns, pair = O.nspec_so3(nl), (2,) if complex_ else ()
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn(ns, B, Fi, *pair, device="cuda", generator=g) * 2.0 ** -118
+    y = torch.randn(ns, Fi, Fo, *pair, device="cuda", generator=g) * 2.0 ** 30
+    want = (product64_complex if complex_ else product64)("fwd", x, y, nl)
+    got = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(x, y)
+    assert ((got.double() - want).norm() / want.norm()).item() <= 4 * bound((2 * nl - 1) * Fi)
