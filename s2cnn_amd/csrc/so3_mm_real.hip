@@ -49,6 +49,7 @@ constexpr int XCD_RUN = 32;       // consecutive tiles of the list that one XCD 
 constexpr int SMALL_GRID = 512;   // workgroups that fill the chip (2 per CU)
 constexpr int SLICES_GRID = 256;  // fewer 128 x 64 tiles than this: the kernel for small problems
 constexpr int SLICES_WIDE = 400;  // as many 32 x 64 tiles: two blocks per wave of it
+constexpr int CHAIN_STEPS = 256;  // contractions of the forward product up to this length: the kernel with one chain per result
 
 enum Mode { FWD = 0, GRADX = 1, GRADY = 2 };
 struct MmParams {
@@ -371,6 +372,95 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
   }
 }
 
+// Forward products of small problems with a short contraction, with the float32 matrix instruction: a wave owns 32 x 32 outputs
+// and takes the steps 8s + t, 8s + 4 + t (t = 0 .. 3) one pair after the other, so that a result is one chain of fused
+// multiply-adds, rounded once per step, in an order that does not depend on the tiling.  These products lie in front of the
+// activations of the small networks: a sample next to zero that falls on the other side of a ReLU is worth 5e-5 of a gradient of
+// the digit network, so the last bit is kept as it is.  What bounds it is the latency of the chain (64 clocks per pair) and of the
+// first loads; operands come straight from memory, 32 steps ahead.  us, slices -> this one: 6 degrees, 20 -> 40, batch 32: 5.6 -> 8.3, batch 1:
+// 4.5 -> 7.6, batch 64: 7.5 -> 8.8 (a pass of the digit network takes 200); 5 degrees, batch 16, 28 -> 28: 4.8 -> 8.9.  Features in multiples of four,
+// for wide loads (17 features: 14 against 6.5), and up to CHAIN_STEPS steps: from there on the chain costs several times the slices.
+__global__ __launch_bounds__(NT) void so3_block_mm_real_chain_kernel(MmParams p, int tiles) {
+  constexpr int T = 32, AHEAD = 4;      // groups of eight steps that are loaded together
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r32 = lane & 31, h = lane >> 5;
+  int t = blockIdx.x * (NT / 64) + wave;
+  if (t >= tiles) return;
+  int l = p.nl - 1, tm = 0, tn = 0, slots = 0;
+  for (;; --l) {
+    tile_counts(2 * l + 1, p.RI, p.CI, T, T, tm, tn, slots);
+    if (t < slots || l == 0) break;
+    t -= slots;
+  }
+  const int L = 2 * l + 1, M = L * p.RI, N = L * p.CI;
+  const int tile_m = t % tm * T, tile_n = t / tm * T;
+  const size_t L0 = (size_t)l * (4 * l * l - 1) / 3;
+  const int ablk = p.RI * p.KI, bblk = p.CI * p.KI;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.A + L0 * ablk), 0, 4 * L * L * ablk, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.B + L0 * bblk), 0, 4 * L * L * bblk, 0x00020000);
+  const int row = tile_m + r32, col = tile_n + r32, cb = col / p.CI, ci = col - cb * p.CI;
+  const unsigned ao = row < M ? 4u * (unsigned)(row / p.RI * L * ablk + row % p.RI * p.KI) : OUTSIDE;
+  const unsigned bo = col < N ? 4u * (unsigned)(cb * L * bblk + ci) : OUTSIDE;
+
+  // block and feature of the lane's first step of the group, and what they add to the offsets; a block that ends adds the way to the next
+  int kb = 4 * h / p.KI, kin = 4 * h - kb * p.KI;
+  const int adv_b = 8 / p.KI, adv_k = 8 - adv_b * p.KI;
+  const unsigned cross_a = 4u * (unsigned)(ablk - p.KI), cross_b = 4u * (unsigned)(bblk - p.KI * p.CI);
+  unsigned oa = ao + 4u * (unsigned)(kb * ablk + kin), ob = bo + 4u * (unsigned)(kb * bblk + kin * p.CI);
+  float a[2][AHEAD][4], b[2][AHEAD][4];
+  const auto load = [&](float (&av)[AHEAD][4], float (&bv)[AHEAD][4]) {
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(ra, (int)(kb < L ? oa : OUTSIDE), 0, 0);      // four steps never straddle a block
+      const unsigned at = kb < L ? ob : OUTSIDE;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        av[g][e] = __uint_as_float(v[e]);
+        bv[g][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rb, (int)at, 4 * e * p.CI, 0));
+      }
+      kin += adv_k;
+      kb += adv_b;
+      oa += 4u * (unsigned)(adv_b * ablk + adv_k);
+      ob += 4u * (unsigned)(adv_b * bblk + adv_k * p.CI);
+      if (kin >= p.KI) { kin -= p.KI; ++kb; oa += cross_a; ob += cross_b; }
+    }
+  };
+
+  v16f acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  const auto multiply = [&](const float (&av)[AHEAD][4], const float (&bv)[AHEAD][4]) {
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[g][e], bv[g][e], acc, 0, 0, 0);
+  };
+  const int K = L * p.KI;
+  load(a[0], b[0]);
+  for (int k0 = 0; k0 < K; k0 += 16 * AHEAD) {      // two rounds; steps behind the end are zeros
+    load(a[1], b[1]);
+    multiply(a[0], b[0]);
+    if (k0 + 8 * AHEAD >= K) break;
+    load(a[0], b[0]);
+    multiply(a[1], b[1]);
+  }
+
+  if (col >= N) return;
+  float* Cl = p.C + L0 * p.RI * p.CI;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int row0 = tile_m + 8 * g + 4 * h;
+    int rb_ = row0 / p.RI, ri = row0 - rb_ * p.RI;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (row0 + v < M) Cl[(size_t)(rb_ * L + cb) * (p.RI * p.CI) + ri * p.CI + ci] = acc[4 * g + v];
+      if (++ri == p.RI) { ri = 0; ++rb_; }
+    }
+  }
+}
+
 long total_slots(int nl, int RI, int CI, int TM, int TN) {
   long n = 0;
   for (int l = 0; l < nl; ++l) {
@@ -405,6 +495,11 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
   const bool divides = near && (C_::A_KC ? wa == 4 : a2) && (C_::B_KC ? wb == 4 : b2) && KI % 8 == 0 && (KI % TK == 0 || TK % KI == 0);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const long tiles64 = total_slots(nl, RI, CI, TM, 64);
+  if (MODE == FWD && near && tiles64 > 0 && tiles64 < SLICES_GRID && wa == 4 && Lmax * KI <= CHAIN_STEPS) {
+    const int tiles = (int)total_slots(nl, RI, CI, 32, 32);
+    hipLaunchKernelGGL(so3_block_mm_real_chain_kernel, dim3((unsigned)((tiles + NT / 64 - 1) / (NT / 64))), dim3(NT), 0, st, p, tiles);
+    return s2cnn::launch_status();
+  }
   if (near && tiles64 > 0 && tiles64 < SLICES_GRID) {
     const long tiles = total_slots(nl, RI, CI, 32, 64);
     const bool two = tiles >= SLICES_WIDE;

@@ -177,7 +177,8 @@ __global__ __launch_bounds__(256) void rft_expand_grad_kernel(const float* __res
 
 // ---- products with the small matrix of a grid
 // out [i][r][c] = scale sum_p E[i][p][r] x[c][idx[i][p]] and its adjoint gx[c][idx[i][p]] = scale sum_r Et[i][r][p] g[i][r][c], on the
-// bf16 matrix cores with operands cut into three parts (split_bf16.h), straight from memory, in blocks of 32 x 32 outputs.
+// bf16 matrix cores with operands cut into three parts (split_bf16.h), straight from memory, in blocks of 32 x 32 outputs; the smallest
+// with the float32 instruction (planes_chain_kernel).
 // fa(k): the lane's row of the first operand at contraction step k < K; fb(k, j): its column of block j of the second.
 
 template <int N, class F>
@@ -261,23 +262,71 @@ __device__ __forceinline__ void split_product(int K, int wave, int lane, FA fa, 
   }
 }
 
-// the sample that group member k of beta i contributes to column col (-1 in idx: no such member)
+// scale times the sample that group member k of beta i contributes to column col (-1 in idx: no such member), rounded as a product of
+// tensors is: what the layer's kernel times its factor gives
 struct Samples {
   const float* x;
   const int* idx;
   int npts;
+  float scale;
   bool ok;
-  __device__ __forceinline__ Samples(const float* x_, const int* idx_, int i, int P, int npts_, long col, long ncols)
-      : x(x_ + (col < ncols ? col : 0) * npts_), idx(idx_ ? idx_ + (size_t)i * P : nullptr), npts(npts_), ok(col < ncols) {}
+  __device__ __forceinline__ Samples(const float* x_, const int* idx_, int i, int P, int npts_, long col, long ncols, float scale_)
+      : x(x_ + (col < ncols ? col : 0) * npts_), idx(idx_ ? idx_ + (size_t)i * P : nullptr), npts(npts_), scale(scale_), ok(col < ncols) {}
   __device__ __forceinline__ float operator()(int k) const {
     const int q = idx ? idx[k] : k;
     const bool in = ok && (unsigned)q < (unsigned)npts;
     const float v = x[in ? q : 0];
-    return in ? v : 0.f;
+    return in ? scale * v : 0.f;
   }
 };
 
-// few blocks, or many points: the contraction split over the waves
+// Up to 16 STEPS points and few outputs, with the float32 matrix instruction: a wave owns 16 x 16 outputs, and a result is one chain
+// of fused multiply-adds in the order in which the library's products take the points: groups of points (idx) one after the
+// other, a single group by 0 2 4 6 1 3 5 7 within each eight of the whole sixteens and the rest one after the other.  So the spectra of the
+// layers of a small network are bit for bit those of the public transforms, as the products behind them are kept (see
+// so3_block_mm_real_chain_kernel).  Bound by the latency of two dependent loads, all of them in flight together.
+constexpr int STEPS = 4;
+template <bool GROUPS>
+__global__ __launch_bounds__(256) void planes_chain_kernel(const float* __restrict__ x, const int* __restrict__ idx, const float* __restrict__ E,
+                                                           float* __restrict__ out, int P, int R, int npts, long ncols, long ld, float scale) {
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
+  const int row0 = (blockIdx.y * 4 + wave) * 16, row = row0 + r16;
+  if (row0 >= R) return;
+  const long col = (long)blockIdx.x * 16 + r16;
+  const bool rok = row < R;
+  const float* e = E + (size_t)blockIdx.z * P * R + (rok ? row : 0);
+  const Samples s(x, idx, blockIdx.z, P, npts, col, ncols, scale);
+  float a[STEPS][4], b[STEPS][4];
+#pragma unroll
+  for (int q = 0; q < STEPS; ++q) {
+    const bool whole = !GROUPS && 16 * q + 16 <= P;
+    if (16 * q < P) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = 16 * q + (whole ? 8 * (j / 2) + (j & 1) + 2 * g : 4 * j + g), kc = k < P ? k : 0;
+        const float av = e[(size_t)kc * R], bv = s(kc);
+        a[q][j] = rok && k < P ? av : 0.f;
+        b[q][j] = k < P ? bv : 0.f;
+      }
+    }
+  }
+  v4f acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < STEPS; ++q)
+    if (16 * q < P)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][j], b[q][j], acc, 0, 0, 0);
+  if (!s.ok) return;
+  float* o = out + (size_t)blockIdx.z * R * ld + col;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {      // register v of lane (r16, g) holds row 4 g + v and column r16
+    const int r = row0 + 4 * g + v;
+    if (r < R) o[(size_t)r * ld] = acc[v];
+  }
+}
+
+// few blocks of many points: the contraction split over the waves
 __global__ __launch_bounds__(256) void planes_split_kernel(const float* __restrict__ x, const int* __restrict__ idx, const float* __restrict__ E,
                                                            float* __restrict__ out, int P, int R, int npts, long ncols, long ld, float scale) {
   __shared__ float part[4][1][16][64];
@@ -286,13 +335,13 @@ __global__ __launch_bounds__(256) void planes_split_kernel(const float* __restri
   const int row0 = blockIdx.y * 32, row = row0 + r32;
   const bool rok = row < R;
   const float* e = E + (size_t)blockIdx.z * P * R + (rok ? row : 0);
-  const Samples s(x, idx, blockIdx.z, P, npts, col, ncols);
+  const Samples s(x, idx, blockIdx.z, P, npts, col, ncols, scale);
   float* o = out + (size_t)blockIdx.z * R * ld + col;
   split_product<4, 1>(
       P, wave, lane, [&](int k) { return rok ? e[(size_t)k * R] : 0.f; }, [&](int k, int) { return s(k); },
       [&](int v, int, float z) {
         const int r = row0 + 8 * (v / 4) + 4 * h + v % 4;
-        if (s.ok && r < R) o[(size_t)r * ld] = scale * z;
+        if (s.ok && r < R) o[(size_t)r * ld] = z;
       },
       part);
 }
@@ -301,7 +350,7 @@ __global__ __launch_bounds__(256) void planes_split_kernel(const float* __restri
 // ROW_BLOCKS blocks of 32 rows of E, each cut into parts once (an octet per thread) and read by the four waves from LDS.  Three betas of
 // 64 points, 4 032 rows, 4 096 columns (198 MB of results): 98 us (129 with every wave cutting the rows for itself; the gather,
 // masking, scaling and library product that this stands for: 131).
-constexpr int STEPS = 4, ROW_BLOCKS = 8, WALK_GRID = 208;
+constexpr int ROW_BLOCKS = 8, WALK_GRID = 208;
 __global__ __launch_bounds__(256) void planes_kernel(const float* __restrict__ x, const int* __restrict__ idx, const float* __restrict__ E,
                                                      float* __restrict__ out, int P, int R, int npts, long ncols, long ld, float scale) {
   static_assert(32 * 2 * STEPS == 256, "an octet of the block per thread");
@@ -309,7 +358,7 @@ __global__ __launch_bounds__(256) void planes_kernel(const float* __restrict__ x
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r32 = lane & 31, h = lane >> 5;
   const int trow = threadIdx.x & 31, toct = threadIdx.x >> 5;
   const long col = (long)blockIdx.x * 128 + 32 * wave + r32;
-  const Samples s(x, idx, blockIdx.z, P, npts, col, ncols);
+  const Samples s(x, idx, blockIdx.z, P, npts, col, ncols, scale);
   const float* Ei = E + (size_t)blockIdx.z * P * R;
   float* o = out + (size_t)blockIdx.z * R * ld + col;
   const int first = blockIdx.y * ROW_BLOCKS * 32, last = first + ROW_BLOCKS * 32 < R ? first + ROW_BLOCKS * 32 : R;
@@ -355,7 +404,7 @@ __global__ __launch_bounds__(256) void planes_kernel(const float* __restrict__ x
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int r = row0 + 8 * (v / 4) + 4 * h + v % 4;
-      if (s.ok && r < R) o[(size_t)r * ld] = scale * acc[v];
+      if (s.ok && r < R) o[(size_t)r * ld] = acc[v];
     }
     __syncthreads();
   }
@@ -399,10 +448,21 @@ int check_planes(const void* a, const void* E, const void* o, int nbeta, int P, 
 // Row blocks in a walk pay once there are workgroups for most CUs and the samples of a column fit the registers.  us split -> walk:
 // 158 workgroups (32 points, 760 rows, 10 000 columns) 19 -> 31; 192 (14 points, 182 rows, 24 500 columns) 22 -> 27; 224 (64 points,
 // 1 892 rows, 3 500 columns) 43 -> 34; 1 536 (three times 64 points, 4 032 rows, 4 096 columns) 245 -> 98.
+// Fewer of both: one chain per result, up to CHAIN_LOADS loads of either operand by its waves.  us split -> chain (with the expansion where
+// there are betas): 24 points, 100 rows, 20 columns (70 tiles of 16 x 16) 3.5 -> 3.6; 400 rows, 78 columns (125) 6.2 -> 3.8; 1 024 rows, 600 columns
+// (2 432) 7.9 -> 6.0; three times 64 points, 132 rows, 800 columns (1 350) 9.2 -> 11.2; 380 rows, 400 columns (1 800) 10.7 -> 12.9; 650 rows,
+// 1 485 columns (11 439) 31 -> 48.
+constexpr long CHAIN_LOADS = 96 * 1024;      // 16 x 16 tiles times points
 int planes(const float* x, const int* idx, const float* E, float* out, int nbeta, int P, int R, int npts, long ncols, long ld, float scale, hipStream_t st) {
-  const dim3 wide((unsigned)((ncols + 127) / 128), (R + ROW_BLOCKS * 32 - 1) / (ROW_BLOCKS * 32), nbeta), narrow((unsigned)((ncols + 31) / 32), (R + 31) / 32, nbeta);
+  const dim3 wide((unsigned)((ncols + 127) / 128), (R + ROW_BLOCKS * 32 - 1) / (ROW_BLOCKS * 32), nbeta), narrow((unsigned)((ncols + 31) / 32), (R + 31) / 32, nbeta),
+      chain((unsigned)((ncols + 15) / 16), (R + 63) / 64, nbeta);
+  const bool chains = P <= 16 * STEPS && (long)chain.x * ((R + 15) / 16) * nbeta * P <= CHAIN_LOADS;
   if (P <= 16 * STEPS && (long)wide.x * wide.y * wide.z >= WALK_GRID)
     hipLaunchKernelGGL(planes_kernel, wide, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
+  else if (chains && idx)
+    hipLaunchKernelGGL(planes_chain_kernel<true>, chain, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
+  else if (chains)
+    hipLaunchKernelGGL(planes_chain_kernel<false>, chain, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
   else
     hipLaunchKernelGGL(planes_split_kernel, narrow, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
   return s2cnn::launch_status();

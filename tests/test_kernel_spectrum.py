@@ -4,6 +4,8 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import cpu_path as O
+
 pytestmark = pytest.mark.gpu
 
 
@@ -75,6 +77,50 @@ def test_kernel_spectrum_of_values_without_bf16_parts(hip):
     want = torch.from_numpy(wigner.so3_ft_matrix_real(b, grid)).t() @ k.double().reshape(45, -1)[finite].t() * 0.0625
     err = (y[:, finite].double() - want).norm(dim=0) / want.norm(dim=0)
     assert err.max().item() <= 4 * bound(len(grid))          # per column, with a quarter of the chip's columns as room
+
+
+def chain(A, B, order):
+    """A [M, K] B [K, N] in float32 as one chain of fused multiply-adds per entry (exact products; sums rounded to float64 on the way,
+    which is another result once in 2^29 times)."""
+    acc = torch.zeros(A.shape[0], B.shape[1], device=A.device)
+    for k in order:
+        acc = (A[:, k, None].double() * B[None, k].double() + acc.double()).float()
+    return acc
+
+
+@pytest.mark.parametrize("b,shape", [(10, (1, 20)), (2, (1, 1)), (20, (3, 26))])
+@pytest.mark.parametrize("n_alpha", [8, 5, 1])
+def test_s2_kernel_spectra_of_small_layers_are_chains(hip, b, shape, n_alpha):
+    """24, 15 and 3 points: one chain per entry, from the rounded product of kernel and factor, by 0 2 4 6 1 3 5 7 within each eight of the whole
+    sixteens and the rest in sequence, bit for bit: what s2_rft_real's library product gave these layers (24 points)."""
+    import s2cnn_amd
+    from s2cnn_amd.s2_real import _setup_s2_ft_real, scaled_kernel_spectrum
+    grid = s2cnn_amd.s2_near_identity_grid(n_alpha=n_alpha)
+    P = len(grid)
+    k = torch.randn(*shape, P, generator=torch.Generator().manual_seed(b)).cuda()
+    m = P // 16 * 16
+    order = [8 * s + t for s in range(m // 8) for t in (0, 2, 4, 6, 1, 3, 5, 7)] + list(range(m, P))
+    F = _setup_s2_ft_real(b, grid, k.device)
+    y = scaled_kernel_spectrum(k, 0.37, b, grid)
+    assert torch.equal(y.reshape(F.size(1), -1), chain(F.t(), (k * 0.37).reshape(-1, P).t(), order))
+
+
+@pytest.mark.parametrize("b,shape", [(6, (20, 40)), (2, (3, 4)), (5, (1, 36))])
+def test_so3_kernel_spectra_of_small_layers_are_chains(hip, b, shape):
+    """The plane coefficients of each beta as one chain over its points in their order, then the expansion: bit for bit the library product
+    and expansion that these layers' spectra were formed with."""
+    import s2cnn_amd
+    from s2cnn_amd import _hip, wigner
+    from s2cnn_amd.so3_real import scaled_kernel_spectrum
+    grid = s2cnn_amd.so3_near_identity_grid()
+    idx, E, dtab = wigner.so3_rft_plan(b, grid)
+    E, dtab = (torch.from_numpy(t.astype(np.float32)).cuda().contiguous() for t in (E, dtab))
+    k = torch.randn(*shape, len(grid), generator=torch.Generator().manual_seed(b)).cuda()
+    ks = (k * 0.37).reshape(-1, len(grid))
+    G = torch.stack([chain(E[i].t(), ks[:, torch.from_numpy(idx[i]).long().cuda()].t(), range(idx.shape[1])) for i in range(len(idx))]).contiguous()
+    want = torch.empty(O.nspec_so3(b), ks.size(0), device="cuda")
+    _hip.call("s2cnn_so3_rft_expand_real", _hip.ptr(G), _hip.ptr(dtab), _hip.ptr(want), b, len(idx), ks.size(0), _hip.stream_ptr())
+    assert torch.equal(scaled_kernel_spectrum(k, 0.37, b, grid).reshape(want.shape), want)
 
 
 def test_kernel_spectrum_gradient_of_the_gradient(hip):

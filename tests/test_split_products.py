@@ -185,3 +185,33 @@ def test_product_of_tiny_values_and_large_partners(hip, nl, B, Fi, Fo, complex_)
     want = (product64_complex if complex_ else product64)("fwd", x, y, nl)
     got = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(x, y)
     assert ((got.double() - want).norm() / want.norm()).item() <= 4 * bound((2 * nl - 1) * Fi)
+
+
+def chain(A, B, order):
+    """A [M, K] B [K, N] in float32 as one chain of fused multiply-adds per entry (exact products; sums rounded to float64 on the way,
+    which is another result once in 2^29 times)."""
+    acc = torch.zeros(A.shape[0], B.shape[1], device=A.device)
+    for k in order:
+        acc = (A[:, k, None].double() * B[None, k].double() + acc.double()).float()
+    return acc
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(1, 1, 4, 1), (2, 3, 8, 5), (4, 33, 36, 7), (6, 32, 20, 40), (6, 1, 20, 40), (3, 70, 12, 33)])
+def test_short_forward_products_are_chains(hip, nl, B, Fi, Fo):
+    """Forward products of the small networks: every result is one chain in the order 8s + t, 8s + 4 + t, bit for bit.  A ReLU
+    behind them takes a sample next to zero or leaves it by the last bit."""
+    import s2cnn_amd
+    ns = O.nspec_so3(nl)
+    g = torch.Generator(device="cuda").manual_seed(nl)
+    x, y = torch.randn(ns, B, Fi, device="cuda", generator=g), torch.randn(ns, Fi, Fo, device="cuda", generator=g)
+    z = s2cnn_amd.so3_mm_real(x, y)
+    pos = 0
+    for l in range(nl):
+        L = 2 * l + 1
+        A = x[pos:pos + L * L].reshape(L, L, B, Fi).transpose(1, 2).reshape(L * B, L * Fi)
+        Y = y[pos:pos + L * L].reshape(L, L, Fi, Fo).permute(1, 2, 0, 3).reshape(L * Fi, L * Fo)
+        order = [8 * s + 4 * h + t for s in range((L * Fi + 7) // 8) for t in range(4) for h in range(2)]
+        want = chain(A, Y, [k for k in order if k < L * Fi]).reshape(L, B, L, Fo).transpose(1, 2).reshape(L * L, B, Fo)
+        assert torch.equal(z[pos:pos + L * L], want), l
+        pos += L * L
