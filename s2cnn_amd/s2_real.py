@@ -44,15 +44,19 @@ def s2_spectrum_to_real(x):
     return (x.index_select(0, src) * w).sum(-1)
 
 
-@lru_cache(maxsize=32)
-def _setup_s2_ft_real(b, grid, device):
+def _s2_ft_real_matrix(b, grid):
     F = wigner.s2_ft_matrix(b, grid)                       # [n_grid, b^2] complex
     out = np.empty(F.shape, dtype=np.float64)
     for l in range(b):
         for r in range(-l, l + 1):
             col = F[:, l * l + l + abs(r)]
             out[:, l * l + l + r] = col.real if r == 0 else math.sqrt(2.0) * (col.real if r > 0 else col.imag)
-    return torch.tensor(out.astype(np.float32), dtype=torch.float32, device=device)
+    return out.astype(np.float32)
+
+
+@lru_cache(maxsize=32)
+def _setup_s2_ft_real(b, grid, device):
+    return torch.tensor(_s2_ft_real_matrix(b, grid), dtype=torch.float32, device=device)
 
 
 def s2_rft_real(x, b, grid):
@@ -70,9 +74,10 @@ def s2_rft_real(x, b, grid):
 
 @lru_cache(maxsize=32)
 def _setup_s2_rft_plan(b, grid, device):
-    """The matrix of `_setup_s2_ft_real` and its transpose, for the product and its adjoint."""
-    F = _setup_s2_ft_real(b, grid, device)
-    return F, F.t().contiguous()
+    """The matrix of `_setup_s2_ft_real` and its transpose, for the product and its adjoint.  Transposed on the host, then copies
+    that wait: a kernel would run on the first caller's stream only, and others read the plan too."""
+    F = _s2_ft_real_matrix(b, grid)
+    return torch.tensor(F, device=device), torch.tensor(np.ascontiguousarray(F.T), device=device)
 
 
 class _KernelSpectrum(torch.autograd.Function):

@@ -120,15 +120,15 @@ def _setup_so3_ft_real(b, grid, device):
 @lru_cache(maxsize=32)
 def _setup_so3_rft_plan(b, grid, device):
     """Factorised form of the matrix of `_setup_so3_ft_real` for grids with few distinct beta values
-    (wigner.so3_rft_plan): (idx, E, its transpose per beta, dtab) on the device; None where it does not apply."""
+    (wigner.so3_rft_plan): (idx, E, its transpose per beta, dtab) on the device; None where it does not apply.
+    Whole on the host, then copies that wait: a kernel would run on the first caller's stream only, and others read the plan too."""
     plan = wigner.so3_rft_plan(b, grid)
     if plan is None:
         return None
     idx, E, dtab = plan
-    return (torch.tensor(idx.astype(np.int32), device=device).contiguous(),
-            torch.tensor(E.astype(np.float32), device=device).contiguous(),
-            torch.tensor(E.astype(np.float32), device=device).transpose(1, 2).contiguous(),
-            torch.tensor(dtab.astype(np.float32), device=device).contiguous())
+    E = E.astype(np.float32)
+    return tuple(torch.tensor(np.ascontiguousarray(t), device=device)
+                 for t in (idx.astype(np.int32), E, E.transpose(0, 2, 1), dtab.astype(np.float32)))
 
 
 class _KernelSpectrum(torch.autograd.Function):
