@@ -266,7 +266,7 @@ def evaluate_sequence(sequence, x):
             a = torch.rsqrt(bn.running_var + bn.eps)
             if bn.weight is not None:
                 a = a * bn.weight
-            shift = (conv.bias.reshape(-1) - bn.running_mean) * a
+            shift = (-bn.running_mean if conv.bias is None else conv.bias.reshape(-1) - bn.running_mean) * a
             if bn.bias is not None:
                 shift = shift + bn.bias
             zr = conv.product_spectrum(x, kernel=conv.kernel * a.view(1, -1, 1))

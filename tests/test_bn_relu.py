@@ -335,3 +335,17 @@ def test_tangents_of_a_normalisation_pass_the_modules(hip):
         seq[1].bias = forward_ad.make_dual(shift, torch.ones_like(shift))
         y, t = forward_ad.unpack_dual(bn_relu.evaluate_sequence(seq, x))
     assert torch.equal(t, (y > 0).float())
+
+
+def test_folding_of_a_layer_without_bias(hip):
+    """A normalisation takes a bias in front of it off again, so networks drop it: layer.bias = None."""
+    import s2cnn_amd
+    from torch import nn
+    torch.manual_seed(3)
+    seq = nn.Sequential(s2cnn_amd.S2Convolution(2, 4, 8, 5, s2cnn_amd.s2_near_identity_grid()), nn.BatchNorm3d(4), nn.ReLU()).cuda().eval()
+    seq[0].bias = None
+    seq[1].running_mean.normal_(0.3, 0.5)
+    x = torch.randn(2, 2, 16, 16, device="cuda")
+    with torch.no_grad():
+        want, got = seq(x), bn_relu.evaluate_sequence(seq, x)
+    assert not torch.equal(want, got) and _rel(got.double(), want.double()) < 2e-6
