@@ -235,8 +235,8 @@ def run_sequence(sequence, x, head=None):
 
 
 def _hooked(*mods):
-    """Whether a call of one of the modules does more than its forward."""
-    return (any(m._forward_hooks or m._forward_pre_hooks for m in mods)
+    """Whether a call of one of the modules does more than, or something else than, its class's forward."""
+    return (any(m._forward_hooks or m._forward_pre_hooks or "forward" in vars(m) for m in mods)
             or bool(_nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks))
 
 

@@ -349,3 +349,17 @@ def test_folding_of_a_layer_without_bias(hip):
     with torch.no_grad():
         want, got = seq(x), bn_relu.evaluate_sequence(seq, x)
     assert not torch.equal(want, got) and _rel(got.double(), want.double()) < 2e-6
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_modules_with_a_forward_of_their_own_run(hip, which):
+    """Tools that record or replace a module's result set `forward` on the instance."""
+    import s2cnn_amd
+    from torch import nn
+    torch.manual_seed(4)
+    seq = nn.Sequential(s2cnn_amd.S2Convolution(2, 4, 8, 5, s2cnn_amd.s2_near_identity_grid()), nn.BatchNorm3d(4), nn.ReLU()).cuda().eval()
+    x = torch.randn(2, 2, 16, 16, device="cuda")
+    inner = seq[which].forward
+    seq[which].forward = lambda t: inner(t) * 2 + 1
+    with torch.no_grad():
+        assert torch.equal(bn_relu.evaluate_sequence(seq, x), seq(x))
