@@ -14,6 +14,7 @@
 #include "common.h"
 #include "split_bf16.h"
 #include "block_loader.h"
+#include "block_float32.h"
 
 namespace {
 
@@ -70,70 +71,24 @@ __device__ __forceinline__ int find_degree(const MmParams& p, int TMV, int TNV, 
 }
 
 // what one of the three products takes from a complex operand: b carries the sign of the conjugation
-template <int KIND> __device__ __forceinline__ float part_of(float2 v) { return KIND == RE ? v.x : KIND == IM ? v.y : v.x + v.y; }
+__device__ __forceinline__ float part_of(float2 v, int kind) { return kind == RE ? v.x : kind == IM ? v.y : v.x + v.y; }
 template <bool CONJ> __device__ __forceinline__ float2 conj_of(float2 v) { return CONJ ? make_float2(v.x, -v.y) : v; }
-
-// A real product of a tile with the float32 matrix instruction, operands straight from memory: for tiles in which the sums of
-// the parts do not hold.  Here infinities, values that round to one in bf16 and tiny values take part as they are, so
-// overflow, infinities and NaN come out as in a float32 product of the same form.
-template <typename C_, int KIND, int NI, int NJ, int STEP>
-__device__ __forceinline__ void contract_float32(const MmParams& p, const float2* A, const float2* B, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h) {
-  const int K = L * p.KI;
-  size_t ao[NI], bo[NJ];
-  bool aok[NI], bok[NJ];
-  const size_t ablk = (size_t)p.RI * p.KI, bblk = (size_t)p.CI * p.KI;
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int row = row0 + STEP * i, rb = row / p.RI, ri = row - rb * p.RI;
-    aok[i] = row < L * p.RI;
-    ao[i] = (C_::A_MNMAJ ? (size_t)rb * L : (size_t)rb) * ablk + (size_t)ri * (C_::A_KC ? p.KI : 1);
-  }
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int col = col0 + STEP * j, cb = col / p.CI, ci = col - cb * p.CI;
-    bok[j] = col < L * p.CI;
-    bo[j] = (C_::B_MNMAJ ? (size_t)cb * L : (size_t)cb) * bblk + (size_t)ci * (C_::B_KC ? p.KI : 1);
-  }
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  int kb = h / p.KI, kin = h - kb * p.KI;
-  for (int k0 = 0; k0 < K; k0 += 2) {
-    const bool ok = k0 + h < K;
-    const size_t ka = (C_::A_MNMAJ ? (size_t)kb : (size_t)kb * L) * ablk + (size_t)kin * (C_::A_KC ? 1 : p.RI);
-    const size_t kbo = (C_::B_MNMAJ ? (size_t)kb : (size_t)kb * L) * bblk + (size_t)kin * (C_::B_KC ? 1 : p.CI);
-    float a[NI], b[NJ];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) a[i] = ok && aok[i] ? part_of<KIND>(A[ao[i] + ka]) : 0.f;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) b[j] = ok && bok[j] ? part_of<KIND>(conj_of<C_::CONJ>(B[bo[j] + kbo])) : 0.f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    kin += 2;
-    while (kin >= p.KI) { kin -= p.KI; ++kb; }
-  }
-}
 
 // One operand's tile in LDS: real parts, imaginary parts (with the sign of the conjugation), their sums, each in bf16 parts.
 struct OperandTile {
   SplitTile<TM, TK> kind[3];
 
   template <bool CONJ> __device__ __forceinline__ void put(int row, int octet, const float2 (&v)[8]) {
-    float x[8];
+    float re[8], im[8], sum[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = v[e].x;
-    kind[RE].put(row, octet, x);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = CONJ ? -v[e].y : v[e].y;
-    kind[IM].put(row, octet, x);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = CONJ ? v[e].x - v[e].y : v[e].x + v[e].y;
-    kind[SUM].put(row, octet, x);
+    for (int e = 0; e < 8; ++e) {
+      re[e] = s2cnn::SCALE * v[e].x;
+      im[e] = (CONJ ? -s2cnn::SCALE : s2cnn::SCALE) * v[e].y;
+      sum[e] = re[e] + im[e];
+    }
+    kind[RE].put<true>(row, octet, re);
+    kind[IM].put<true>(row, octet, im);
+    kind[SUM].put<true>(row, octet, sum);
   }
 };
 
@@ -252,21 +207,10 @@ __global__ __launch_bounds__(NT, 3) void so3_block_mm_kernel(MmParams p) {
   const bool full = ni == NB && nj == NB;
   const int nstage = s2cnn::ceil_div(L * p.KI, TK);
   const int u = threadIdx.x & (GROUP - 1);
-  const auto holds = [&]() {
-    bool ok = true;
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) ok = ok && s2cnn::sum_holds(acc[i][j][v]);
-    return __all(ok);
-  };
 #define S2CNN_GROUP(G, LDR)                                                                                                       \
   do {                                                                                                                            \
     if (full) contract<G, true, C_::CONJ>(LDR, s, acc, nstage, row, octet, wrow + r32, wcol + r32, h, ni, nj);                     \
     else contract<G, false, C_::CONJ>(LDR, s, acc, nstage, row, octet, wrow + r32, wcol + r32, h, ni, nj);                         \
-    if (!holds()) contract_float32<C_, G, NB, NB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);            \
   } while (0)
   if (group == 0) {            // K-contiguous: two threads on a row; MN-contiguous: neighbouring threads on neighbouring rows
     const int row = C_::A_KC ? u >> 1 : u & (TM - 1), octet = C_::A_KC ? u & 1 : u / TM;
@@ -284,6 +228,17 @@ __global__ __launch_bounds__(NT, 3) void so3_block_mm_kernel(MmParams p) {
     S2CNN_GROUP(2, ld);
   }
 #undef S2CNN_GROUP
+  bool finite = true;
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) finite = finite && s2cnn::finite(acc[i][j]);
+  float unscale = s2cnn::UNSCALE;
+  if (!__all(finite)) {
+    contract_float32<C_, NB, NB, BSTR>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h,
+                                       [&](float2 v) { return part_of(v, group); }, [&](float2 v) { return part_of(conj_of<C_::CONJ>(v), group); });
+    unscale = 1.f;
+  }
 
   // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32 of its 32x32 block.  64 rows of the tile at a
   // time; a thread stores every sixth row of one column.
@@ -298,7 +253,7 @@ __global__ __launch_bounds__(NT, 3) void so3_block_mm_kernel(MmParams p) {
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v)
-        s.product[group][wrow + 8 * (v / 4) + 4 * h + v % 4][wcol + BSTR * j + r32] = acc[i][j][v];
+        s.product[group][wrow + 8 * (v / 4) + 4 * h + v % 4][wcol + BSTR * j + r32] = unscale * acc[i][j][v];
     __syncthreads();
     if (col < N) {
       for (int r = threadIdx.x / TM; r < 64; r += NT / TM) {
@@ -395,20 +350,25 @@ __global__ __launch_bounds__(NTS) void so3_block_mm_slices_kernel(MmParams p) {
   for (int v = 0; v < 16; ++v) { part[wave][0][v][lane] = re[v]; part[wave][1][v][lane] = im[v]; }
   __syncthreads();
   float2 sum[4];
-  bool holds = true;
+  float part_sums[8];
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     float2 z = make_float2(part[0][0][4 * wave + v][lane], part[0][1][4 * wave + v][lane]);
 #pragma unroll
     for (int w = 1; w < NW; ++w) { z.x += part[w][0][4 * wave + v][lane]; z.y += part[w][1][4 * wave + v][lane]; }
-    sum[v] = z;
-    holds = holds && s2cnn::sum_holds(z.x) && s2cnn::sum_holds(z.y);
+    part_sums[2 * v] = z.x;
+    part_sums[2 * v + 1] = z.y;
+    sum[v] = make_float2(s2cnn::UNSCALE * z.x, s2cnn::UNSCALE * z.y);
   }
-  if (!__all(holds)) {
+  if (!__all(s2cnn::finite(part_sums))) {
     v16f p1[1][1], p2[1][1], p3[1][1];
-    contract_float32<C_, RE, 1, 1, 32>(p, A, B, p1, L, tile_m + r32, tile_n + r32, h);
-    contract_float32<C_, IM, 1, 1, 32>(p, A, B, p2, L, tile_m + r32, tile_n + r32, h);
-    contract_float32<C_, SUM, 1, 1, 32>(p, A, B, p3, L, tile_m + r32, tile_n + r32, h);
+    const auto contract_kind = [&](int kind, v16f (&acc)[1][1]) {
+      contract_float32<C_, 1, 1, 32>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + r32, tile_n + r32, h, [&](float2 v) { return part_of(v, kind); },
+                                     [&](float2 v) { return part_of(conj_of<C_::CONJ>(v), kind); });
+    };
+    contract_kind(RE, p1);
+    contract_kind(IM, p2);
+    contract_kind(SUM, p3);
 #pragma unroll
     for (int v = 0; v < 16; ++v)
       if (v / 4 == wave) sum[v % 4] = make_float2(p1[0][0][v] - p2[0][0][v], p3[0][0][v] - p1[0][0][v] - p2[0][0][v]);

@@ -32,6 +32,7 @@
 #include "common.h"
 #include "split_bf16.h"
 #include "block_loader.h"
+#include "block_float32.h"
 
 namespace {
 
@@ -92,52 +93,6 @@ __host__ __device__ inline void tile_counts(int L, int RI, int CI, int TM, int T
   tm = s2cnn::ceil_div(L * RI, TM);
   tn = s2cnn::ceil_div(L * CI, TN);
   slots = tm * tn;
-}
-
-// The tile again with the float32 matrix instruction, operands straight from memory: for tiles in which a sum of the parts does
-// not hold.  Here infinities, values that round to one in bf16 and tiny values take part as they are, so overflow,
-// infinities and NaN come out as in any float32 product.
-template <typename C_, int NI, int NJ, int STEP>
-__device__ __forceinline__ void contract_float32(const MmParams& p, const float* A, const float* B, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h) {
-  const int K = L * p.KI;
-  size_t ao[NI], bo[NJ];
-  bool aok[NI], bok[NJ];
-  const size_t ablk = (size_t)p.RI * p.KI, bblk = (size_t)p.CI * p.KI;
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int row = row0 + STEP * i, rb = row / p.RI, ri = row - rb * p.RI;
-    aok[i] = row < L * p.RI;
-    ao[i] = (C_::A_MNMAJ ? (size_t)rb * L : (size_t)rb) * ablk + (size_t)ri * (C_::A_KC ? p.KI : 1);
-  }
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) {
-    const int col = col0 + STEP * j, cb = col / p.CI, ci = col - cb * p.CI;
-    bok[j] = col < L * p.CI;
-    bo[j] = (C_::B_MNMAJ ? (size_t)cb * L : (size_t)cb) * bblk + (size_t)ci * (C_::B_KC ? p.KI : 1);
-  }
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  int kb = h / p.KI, kin = h - kb * p.KI;
-  for (int k0 = 0; k0 < K; k0 += 2) {
-    const bool ok = k0 + h < K;
-    const size_t ka = (C_::A_MNMAJ ? (size_t)kb : (size_t)kb * L) * ablk + (size_t)kin * (C_::A_KC ? 1 : p.RI);
-    const size_t kbo = (C_::B_MNMAJ ? (size_t)kb : (size_t)kb * L) * bblk + (size_t)kin * (C_::B_KC ? 1 : p.CI);
-    float a[NI], b[NJ];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) a[i] = ok && aok[i] ? A[ao[i] + ka] : 0.f;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) b[j] = ok && bok[j] ? B[bo[j] + kbo] : 0.f;
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-    kin += 2;
-    while (kin >= p.KI) { kin -= p.KI; ++kb; }
-  }
 }
 
 // One LDS buffer: the operands of a stage are split and written while the loads of the next stage are issued, a barrier,
@@ -230,14 +185,17 @@ __global__ __launch_bounds__(NT, 2) void so3_block_mm_real_kernel(MmParams p) {
   else contract<NCB, false>(la, lb, As, Bs, acc, nstage, wrow + r32, wcol + r32, h, ni, nj);
 
   // Accumulator register v of lane (r32, h) holds row 8*(v/4) + 4*h + v%4 and column r32 of its 32x32 block.
-  bool holds = true;
+  bool finite = true;
 #pragma unroll
   for (int i = 0; i < NRB; ++i)
 #pragma unroll
-    for (int j = 0; j < NCB; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) holds = holds && s2cnn::sum_holds(acc[i][j][v]);
-  if (!__all(holds)) contract_float32<C_, NRB, NCB, BSTR>(p, A, B, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h);
+    for (int j = 0; j < NCB; ++j) finite = finite && s2cnn::finite(acc[i][j]);
+  const auto same = [](float v) { return v; };
+  float unscale = s2cnn::UNSCALE;
+  if (!__all(finite)) {
+    contract_float32<C_, NRB, NCB, BSTR>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h, same, same);
+    unscale = 1.f;
+  }
 
   float* Cl = p.C + L0 * p.RI * p.CI;
   const int blk_elems = p.RI * p.CI;
@@ -257,7 +215,7 @@ __global__ __launch_bounds__(NT, 2) void so3_block_mm_real_kernel(MmParams p) {
         for (int v = 0; v < 4; ++v) {
           if (row0 + v < M) {
             const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
-            Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = acc[i][j][4 * g + v];
+            Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = unscale * acc[i][j][4 * g + v];
           }
           if (++ri == p.RI) { ri = 0; ++rb; }
         }
@@ -332,7 +290,6 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
     for (int v = 0; v < 16; ++v) part[wave][j][v][lane] = acc[0][j][v];
   __syncthreads();
   float sum[NJ][4];
-  bool holds = true;
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -341,10 +298,15 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
 #pragma unroll
       for (int w = 1; w < NW; ++w) s += part[w][j][4 * wave + v][lane];
       sum[j][v] = s;
-      holds = holds && s2cnn::sum_holds(s);
     }
-  if (!__all(holds)) {
-    contract_float32<C_, 1, NJ, 32>(p, A, B, acc, L, tile_m + r32, tile_n + r32, h);
+  bool finite = true;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) finite = finite && s2cnn::finite(sum[j]);
+  float unscale = s2cnn::UNSCALE;
+  if (!__all(finite)) {
+    const auto same = [](float v) { return v; };
+    contract_float32<C_, 1, NJ, 32>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + r32, tile_n + r32, h, same, same);
+    unscale = 1.f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -365,7 +327,7 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
     for (int v = 0; v < 4; ++v) {
       if (row0 + v < M) {
         const int blk = C_::C_RMAJ ? rb * L + cb : cb * L + rb;
-        Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = sum[j][v];
+        Cl[(size_t)blk * blk_elems + ri * p.CI + ci] = unscale * sum[j][v];
       }
       if (++ri == p.RI) { ri = 0; ++rb; }
     }

@@ -195,7 +195,7 @@ __device__ __forceinline__ void load_octets(float (&o)[N][8], int K, int k0, int
   }
 }
 
-// a block again with the float32 instruction (see s2cnn::sum_holds)
+// a block again with the float32 instruction (see s2cnn::finite)
 template <class FA, class FB> __device__ __forceinline__ s2cnn::v16f block_float32(int K, int h, FA fa, FB fb) {
   s2cnn::v16f acc;
 #pragma unroll
@@ -241,24 +241,23 @@ __device__ __forceinline__ void split_product(int K, int wave, int lane, FA fa, 
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    float sum[PER];
-    bool holds = true;
+    float sum[PER], unscale = s2cnn::UNSCALE;
 #pragma unroll
     for (int v = 0; v < PER; ++v) {
       const int r = PER * wave + v;
       sum[v] = part[0][j][r][lane];
 #pragma unroll
       for (int w = 1; w < NW; ++w) sum[v] += part[w][j][r][lane];
-      holds = holds && s2cnn::sum_holds(sum[v]);
     }
-    if (!__all(holds)) {
+    if (!__all(s2cnn::finite(sum))) {
       const s2cnn::v16f again = block_float32(K, h, fa, [&](int k) { return fb(k, j); });
 #pragma unroll
       for (int v = 0; v < 16; ++v)
         if (v / PER == wave) sum[v % PER] = again[v];
+      unscale = 1.f;
     }
 #pragma unroll
-    for (int v = 0; v < PER; ++v) store(PER * wave + v, j, sum[v]);
+    for (int v = 0; v < PER; ++v) store(PER * wave + v, j, unscale * sum[v]);
   }
 }
 
@@ -394,17 +393,16 @@ __global__ __launch_bounds__(256) void planes_kernel(const float* __restrict__ x
     for (int q = 0; q < STEPS; ++q) s2cnn::split_mma_one(tile[cur].get(r32, 2 * q + h), frb[q], acc);
     if (row0 + 32 < last) tile[cur ^ 1].put(trow, toct, a);        // last read in the round before, which every wave has left
     if (row0 + 64 < last) load(row0 + 64);
-    bool holds = true;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) holds = holds && s2cnn::sum_holds(acc[v]);
-    if (!__all(holds)) {
+    float unscale = s2cnn::UNSCALE;
+    if (!__all(s2cnn::finite(acc))) {
       const bool rok = row0 + r32 < R;
       acc = block_float32(P, h, [&](int k) { return rok ? Ei[(size_t)k * R + row0 + r32] : 0.f; }, [&](int k) { return s(k); });
+      unscale = 1.f;
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int r = row0 + 8 * (v / 4) + 4 * h + v % 4;
-      if (s.ok && r < R) o[(size_t)r * ld] = acc[v];
+      if (s.ok && r < R) o[(size_t)r * ld] = unscale * acc[v];
     }
     __syncthreads();
   }

@@ -19,30 +19,41 @@ __device__ __forceinline__ unsigned pack_bf16(float x, float y) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{x, y}, v2bf));
 }
 
-// the three parts of two values, each a packed pair
-__device__ __forceinline__ void split_pair(float x, float y, unsigned& h, unsigned& m, unsigned& l) {
-  h = pack_bf16(x, y);
-  const float xr = x - __uint_as_float(h << 16), yr = y - __uint_as_float(h & 0xffff0000u);
+// Values are cut times SCALE.  Every float32 value, subnormal ones included, is a multiple of 2^-149, so that its parts are multiples of
+// 2^-125: none is subnormal in bf16, and every cut of a finite value below 2^104 is exact.  Sums of products of cut values come
+// out times SCALE^2: UNSCALE takes that off (exactly, but for results that are subnormal and rounded once more).
+// (Unscaled, parts below 2^-133 are lost: relative errors of products of values around 2^-118 and 1: 9e-6, 2^-124: 5e-4, 2^-140: 1.)
+constexpr float SCALE = 0x1p24f, UNSCALE = 0x1p-48f;
+
+// the three parts of two values (SCALED: that are times SCALE already), each a packed pair
+template <bool SCALED = false> __device__ __forceinline__ void split_pair(float x, float y, unsigned& h, unsigned& m, unsigned& l) {
+  const float xs = SCALED ? x : x * SCALE, ys = SCALED ? y : y * SCALE;
+  h = pack_bf16(xs, ys);
+  const float xr = xs - __uint_as_float(h << 16), yr = ys - __uint_as_float(h & 0xffff0000u);
   m = pack_bf16(xr, yr);
   l = pack_bf16(xr - __uint_as_float(m << 16), yr - __uint_as_float(m & 0xffff0000u));
 }
 
 struct SplitFragment { v8bf h, m, l; };
 
-// Whether a sum of part products is what a float32 product gives.  It is not where it is not finite (the parts of an infinity,
-// and of a value that rounds to one in bf16, are not its sum), and where operands are so small that their low parts are
-// subnormal in bf16, which the matrix cores take as zero: below 2^-108 (relative errors of the products at 2^-112: 1.3 times
-// those at 1, at 2^-116: 13 times).  The line at 2^-70 takes in such values beside partners of up to 2^38.
-__device__ __forceinline__ bool sum_holds(float v) {
-  const float a = fabsf(v);
-  return a == 0.f || (a >= 0x1p-70f && a <= 3.402823466e38f);
+// Whether all of these sums are finite.  If not they may be none of a float32 product: the parts of an infinity, and of a value that
+// rounds to one in bf16, are not its sum, and scaled sums leave the range of float32 from 2^80 on.
+template <int N> __device__ __forceinline__ bool finite(const float (&v)[N]) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) t = fmaf(v[i], 0.f, t);
+  return t == 0.f;
+}
+__device__ __forceinline__ bool finite(v16f v) {
+  struct Row { float f[16]; };
+  return finite(__builtin_bit_cast(Row, v).f);
 }
 
-__device__ __forceinline__ void split_octet(const float (&x)[8], uint4& h, uint4& m, uint4& l) {
-  split_pair(x[0], x[1], h.x, m.x, l.x);
-  split_pair(x[2], x[3], h.y, m.y, l.y);
-  split_pair(x[4], x[5], h.z, m.z, l.z);
-  split_pair(x[6], x[7], h.w, m.w, l.w);
+template <bool SCALED = false> __device__ __forceinline__ void split_octet(const float (&x)[8], uint4& h, uint4& m, uint4& l) {
+  split_pair<SCALED>(x[0], x[1], h.x, m.x, l.x);
+  split_pair<SCALED>(x[2], x[3], h.y, m.y, l.y);
+  split_pair<SCALED>(x[4], x[5], h.z, m.z, l.z);
+  split_pair<SCALED>(x[6], x[7], h.w, m.w, l.w);
 }
 __device__ __forceinline__ SplitFragment split_octet(const float (&x)[8]) {
   uint4 h, m, l;
@@ -60,9 +71,9 @@ template <int EXT, int TK> struct SplitTile {
 
   static __device__ __forceinline__ int slot(int row) { return row ^ ((row >> 3) & 1); }
 
-  __device__ __forceinline__ void put(int row, int octet, const float (&x)[8]) {
+  template <bool SCALED = false> __device__ __forceinline__ void put(int row, int octet, const float (&x)[8]) {
     uint4 h, m, l;
-    split_octet(x, h, m, l);
+    split_octet<SCALED>(x, h, m, l);
     const int s = slot(row);
     part[0][octet][s] = h;
     part[1][octet][s] = m;

@@ -79,6 +79,30 @@ def test_kernel_spectrum_of_values_without_bf16_parts(hip):
     assert err.max().item() <= 4 * bound(len(grid))          # per column, with a quarter of the chip's columns as room
 
 
+@pytest.mark.parametrize("ex", [-118, -128, -140])
+def test_kernel_spectrum_gradients_of_tiny_values(hip, ex):
+    """Incoming gradients that are subnormal or next to it, brought back by the factor: the accuracy of ordinary ones."""
+    import s2cnn_amd
+    from s2cnn_amd import wigner
+    from s2cnn_amd.s2_real import _setup_s2_ft_real
+    from s2cnn_amd import s2_real, so3_real
+    b, scale = 10, 2.0 ** 100
+    for mod, grid in ((so3_real, s2cnn_amd.so3_near_identity_grid()), (s2_real, s2cnn_amd.s2_near_identity_grid())):
+        F = (torch.from_numpy(wigner.so3_ft_matrix_real(b, grid)) if mod is so3_real else _setup_s2_ft_real(b, grid, torch.device("cpu")).double()) * scale
+        k = torch.randn(3, 20, len(grid), device="cuda").requires_grad_()
+        y = mod.scaled_kernel_spectrum(k, scale, b, grid)
+        gy = (torch.randn(y.shape, generator=torch.Generator().manual_seed(1)).double() * 2.0 ** ex).float()
+        (gk,) = torch.autograd.grad(y, k, gy.cuda())
+        flat = gy.double().reshape(F.size(1), -1).t()
+        want = (flat @ F.t()).reshape(k.shape)
+        # before the factor a gradient is rounded to float32, as a subnormal here: half of 2^-149.  So are the gradients of SO(3) plane
+        # coefficients: b sums of a degree each and two of the change of basis, for each of the 2 b (2b - 1) coefficients that a sample's sum
+        # takes, times up to 1
+        slack = scale * 2.0 ** -150 * k.numel() ** 0.5 * (1 + ((b + 2) * 2 * b * (2 * b - 1) if mod is so3_real else 0))
+        size = ((flat ** 2) @ (F.t() ** 2)).sum().sqrt()
+        assert (gk.double().cpu() - want).norm().item() <= bound(F.size(1)) * size.item() + slack
+
+
 def chain(A, B, order):
     """A [M, K] B [K, N] in float32 as one chain of fused multiply-adds per entry (exact products; sums rounded to float64 on the way,
     which is another result once in 2^29 times)."""

@@ -187,6 +187,34 @@ def test_product_of_tiny_values_and_large_partners(hip, nl, B, Fi, Fo, complex_)
     assert ((got.double() - want).norm() / want.norm()).item() <= 4 * bound((2 * nl - 1) * Fi)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(3, 5, 9, 7), (16, 8, 40, 40)])      # either kernel
+@pytest.mark.parametrize("complex_", [False, True])
+@pytest.mark.parametrize("ex,ey", [(-118, 60), (-126, 60), (-140, 60), (-140, 100), (-60, -60), (30, 45), (105, -60)])
+def test_products_over_the_exponents_of_float32(hip, nl, B, Fi, Fo, complex_, ex, ey):
+    """Operands that are subnormal or next to it beside partners of any size, tiny products, scaled sums outside the range of float32:
+    in both directions the errors of float32 products, one rounding per step."""
+    import s2cnn_amd
+    ns, pair = O.nspec_so3(nl), (2,) if complex_ else ()
+    print(f"exponents nl={nl} B={B} Fi={Fi} Fo={Fo} complex={complex_} 2^{ex} 2^{ey}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    x, gz = ((torch.randn(ns, B, f, *pair, device="cuda", generator=g).double() * 2.0 ** ex).float() for f in (Fi, Fo))
+    y = (torch.randn(ns, Fi, Fo, *pair, device="cuda", generator=g).double() * 2.0 ** ey).float()
+    exact = product64_complex if complex_ else product64
+    xg, yg = x.requires_grad_(), y.requires_grad_()
+    z = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(xg, yg)
+    (gx,) = torch.autograd.grad(z, xg, gz)
+    L = 2 * nl - 1
+    for got, want, K in ((z.detach(), exact("fwd", x.detach(), y.detach(), nl), L * Fi), (gx, exact("gradx", gz, y.detach(), nl), L * Fo)):
+        assert ((got.double() - want).norm() / want.norm()).item() <= 4 * bound(K)
+    if ex < -100:      # grad y is a product of two operands of x's size: one of them as it is, the other of the size of y
+        big = (torch.randn(ns, B, Fi, *pair, device="cuda", generator=g).double() * 2.0 ** ey).float().requires_grad_()
+        zb = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(big, yg)
+        (gy,) = torch.autograd.grad(zb, yg, gz)
+        want = exact("grady", gz, big.detach(), nl)
+        assert ((gy.double() - want).norm() / want.norm()).item() <= 4 * bound(L * B)
+
+
 def chain(A, B, order):
     """A [M, K] B [K, N] in float32 as one chain of fused multiply-adds per entry (exact products; sums rounded to float64 on the way,
     which is another result once in 2^29 times)."""
