@@ -427,7 +427,8 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
     else S2CNN_SLICES(1, 1);
     return s2cnn::launch_status();
   }
-  if (!near) S2CNN_LAUNCH(1, FAR, 1);
+  if (!near && pairs && KI % 4 == 0) S2CNN_LAUNCH(2, FAR, 4);
+  else if (!near) S2CNN_LAUNCH(1, FAR, 1);
   else if (divides) S2CNN_LAUNCH(2, DIVIDES, 8);
   else if (pairs && KI % 4 == 0) S2CNN_LAUNCH(2, WALK, 4);
   else if (pairs) S2CNN_LAUNCH(2, WALK, 2);

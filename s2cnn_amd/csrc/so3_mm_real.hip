@@ -454,7 +454,8 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
   const int wa = width(C_::A_KC ? KI : RI, a), wb = width(C_::B_KC ? KI : CI, b);
   const bool a2 = wa >= 2, b2 = wb >= 2;
   const bool near = Lmax * Lmax * RI * KI < (1L << 29) && Lmax * Lmax * CI * KI < (1L << 29);   // 32-bit byte offsets below OUTSIDE
-  const bool divides = near && (C_::A_KC ? wa == 4 : a2) && (C_::B_KC ? wb == 4 : b2) && KI % 8 == 0 && (KI % TK == 0 || TK % KI == 0);
+  const bool wide = (C_::A_KC ? wa == 4 : a2) && (C_::B_KC ? wb == 4 : b2);
+  const bool divides = near && wide && KI % 8 == 0 && (KI % TK == 0 || TK % KI == 0);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const long tiles64 = total_slots(nl, RI, CI, TM, 64);
   if (MODE == FWD && near && tiles64 > 0 && tiles64 < SLICES_GRID && wa == 4 && Lmax * KI <= CHAIN_STEPS) {
@@ -484,7 +485,9 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
     if (narrow) hipLaunchKernelGGL((so3_block_mm_real_kernel<MODE, VA, (C_::B_KC ? VB : 1), HOW, GR, 1>), dim3(grid), dim3(NT), 0, st, p); \
     else hipLaunchKernelGGL((so3_block_mm_real_kernel<MODE, VA, VB, HOW, GR, 2>), dim3(grid), dim3(NT), 0, st, p);                        \
   } while (0)
-  if (!near) S2CNN_LAUNCH(1, 1, FAR, 1);
+  if (!near && wide && KI % 4 == 0) S2CNN_LAUNCH((C_::A_KC ? 4 : 2), (C_::B_KC ? 4 : 2), FAR, 4);
+  else if (!near && a2 && b2 && KI % 2 == 0) S2CNN_LAUNCH(2, 2, FAR, 2);
+  else if (!near) S2CNN_LAUNCH(1, 1, FAR, 1);
   else if (divides) S2CNN_LAUNCH((C_::A_KC ? 4 : 2), (C_::B_KC ? 4 : 2), DIVIDES, 8);
   else if constexpr (MODE == FWD) {
     if (wa == 4) { if (b2) S2CNN_LAUNCH(4, 2, WALK, 4); else S2CNN_LAUNCH(4, 1, WALK, 4); }

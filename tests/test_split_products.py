@@ -215,6 +215,38 @@ def test_products_over_the_exponents_of_float32(hip, nl, B, Fi, Fo, complex_, ex
         assert ((gy.double() - want).norm() / want.norm()).item() <= 4 * bound(L * B)
 
 
+# Operands beyond 32-bit byte offsets: 49 blocks of 2^24 floats at the top degree, 25 of complex numbers.  Loads of four, two
+# and one, for x, y and gz the large operand.
+@pytest.mark.gpu
+@pytest.mark.parametrize("complex_,nl", [(False, 4), (True, 3)])
+@pytest.mark.parametrize("B,Fi,Fo", [(3, 4096, 4096), (2, 4095, 4097), (2, 4094, 4098), (4096, 4096, 8), (4097, 4095, 3), (4096, 8, 4096), (4094, 6, 4097), (4094, 6, 4098)])
+def test_products_of_operands_beyond_32_bit_offsets(hip, complex_, nl, B, Fi, Fo):
+    import s2cnn_amd
+    print(f"far product complex={complex_} nl={nl} B={B} Fi={Fi} Fo={Fo}", flush=True)
+    ns, pair = O.nspec_so3(nl), (2,) if complex_ else ()
+    g = torch.Generator(device="cuda").manual_seed(B)
+    x, y, gz = (torch.randn(ns, *s, *pair, device="cuda", generator=g) for s in ((B, Fi), (Fi, Fo), (B, Fo)))
+    z = (s2cnn_amd.so3_mm if complex_ else s2cnn_amd.so3_mm_real)(x.requires_grad_(), y.requires_grad_())
+    gx, gy = torch.autograd.grad(z, (x, y), gz)
+    l = nl - 1
+    L, first = 2 * l + 1, O.nspec_so3(l)
+
+    def matrix(t, columns_first):      # the top degree in float64, [(spectral row, feature row), (spectral column, feature column)] or transposed blocks
+        t = t.detach()[first:].reshape(L, L, *t.shape[1:])
+        t = torch.complex(t[..., 0].double(), t[..., 1].double()) if complex_ else t.double()
+        return t.permute(1, 2, 0, 3).reshape(L * t.shape[2], -1) if columns_first else t.transpose(1, 2).reshape(L * t.shape[2], -1)
+
+    def check(got, A, Bm, K):
+        want = A @ Bm
+        assert ((got - want).norm() / want.norm()).item() <= (2 if complex_ else 1) * bound(K)
+
+    conj = (lambda t: t.conj()) if complex_ else (lambda t: t)
+    X, Y, GZ = matrix(x, False), matrix(y, True), matrix(gz, False)      # Z = X Y^*, GX = GZ Y^T, GY: its blocks (column, row) X^T GZ^*
+    check(matrix(z, False), X, conj(Y), L * Fi)
+    check(matrix(gx, False), GZ, Y.t(), L * Fo)
+    check(matrix(gy, True), X.t(), conj(GZ), L * B)
+
+
 def chain(A, B, order):
     """A [M, K] B [K, N] in float32 as one chain of fused multiply-adds per entry (exact products; sums rounded to float64 on the way,
     which is another result once in 2^29 times)."""
