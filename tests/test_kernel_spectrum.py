@@ -174,3 +174,30 @@ def test_s2_analysis_in_the_real_basis(hip, b_in, b_out, batch):
     g = torch.randn_like(want)
     gw, gg = (torch.autograd.grad(y, x, g)[0] for y in (want, got))
     assert ((gg - gw).norm() / gw.norm()).item() <= 2.0 ** -22
+
+
+@pytest.mark.parametrize("ncols", [4, 36, 1028])
+def test_expansions_alone(hip, ncols):
+    """The expansion over the degrees and its adjoint as entry points of their own, behind and in front of the products that s2cnn_so3_rft and its
+    adjoint run: the same bits; the complex one against its change of basis."""
+    import s2cnn_amd
+    from s2cnn_amd import _hip, so3_real
+    b, grid = 5, s2cnn_amd.so3_near_identity_grid()
+    idx, E, Et, dtab = so3_real._setup_so3_rft_plan(b, grid, torch.device("cuda", torch.cuda.current_device()))
+    (nbeta, P), R, npts, ns = idx.shape, E.size(2), len(grid), O.nspec_so3(b)
+    P_, st = _hip.ptr, _hip.stream_ptr()
+    g = torch.Generator(device="cuda").manual_seed(ncols)
+    x, gy = torch.randn(ncols, npts, device="cuda", generator=g), torch.randn(ns, ncols, device="cuda", generator=g)
+    G, gG = torch.empty(nbeta, R, ncols, device="cuda"), torch.empty(nbeta, R, ncols, device="cuda")
+    y, yc, gx = torch.empty(ns, ncols, device="cuda"), torch.empty(ns, ncols, 2, device="cuda"), torch.empty(ncols, npts, device="cuda")
+    _hip.call("s2cnn_rft_planes", P_(x), P_(idx), P_(E), P_(G), nbeta, P, R, npts, ncols, ncols, 0.5, st)
+    _hip.call("s2cnn_so3_rft_expand_real", P_(G), P_(dtab), P_(y), b, nbeta, ncols, st)
+    _hip.call("s2cnn_so3_rft_expand", P_(G), P_(dtab), P_(yc), b, nbeta, ncols, st)
+    _hip.call("s2cnn_so3_rft_expand_real_grad", P_(gy), P_(dtab), P_(gG), b, nbeta, ncols, st)
+    _hip.call("s2cnn_rft_planes_grad", P_(gG), P_(idx), P_(Et), P_(gx), nbeta, P, R, npts, ncols, ncols, 0.5, st)
+    xg = x.clone().requires_grad_()
+    want = so3_real._KernelSpectrum.apply(xg, b, (idx, E, Et, dtab), 0.5)
+    (wgx,) = torch.autograd.grad(want, xg, gy)
+    assert torch.equal(y, want) and torch.equal(gx, wgx)
+    back = so3_real.so3_spectrum_to_real(yc)      # sums of two products with 1/sqrt2 or sqrt2: a few roundings
+    assert ((back - y).norm() / y.norm()).item() <= 2.0 ** -22
