@@ -160,11 +160,11 @@ __device__ __forceinline__ void contract(LD& ld, Smem& s, v16f (&acc)[NB][NB], i
 // One workgroup per CU (149 KB), tiles listed in bands and dealt to the XCDs in runs as in so3_mm_real.hip.
 //
 // Measured (us, fwd / gradx / grady; before: v_mfma_f32_32x32x2_f32 in tiles of 128 x 64, at 77 % of its peak):
-//   32 degrees, batch 16,  64 ->  64:  6849 / 6839 / 6553 -> 4312 / 4240 / 4294, 1.15 PFLOP/s of bf16 instructions, the rate that
+//   32 degrees, batch 16,  64 ->  64:  6849 / 6839 / 6553 -> 4449 / 4453 / 4527, 1.1 PFLOP/s of bf16 instructions, the rate that
 //                                      the real product reaches as well (energy: the clock falls with the power drawn)
-//   22 degrees, batch 32, 100 -> 100:  8190 / 8365 / 7246 -> 4670 / 4719 / 4592
-//   16 degrees, batch 16,  64 ->  64:   539 /  588 /  465 ->  366 /  363 /  300
-//   24 degrees, batch  4,  30 ->  30:   277 /  267 /  503 ->  154 /  153 /  127
+//   22 degrees, batch 32, 100 -> 100:  8190 / 8365 / 7246 -> 4888 / 4880 / 4889
+//   16 degrees, batch 16,  64 ->  64:   539 /  588 /  465 ->  367 /  371 /  307
+//   24 degrees, batch  4,  30 ->  30:   277 /  267 /  503 ->  148 /  150 /  123
 // Errors against 64 bits (relative 2-norm) at the first size 1.56e-6 / 1.56e-6 / 7.8e-7 -> 1.33e-6 / 1.33e-6 / 6.6e-7, smaller at all
 // sizes measured.
 template <int MODE, int VA, int VB, int HOW, int GA, int GB>
@@ -279,7 +279,7 @@ __device__ __forceinline__ s2cnn::v8bf negated(s2cnn::v8bf v) {
 // cutting of operands that each wave has to itself, so the four products of the direct form take the place of three with
 // sums that would have to be cut as well (and the errors halve).
 // us of fwd / gradx / grady, float32 kernel before -> tiles of 128 x 128 -> this one: 6 degrees, batch 32, 20 -> 40: 49 / 66 / 49 -> 30 / 48 / 40
-// -> 12 / 12 / 11; 13 degrees, batch 11, 33 -> 45: 178 / 151 / 109 -> 96 / 134 / 65 -> 70 / 91 / 72.  The line, in 32 x 32 tiles: 1 792 (32
+// -> 12 / 12 / 11; 13 degrees, batch 11, 33 -> 45: 178 / 151 / 109 -> 96 / 134 / 65 -> 72 / 86 / 62.  The line, in 32 x 32 tiles: 1 792 (32
 // degrees, batch 1, 32 -> 32) 190 us in tiles of 128, 144 here; 2 460 (24 degrees, batch 4, 30 -> 30) 154 and 165; 2 720 24.7 and 26;
 // 3 174 59 and 69; 4 148 equal; 5 712 366 and 466.
 template <int MODE, int VA, int VB, int HOW, int GR>

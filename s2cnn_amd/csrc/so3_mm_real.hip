@@ -16,7 +16,7 @@
 //
 // Arithmetic: every operand value is cut into three bf16 parts and six of the nine part products are summed in float32
 // (split_bf16.h).  At nl = 32, batch 16, 64 -> 64 features a product took 2.25 .. 2.35 ms with v_mfma_f32_32x32x2_f32 (77 % of
-// the float32 matrix peak) and takes 1.40 / 1.43 / 1.50 ms now (gradx, fwd, grady): 1.15 PFLOP/s of bf16 instructions, the
+// the float32 matrix peak) and takes 1.42 / 1.46 / 1.51 ms now (gradx, fwd, grady): 1.1 PFLOP/s of bf16 instructions, the
 // rate that a large library product in bf16 reaches on this card (its clock falls with the power the matrix cores draw), so
 // what bounds it is energy.  Errors against 64 bits fall as well (relative 2-norm 1.02e-6 -> 8.9e-7 at that size, 3.5e-7 ->
 // 2.9e-7 at 6 degrees): the products are exact and six roundings take the place of sixteen.
