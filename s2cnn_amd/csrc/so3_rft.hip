@@ -24,6 +24,7 @@ namespace {
 
 constexpr float SQRT2 = 1.41421356237309504880f, RSQRT2 = 0.70710678118654752440f;
 constexpr int NBMAX = 4;
+constexpr unsigned OUTSIDE = 0x80000000u;   // a byte offset behind the end of every buffer: such loads return 0
 
 __device__ __forceinline__ int lmn_index(int l, int m, int n) { return l * (4 * l * l - 1) / 3 + (l + m) * (2 * l + 1) + (l + n); }
 __device__ __forceinline__ float4 fma4(float s, float4 v, float4 acc) {
@@ -408,6 +409,91 @@ __global__ __launch_bounds__(256) void planes_kernel(const float* __restrict__ x
   }
 }
 
+// More points and enough outputs: 128 rows x 128 columns per workgroup, in stages of 32 points.  E is cut once per stage, two octets per thread,
+// on its way to LDS; the samples go there as they are, fetched along the points (a wave's load covers two columns; a lane per column
+// would touch a line with every value), and each wave cuts those of its 32 columns.  The next stage is in flight meanwhile.
+constexpr int TILE_BLOCKS = 4, TILE_STEPS = 32;
+__global__ __launch_bounds__(256, 2) void planes_tile_kernel(const float* __restrict__ x, const int* __restrict__ idx, const float* __restrict__ E,
+                                                             float* __restrict__ out, int P, int R, int npts, long ncols, long ld, float scale) {
+  constexpr int ROWS = 32 * TILE_BLOCKS, COLS = 128, PITCH = TILE_STEPS + 4, NX = COLS / 8;
+  static_assert(ROWS * TILE_STEPS == 256 * 16 && TILE_STEPS == 32, "two octets of E per thread, a wave over two columns");
+  __shared__ s2cnn::SplitTile<ROWS, TILE_STEPS> tile;
+  __shared__ __attribute__((aligned(16))) float samples[COLS][PITCH];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r32 = lane & 31, h = lane >> 5;
+  const int trow = threadIdx.x % ROWS, toct = threadIdx.x / ROWS, row0 = blockIdx.y * ROWS;
+  const int tpoint = threadIdx.x % TILE_STEPS, tcol = threadIdx.x / TILE_STEPS;
+  const long col0 = (long)blockIdx.x * COLS;
+  const float* Ei = E + (size_t)blockIdx.z * P * R;
+  const int* group = idx ? idx + (size_t)blockIdx.z * P : nullptr;
+  // loads behind the end of a buffer are zeros, so that nothing has to be done to a value before it is used
+  const long rest = ncols - col0 < COLS ? ncols - col0 : COLS;
+  const __amdgpu_buffer_rsrc_t re = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Ei), 0, 4 * P * R, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x + col0 * npts), 0, (int)(4 * rest * npts), 0x00020000);
+  const unsigned eo = row0 + trow < R ? 4u * (unsigned)(8 * toct * R + row0 + trow) : OUTSIDE, xo = 4u * (unsigned)(tcol * npts);
+  float a[2][8], xs[NX];
+  const auto load = [&](int k0, int place) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int n = 0; n < 8; ++n)
+        a[o][n] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(re, (int)(eo + 4u * (unsigned)((k0 + 16 * o + n) * R)), 0, 0));
+    const int q = k0 + tpoint < P ? (group ? place : k0 + tpoint) : -1;
+    const unsigned at = (unsigned)q < (unsigned)npts ? xo + 4u * (unsigned)q : OUTSIDE;
+#pragma unroll
+    for (int n = 0; n < NX; ++n) xs[n] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, (int)(at + 32u * (unsigned)(n * npts)), 0, 0));
+  };
+  const auto place = [&](int k0) { return group && k0 + tpoint < P ? group[k0 + tpoint] : 0; };
+  s2cnn::v16f acc[TILE_BLOCKS][1];
+#pragma unroll
+  for (int i = 0; i < TILE_BLOCKS; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i][0][v] = 0.f;
+  load(0, place(0));
+  int next = place(TILE_STEPS);
+  for (int k0 = 0; k0 < P; k0 += TILE_STEPS) {
+#pragma unroll
+    for (int o = 0; o < 2; ++o) tile.put(trow, toct + 2 * o, a[o]);
+#pragma unroll
+    for (int n = 0; n < NX; ++n) samples[tcol + 8 * n][tpoint] = scale * xs[n];
+    if (k0 + TILE_STEPS < P) {
+      load(k0 + TILE_STEPS, next);
+      next = place(k0 + 2 * TILE_STEPS);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < TILE_STEPS / 16; ++s) {
+      s2cnn::SplitFragment fa[TILE_BLOCKS], fb[1];
+      const float4* o = reinterpret_cast<const float4*>(&samples[32 * wave + r32][16 * s + 8 * h]);
+      const float4 u = o[0], w = o[1];
+      const float octet[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+      fb[0] = s2cnn::split_octet(octet);
+#pragma unroll
+      for (int i = 0; i < TILE_BLOCKS; ++i) fa[i] = tile.get(32 * i + r32, 2 * s + h);
+      s2cnn::split_mma<TILE_BLOCKS, 1>(fa, fb, acc);
+    }
+    __syncthreads();
+  }
+  const long col = col0 + 32 * wave + r32;
+  const Samples all(x, idx, blockIdx.z, P, npts, col, ncols, scale);
+  float* o = out + (size_t)blockIdx.z * R * ld + col;
+#pragma unroll
+  for (int i = 0; i < TILE_BLOCKS; ++i) {
+    const int first = row0 + 32 * i;
+    s2cnn::v16f z = acc[i][0];
+    float unscale = s2cnn::UNSCALE;
+    if (!__all(s2cnn::finite(z))) {
+      const bool ok = first + r32 < R;
+      z = block_float32(P, h, [&](int k) { return ok ? Ei[(size_t)k * R + first + r32] : 0.f; }, [&](int k) { return all(k); });
+      unscale = 1.f;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int r = first + 8 * (v / 4) + 4 * h + v % 4;
+      if (all.ok && r < R) o[(size_t)r * ld] = unscale * z[v];
+    }
+  }
+}
+
 // rows: columns c of g, columns: points; 32 columns and 64 points per workgroup of NW waves.  The transposed matrix makes both operands
 // coalesced; g is read once for up to 64 points.  At the size above 100 us (118 with four waves; 229 in blocks of 32 points with the
 // matrix as it lies).
@@ -451,9 +537,14 @@ int check_planes(const void* a, const void* E, const void* o, int nbeta, int P, 
 // (2 432) 7.9 -> 6.0; three times 64 points, 132 rows, 800 columns (1 350) 9.2 -> 11.2; 380 rows, 400 columns (1 800) 10.7 -> 12.9; 650 rows,
 // 1 485 columns (11 439) 31 -> 48.
 constexpr long CHAIN_LOADS = 96 * 1024;      // 16 x 16 tiles times points
+// More of either: tiles of 128 x 128 from TILE_GRID of them on.  us split -> tiles: 128 points, 1 024 rows, 800 columns (56 tiles) 11.5 -> 12.7, 1 200
+// columns (80) 14.0 -> 12.8; 100 points, 992 rows, 1 485 columns (96) 12.9 -> 13.5; three times 64 points, 380 rows, 1 485 columns (108) 14.2 -> 9.6;
+// 256 points, 400 rows, 1 200 columns (40) 12.5 -> 19.9, 1 024 rows, 4 096 columns (256) 72 -> 24; 128 points, 4 032 rows, 4 096 columns (1 024) 143
+// -> 41; three times 256 points, 1 560 rows, 2 048 columns (624) 170 -> 48.
+constexpr long TILE_GRID = 100;
 int planes(const float* x, const int* idx, const float* E, float* out, int nbeta, int P, int R, int npts, long ncols, long ld, float scale, hipStream_t st) {
   const dim3 wide((unsigned)((ncols + 127) / 128), (R + ROW_BLOCKS * 32 - 1) / (ROW_BLOCKS * 32), nbeta), narrow((unsigned)((ncols + 31) / 32), (R + 31) / 32, nbeta),
-      chain((unsigned)((ncols + 15) / 16), (R + 63) / 64, nbeta);
+      chain((unsigned)((ncols + 15) / 16), (R + 63) / 64, nbeta), tiles((unsigned)((ncols + 127) / 128), (R + 32 * TILE_BLOCKS - 1) / (32 * TILE_BLOCKS), nbeta);
   const bool chains = P <= 16 * STEPS && (long)chain.x * ((R + 15) / 16) * nbeta * P <= CHAIN_LOADS;
   if (P <= 16 * STEPS && (long)wide.x * wide.y * wide.z >= WALK_GRID)
     hipLaunchKernelGGL(planes_kernel, wide, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
@@ -461,6 +552,8 @@ int planes(const float* x, const int* idx, const float* E, float* out, int nbeta
     hipLaunchKernelGGL(planes_chain_kernel<true>, chain, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
   else if (chains)
     hipLaunchKernelGGL(planes_chain_kernel<false>, chain, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
+  else if ((long)tiles.x * tiles.y * tiles.z >= TILE_GRID && (P + 2L * TILE_STEPS) * R < (1L << 29) && npts < (1 << 22))      // 32-bit offsets below OUTSIDE
+    hipLaunchKernelGGL(planes_tile_kernel, tiles, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
   else
     hipLaunchKernelGGL(planes_split_kernel, narrow, dim3(256), 0, st, x, idx, E, out, P, R, npts, ncols, ld, scale);
   return s2cnn::launch_status();

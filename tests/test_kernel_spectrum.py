@@ -147,6 +147,30 @@ def test_so3_kernel_spectra_of_small_layers_are_chains(hip, b, shape):
     assert torch.equal(scaled_kernel_spectrum(k, 0.37, b, grid).reshape(want.shape), want)
 
 
+@pytest.mark.parametrize("b,shape,points", [(13, (33, 45), 64), (20, (32, 40), 128), (7, (64, 320), 130)])
+def test_tiled_kernel_spectrum_of_values_without_bf16_parts(hip, b, shape, points):
+    """The same in tiles of 128 x 128: three betas of 64 points, one of 128, and a spectrum of the sphere."""
+    import s2cnn_amd
+    from s2cnn_amd import s2_real, so3_real, wigner
+    n = shape[0] * shape[1]
+    print(f"tiled kernel spectrum b={b} columns={n} points={points}", flush=True)
+    if points == 130:
+        mod, grid = s2_real, s2cnn_amd.s2_equatorial_grid(max_beta=0, n_alpha=130, n_beta=1)
+        F = s2_real._setup_s2_ft_real(b, grid, torch.device("cpu")).double()
+    else:
+        mod = so3_real
+        grid = s2cnn_amd.so3_near_identity_grid() if points == 64 else s2cnn_amd.so3_equatorial_grid(max_beta=0, max_gamma=0, n_alpha=128, n_beta=1, n_gamma=1)
+        F = torch.from_numpy(wigner.so3_ft_matrix_real(b, grid))
+    k = torch.randn(n, len(grid), generator=torch.Generator().manual_seed(0))
+    k[0, 7], k[130, 3], k[257, 60], k[n - 1, 1] = float("inf"), float("nan"), 3.4e38 * 0.9999, 2.0 ** 105
+    y = mod.scaled_kernel_spectrum(k.cuda().view(*shape, -1), 0.0625, b, grid).cpu().reshape(-1, n)
+    finite = torch.isfinite(y).all(0)
+    assert finite.sum() == n - 2 and not finite[0] and not finite[130]
+    want = F.t() @ k.double()[finite].t() * 0.0625
+    err = (y[:, finite].double() - want).norm(dim=0) / want.norm(dim=0)
+    assert err.max().item() <= 4 * bound(len(grid))          # per column, with a quarter of the chip's columns as room
+
+
 def test_kernel_spectrum_gradient_of_the_gradient(hip):
     """The transform is linear: the gradient of a function of its gradient is the transform again."""
     import s2cnn_amd
