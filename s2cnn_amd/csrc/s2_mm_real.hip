@@ -17,7 +17,7 @@
 
 namespace {
 
-constexpr int KC = 8;       // input features per register pass
+constexpr int KC = 8;       // input features per register pass (grad y: two loads of four)
 constexpr int NSPLIT = 8;   // forward: workgroups along n per (l, r)
 constexpr int IPT = 2;      // forward: batch items per thread
 constexpr int IB = 4;       // grad x: batch items per workgroup
@@ -157,47 +157,87 @@ __global__ __launch_bounds__(256) void s2_mm_real_gradx_kernel(const float* __re
 }
 
 // ---- grad y.  grid.x = nl^2 (l, s), grid.y = tile of JT j groups, grid.z = feature pass.  The threads form
-// SL = 256 / JT slices of JT lanes; slice q takes the (r, i) pairs q, q + SL, ...; a lane accumulates KC pieces (x is
-// uniform over a slice), then the slices are reduced through LDS.
-template <int VEC, int JT>
+// SL = 256 / JT slices of JT lanes; slice q takes the (r, i) pairs q, q + SL, ...: where one tile holds all j groups, the slices read
+// gz[l,r,s] row after row without gaps.  A lane accumulates KC pieces in two sums each, four pairs in flight; the values of x come
+// through LDS, PAIRS pairs at a time; the slices are reduced through LDS.
+// What bounds it is the stream of gz.  us before -> now (a slice's values of x from memory, KC loads beside one of gz, and 16, 32 or 64 lanes
+// a slice whatever F_out): 32 degrees, batch 32, 6 -> 100: 266 -> 188, 3.0 TB/s; 32 degrees, batch 16, 6 -> 50: 96 -> 62; 20 degrees, batch 9,
+// 3 -> 26: 19 -> 11; 16 degrees, batch 20, 3 -> 45: 61 -> 17; 10 degrees, batch 32, 1 -> 20: 13 -> 12.  Errors against 64 bits fall (1.9e-7 ->
+// 1.7e-7 at the first size): shorter chains.
+template <int VEC>
 __global__ __launch_bounds__(256) void s2_mm_real_grady_kernel(const float* __restrict__ gz, const float* __restrict__ x,
-                                                               float* __restrict__ gy, int nl, int nbatch, int fi, int fo) {
+                                                               float* __restrict__ gy, int nl, int nbatch, int fi, int fo, int jt) {
   typedef typename Pack<VEC>::type vec_t;
-  constexpr int SL = 256 / JT;
-  __shared__ float part[SL][KC][JT * VEC];
+  constexpr int PAIRS = 256, AHEAD = 4;
+  __shared__ __attribute__((aligned(16))) float part[256 * KC * VEC];      // [slice][u][jt * VEC]
+  __shared__ __attribute__((aligned(16))) float xs[PAIRS][KC];
   const int ls = blockIdx.x, k0 = blockIdx.z * KC;
   const int l = isqrt_floor(ls), sn = ls - l * l - l;
   const int L = 2 * l + 1;
   const size_t zcol = (size_t)l * (4 * l * l - 1) / 3 + (size_t)(l + sn);
-  const int fov = fo / VEC;
-  const int slice = threadIdx.x / JT, jl = threadIdx.x - slice * JT;
-  const int jv = blockIdx.y * JT + jl;
-  vec_t acc[KC];
+  const int fov = fo / VEC, nslice = 256 / jt;
+  const int slice = threadIdx.x / jt, jl = threadIdx.x - slice * jt;
+  const int jv = blockIdx.y * jt + jl;
+  const bool active = slice < nslice && jv < fov;
+  vec_t acc[2][KC];
 #pragma unroll
-  for (int u = 0; u < KC; ++u) acc[u] = Pack<VEC>::zero();
+  for (int u = 0; u < KC; ++u) acc[0][u] = acc[1][u] = Pack<VEC>::zero();
   const int total = L * nbatch;                                    // (r, i) pairs
-  int rr = slice / nbatch, i = slice - rr * nbatch;                // walks the pairs with stride SL
-  const int dr = SL / nbatch, di = SL - dr * nbatch;
-  for (int p = slice; p < total; p += SL) {
-    const vec_t a = jv < fov ? reinterpret_cast<const vec_t*>(gz + ((zcol + (size_t)rr * L) * nbatch + i) * fo)[jv] : Pack<VEC>::zero();
-    const float* xx = x + ((size_t)(l * l + rr) * nbatch + i) * fi + k0;
+  const int dr = nslice / nbatch, di = nslice - dr * nbatch;
+  for (int c0 = 0; c0 < total; c0 += PAIRS) {
+    const int n = total - c0 < PAIRS ? total - c0 : PAIRS;
+    if (c0) __syncthreads();
+    for (int e = threadIdx.x; e < n * KC; e += 256) {
+      const int p = e / KC, u = e - p * KC;
+      xs[p][u] = k0 + u < fi ? x[((size_t)l * l * nbatch + c0 + p) * fi + k0 + u] : 0.f;
+    }
+    __syncthreads();
+    if (!active) continue;
+    int rr = (c0 + slice) / nbatch, i = c0 + slice - rr * nbatch;  // walks the pairs with stride nslice
+    for (int p = slice; p < n; p += AHEAD * nslice) {
+      vec_t a[AHEAD];
 #pragma unroll
-    for (int u = 0; u < KC; ++u)
-      if (k0 + u < fi) Pack<VEC>::fma(xx[u], a, acc[u]);
-    rr += dr; i += di;
-    if (i >= nbatch) { i -= nbatch; ++rr; }
+      for (int q = 0; q < AHEAD; ++q) {
+        if (p + q * nslice < n) a[q] = reinterpret_cast<const vec_t*>(gz + ((zcol + (size_t)rr * L) * nbatch + i) * fo)[jv];
+        rr += dr; i += di;
+        if (i >= nbatch) { i -= nbatch; ++rr; }
+      }
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q)
+        if (p + q * nslice < n) {
+          const float4 lo = *reinterpret_cast<const float4*>(&xs[p + q * nslice][0]), hi = *reinterpret_cast<const float4*>(&xs[p + q * nslice][4]);
+          const float xx[KC] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+          for (int u = 0; u < KC; ++u)
+            if (k0 + u < fi) Pack<VEC>::fma(xx[u], a[q], acc[q & 1][u]);
+        }
+    }
   }
+  if (slice < nslice) {
 #pragma unroll
-  for (int u = 0; u < KC; ++u) reinterpret_cast<vec_t*>(&part[slice][u][0])[jl] = acc[u];
+    for (int u = 0; u < KC; ++u) {
+      Pack<VEC>::fma(1.f, acc[1][u], acc[0][u]);
+      reinterpret_cast<vec_t*>(part + ((size_t)slice * KC + u) * jt * VEC)[jl] = acc[0][u];
+    }
+  }
   __syncthreads();
-  for (int o = threadIdx.x; o < KC * JT * VEC; o += 256) {
-    const int u = o / (JT * VEC), jj = o - u * (JT * VEC);
-    const int j = blockIdx.y * JT * VEC + jj;
+  const int row = jt * VEC;
+  for (int o = threadIdx.x; o < KC * row; o += 256) {
+    const int u = o / row, jj = o - u * row;
+    const int j = blockIdx.y * row + jj;
     if (k0 + u < fi && j < fo) {
-      float v = 0.f;
+      float v[16];                 // sixteen short sums, then their tree
 #pragma unroll
-      for (int q = 0; q < SL; ++q) v += part[q][u][jj];
-      gy[((size_t)ls * fi + k0 + u) * fo + j] = v;
+      for (int w = 0; w < 16; ++w) v[w] = 0.f;
+      for (int q = 0; q < nslice; q += 16)
+#pragma unroll
+        for (int w = 0; w < 16; ++w)
+          if (q + w < nslice) v[w] += part[((q + w) * KC + u) * row + jj];
+#pragma unroll
+      for (int h = 8; h > 0; h >>= 1)
+#pragma unroll
+        for (int w = 0; w < h; ++w) v[w] += v[w + h];
+      gy[((size_t)ls * fi + k0 + u) * fo + j] = v[0];
     }
   }
 }
@@ -256,15 +296,16 @@ extern "C" int s2cnn_s2_mm_real_grady(const float* gz, const float* x, float* gy
   s2cnn::clear_stale_error();
   if (int rc = check(gz, x, gy, nl, nbatch, f_in, f_out)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (vec4(gz, gz, gy, f_out)) {
-    const dim3 grid(nl * nl, (f_out / 4 + 15) / 16, (f_in + KC - 1) / KC);
-    hipLaunchKernelGGL((s2_mm_real_grady_kernel<4, 16>), grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out);
-  } else if (vec2(gz, gz, gy, f_out)) {
-    const dim3 grid(nl * nl, (f_out / 2 + 31) / 32, (f_in + KC - 1) / KC);
-    hipLaunchKernelGGL((s2_mm_real_grady_kernel<2, 32>), grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out);
-  } else {
-    const dim3 grid(nl * nl, (f_out + 63) / 64, (f_in + KC - 1) / KC);
-    hipLaunchKernelGGL((s2_mm_real_grady_kernel<1, 64>), grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out);
-  }
+  const int vec = vec4(gz, gz, gy, f_out) ? 4 : vec2(gz, gz, gy, f_out) ? 2 : 1;
+  // slices of up to 64 lanes, as even as they come, and of 16 where there would be fewer workgroups than four for each CU: 16 degrees, batch
+  // 32, 6 -> 100 with 256 workgroups 59 us, with 512 40 (before 47)
+  const int fov = f_out / vec;
+  int tiles = (fov + 63) / 64;
+  while (nl * nl * tiles < 1024 && fov > 16 * tiles) tiles *= 2;
+  const int even = (fov + tiles - 1) / tiles, jt = even < 4 ? 4 : even;      // at most 64 slices: with 256 of one lane 13 degrees, batch 7, 8 -> 4 took 14 us (before 9)
+  const dim3 grid(nl * nl, (fov + jt - 1) / jt, (f_in + KC - 1) / KC);
+  if (vec == 4) hipLaunchKernelGGL(s2_mm_real_grady_kernel<4>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
+  else if (vec == 2) hipLaunchKernelGGL(s2_mm_real_grady_kernel<2>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
+  else hipLaunchKernelGGL(s2_mm_real_grady_kernel<1>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
   return s2cnn::launch_status();
 }
