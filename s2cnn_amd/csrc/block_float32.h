@@ -8,9 +8,9 @@
 namespace s2cnn {
 namespace block {
 
-// acc = the NI x NJ blocks of 32 x 32 outputs, RSTEP rows and CSTEP columns apart, of which this lane holds row row0 and column col0 of the first; A, B: the
+// acc = the NI x NJ blocks of 32 x 32 outputs, STEP apart, of which this lane holds row row0 and column col0 of the first; A, B: the
 // operands of the degree, L x L blocks of RI (CI) x KI elements; fa, fb: the float of an element that takes part.
-template <typename C_, int NI, int NJ, int RSTEP, int CSTEP, typename E, class FA, class FB>
+template <typename C_, int NI, int NJ, int STEP, typename E, class FA, class FB>
 __device__ __forceinline__ void contract_float32(const E* A, const E* B, int RI, int CI, int KI, v16f (&acc)[NI][NJ], int L, int row0, int col0, int h,
                                                  FA fa, FB fb) {
   const int K = L * KI;
@@ -19,13 +19,13 @@ __device__ __forceinline__ void contract_float32(const E* A, const E* B, int RI,
   const size_t ablk = (size_t)RI * KI, bblk = (size_t)CI * KI;
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int row = row0 + RSTEP * i, rb = row / RI, ri = row - rb * RI;
+    const int row = row0 + STEP * i, rb = row / RI, ri = row - rb * RI;
     aok[i] = row < L * RI;
     ao[i] = (C_::A_MNMAJ ? (size_t)rb * L : (size_t)rb) * ablk + (size_t)ri * (C_::A_KC ? KI : 1);
   }
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    const int col = col0 + CSTEP * j, cb = col / CI, ci = col - cb * CI;
+    const int col = col0 + STEP * j, cb = col / CI, ci = col - cb * CI;
     bok[j] = col < L * CI;
     bo[j] = (C_::B_MNMAJ ? (size_t)cb * L : (size_t)cb) * bblk + (size_t)ci * (C_::B_KC ? KI : 1);
   }

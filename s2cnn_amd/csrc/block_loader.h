@@ -25,48 +25,26 @@ template <> struct VecT<float, 2> { typedef float2 type; };
 template <> struct VecT<float, 4> { typedef float4 type; };
 template <> struct VecT<float2, 2> { typedef float4 type; };
 
-// N of 16 samples of a row, those of part, and the blocks they lie in: evenly apart, those of neighbouring rows in others.  0 for rows outside.
-template <bool KC, bool MNMAJ, int N, class E>
-__device__ __forceinline__ void sample_row(const E* base, int L, int MNI, int KI, int row, int part, E (&value)[N], int (&block)[N]) {
-  const bool inside = row < L * MNI;
-  const int mb = inside ? row / MNI : 0, mi = inside ? row - mb * MNI : 0;
-  const size_t blk = (size_t)MNI * KI, row_at = (MNMAJ ? (size_t)mb * L : (size_t)mb) * blk + (size_t)mi * (KC ? KI : 1);
-  const int step_b = L < 16 ? 1 : L / 16, step_k = 7 % KI;
-  int kb = (row + part * N * step_b) % L, kin = (row * 5 + part * N * step_k) % KI;
-#pragma unroll
-  for (int s = 0; s < N; ++s) {
-    value[s] = inside ? base[row_at + (size_t)kb * (MNMAJ ? 1 : L) * blk + (size_t)kin * (KC ? 1 : MNI)] : E{};
-    block[s] = kb;
-    kb += step_b;
-    kin += step_k;
-    if (kb >= L) kb -= L;
-    if (kin >= KI) kin -= KI;
-  }
-}
-
-// One operand's loader.  A thread owns NMN rows (K-contiguous: ROWSTEP apart; MN-contiguous: neighbours)
-// of NK contraction steps, starting at step k0 and ADV further on with every load(): an octet of a row is what a lane feeds to
-// the matrix instruction, and what one 16-byte LDS store takes, whichever index is the fast one in memory.  The steps are
-// consecutive, or (JUMP) four of them and four JUMP further on: then four threads with the granules of a row side by side read 64 bytes of it
-// with one instruction.  VEC = elements per global access, along the contraction (K-contiguous) or along the rows
-// (MN-contiguous).  Rows outside the matrix and steps behind the last block are loaded from OUTSIDE, that is as zeros.
-template <typename E, bool KC, bool MNMAJ, int NMN, int ROWSTEP, int VEC, int HOW, int GR, int ADV, int NK = 8, int JUMP = 0>
+// One operand's loader.  A thread owns NMN rows (ROWSTEP apart) of 8 contraction steps, starting at step k0 and ADV further on with
+// every load(): an octet of a row is what a lane feeds to the matrix instruction, and what one 16-byte LDS store takes,
+// whichever index is the fast one in memory.  VEC = elements per global access, along the contraction (K-contiguous) or along
+// the rows (MN-contiguous).  Rows outside the matrix and steps behind the last block are loaded from OUTSIDE, that is as
+// zeros.
+template <typename E, bool KC, bool MNMAJ, int NMN, int ROWSTEP, int VEC, int HOW, int GR, int ADV>
 struct Loader {
   static constexpr unsigned ES = sizeof(E);
   static_assert(NMN >= 1 && (KC || VEC == 1 || (VEC <= NMN && ROWSTEP == 1)), "no such loader");
-  static constexpr int HALF = JUMP ? 4 : NK, NP = NK / HALF;      // consecutive steps, and how many runs of them
-  static_assert(HOW == DIVIDES || GR <= HALF, "granules lie in a run");
   typedef typename VecT<E, VEC>::type vec_t;
 
-  E reg[NMN][NK];
+  E reg[NMN][8];
   const E* base;
   __amdgpu_buffer_rsrc_t rsrc;
   unsigned off[NMN];            // offset of the row (DIVIDES: and of the octet): bytes, FAR: elements; OUTSIDE for no row
   int MNI, KI, L, blk_k_stride;
-  int kb[NP], kin[NP], adv_b, adv_k;    // WALK, FAR: block and feature of the first step of a run; what a stage adds to them
+  int kb, kin, adv_b, adv_k;    // WALK, FAR: block and feature of this thread's first step; what a stage adds to them
   unsigned soff, step_in, step_cross;   // DIVIDES: uniform byte offset of the stage and its increments
-  unsigned jump;                        // DIVIDES: bytes from the first run to the second
-  int sub, nsub, stage_i, stages[NP];   // the stage, and how many there are with steps of this thread's runs in them
+  int sub, nsub, stage_i, last_ragged;
+  bool tail_ok;
 
   __device__ __forceinline__ void init(const E* base_l, int L_, int MNI_, int KI_, int row0, int k0) {
     base = base_l; MNI = MNI_; KI = KI_; L = L_;
@@ -75,27 +53,23 @@ struct Loader {
     blk_k_stride = (MNMAJ ? 1 : L) * blk_elems;
     const int unit = KC ? 1 : MNI;                       // stride of one contraction step inside a block
     rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<E*>(base_l), 0, HOW == FAR ? 0 : (int)ES * L * L * MNI * KI, 0x00020000);
-#pragma unroll
-    for (int r = 0; r < NP; ++r) {
-      kb[r] = (k0 + r * JUMP) / KI;
-      kin[r] = k0 + r * JUMP - kb[r] * KI;
-    }
+    kb = k0 / KI;
+    kin = k0 - kb * KI;
     const int K = L * KI, nstage = (K + ADV - 1) / ADV, ktail = K - (nstage - 1) * ADV;
 #pragma unroll
     for (int q = 0; q < NMN; ++q) {
       const int row = row0 + q * ROWSTEP;
       const int mb = row / MNI, mi = row - mb * MNI;
       unsigned o = (unsigned)(mb * blk_mn_stride + mi * (KC ? KI : 1));
-      if (HOW == DIVIDES) o += (unsigned)((KI >= ADV ? 0 : kb[0]) * blk_k_stride + kin[0] * unit);
+      if (HOW == DIVIDES) o += (unsigned)((KI >= ADV ? 0 : kb) * blk_k_stride + kin * unit);
       off[q] = row >= L * MNI ? OUTSIDE : HOW == FAR ? o : ES * o;
     }
     if (HOW == DIVIDES) {
       soff = 0; sub = 0; stage_i = 0;
       if (KI >= ADV) { nsub = KI / ADV; step_in = ES * ADV * unit; step_cross = ES * (unsigned)(blk_k_stride - (KI - ADV) * unit); }
       else { nsub = 1; step_in = 0; step_cross = ES * (unsigned)(ADV / KI * blk_k_stride); }
-      jump = ES * (unsigned)(KI >= ADV ? JUMP * unit : JUMP / KI * blk_k_stride);
-#pragma unroll
-      for (int r = 0; r < NP; ++r) stages[r] = k0 + r * JUMP < ktail ? nstage : nstage - 1;
+      last_ragged = ktail < ADV ? nstage - 1 : -1;
+      tail_ok = k0 < ktail;
     } else {
       adv_b = ADV / KI;
       adv_k = ADV - adv_b * KI;
@@ -120,65 +94,58 @@ struct Loader {
   __device__ __forceinline__ void put(int q, int e, vec_t v) {
     if constexpr (VEC == 1) reg[q][e] = v;
     else if constexpr (sizeof(E) == 8) { reg[q][e] = make_float2(v.x, v.y); reg[KC ? q : q + 1][KC ? e + 1 : e] = make_float2(v.z, v.w); }
-    else if constexpr (VEC == 2) { reg[q][e] = v.x; reg[KC ? q : q + 1][KC ? e + 1 : e] = v.y; }
-    else if constexpr (KC) { reg[q][e] = v.x; reg[q][e + 1] = v.y; reg[q][e + 2] = v.z; reg[q][e + 3] = v.w; }
-    else { reg[q][e] = v.x; reg[q + 1][e] = v.y; reg[q + 2][e] = v.z; reg[q + 3][e] = v.w; }
+    else if constexpr (KC && VEC == 2) { reg[q][e] = v.x; reg[q][e + 1] = v.y; }
+    else if constexpr (KC && VEC == 4) { reg[q][e] = v.x; reg[q][e + 1] = v.y; reg[q][e + 2] = v.z; reg[q][e + 3] = v.w; }
+    else { reg[q][e] = v.x; reg[q + 1][e] = v.y; }
   }
 
   // fetches the current stage and steps to the next one
   __device__ __forceinline__ void load() {
     constexpr int QSTEP = KC ? 1 : VEC, ESTEP = KC ? VEC : 1;
-    if constexpr (HOW == DIVIDES) {
+    if (HOW == DIVIDES) {
+      const bool ok = stage_i != last_ragged || tail_ok;
 #pragma unroll
-      for (int r = 0; r < NP; ++r) {
-        const bool ok = stage_i < stages[r];
-        const unsigned so = r ? soff + jump : soff;
+      for (int q = 0; q < NMN; q += QSTEP) {
+        const unsigned o = ok ? off[q] : OUTSIDE;
 #pragma unroll
-        for (int q = 0; q < NMN; q += QSTEP) {
-          const unsigned o = ok ? off[q] : OUTSIDE;
-#pragma unroll
-          for (int e = 0; e < HALF; e += ESTEP)
-            put(q, r * HALF + e, KC ? fetch(o + ES * e, so) : fetch(o, so + ES * (unsigned)(e * MNI)));
-        }
+        for (int e = 0; e < 8; e += ESTEP)
+          put(q, e, KC ? fetch(o + ES * e, soff) : fetch(o, soff + ES * (unsigned)(e * MNI)));
       }
       ++stage_i;
       if (++sub == nsub) { sub = 0; soff += step_cross; }
       else soff += step_in;
-    } else {
-      const unsigned scale = HOW == FAR ? 1u : ES, unit = scale * (unsigned)(KC ? 1 : MNI), bstride = scale * (unsigned)blk_k_stride;
-      const unsigned cross = bstride - (unsigned)KI * unit;      // from behind the end of a block to the start of the next
-#pragma unroll
-      for (int r = 0; r < NP; ++r) {
-        int k = kin[r], b = kb[r];
-        unsigned o = (unsigned)b * bstride + (unsigned)k * unit;
-#pragma unroll
-        for (int g = 0; g < HALF; g += GR) {
-#pragma unroll
-          for (int q = 0; q < NMN; q += QSTEP) {
-            if constexpr (HOW == FAR) {
-              const bool in = b < L && off[q] != OUTSIDE;
-              const E* at = base + (in ? (size_t)off[q] + o : 0);
-#pragma unroll
-              for (int e = 0; e < GR; e += ESTEP) {
-                const vec_t v = *reinterpret_cast<const vec_t*>(in ? at + (size_t)e * unit : base);
-                put(q, r * HALF + g + e, in ? v : vec_t{});
-              }
-            } else {
-              const unsigned at = b < L ? off[q] + o : OUTSIDE;                                      // OUTSIDE + o is outside as well
-#pragma unroll
-              for (int e = 0; e < GR; e += ESTEP)
-                put(q, r * HALF + g + e, KC ? fetch(at + scale * e, 0) : fetch(at, e * unit));
-            }
-          }
-          k += GR;
-          o += (unsigned)GR * unit;
-          if (k >= KI) { k = 0; ++b; o += cross; }                // KI is a multiple of GR
-        }
-        kin[r] += adv_k;
-        kb[r] += adv_b;
-        if (kin[r] >= KI) { kin[r] -= KI; ++kb[r]; }
-      }
+      return;
     }
+    const unsigned scale = HOW == FAR ? 1u : ES, unit = scale * (unsigned)(KC ? 1 : MNI), bstride = scale * (unsigned)blk_k_stride;
+    const unsigned cross = bstride - (unsigned)KI * unit;      // from behind the end of a block to the start of the next
+    int k = kin, b = kb;
+    unsigned o = (unsigned)b * bstride + (unsigned)k * unit;
+#pragma unroll
+    for (int g = 0; g < 8; g += GR) {
+#pragma unroll
+      for (int q = 0; q < NMN; q += QSTEP) {
+        if constexpr (HOW == FAR) {
+          const bool in = b < L && off[q] != OUTSIDE;
+          const E* at = base + (in ? (size_t)off[q] + o : 0);
+#pragma unroll
+          for (int e = 0; e < GR; e += ESTEP) {
+            const vec_t v = *reinterpret_cast<const vec_t*>(in ? at + (size_t)e * unit : base);
+            put(q, g + e, in ? v : vec_t{});
+          }
+        } else {
+          const unsigned at = b < L ? off[q] + o : OUTSIDE;                                      // OUTSIDE + o is outside as well
+#pragma unroll
+          for (int e = 0; e < GR; e += ESTEP)
+            put(q, g + e, KC ? fetch(at + scale * e, 0) : fetch(at, e * unit));
+        }
+      }
+      k += GR;
+      o += (unsigned)GR * unit;
+      if (k >= KI) { k = 0; ++b; o += cross; }                // KI is a multiple of GR
+    }
+    kin += adv_k;
+    kb += adv_b;
+    if (kin >= KI) { kin -= KI; ++kb; }
   }
 };
 

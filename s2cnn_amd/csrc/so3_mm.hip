@@ -235,7 +235,7 @@ __global__ __launch_bounds__(NT, 3) void so3_block_mm_kernel(MmParams p) {
     for (int j = 0; j < NB; ++j) finite = finite && s2cnn::finite(acc[i][j]);
   float unscale = s2cnn::UNSCALE;
   if (!__all(finite)) {
-    contract_float32<C_, NB, NB, BSTR, BSTR>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h,
+    contract_float32<C_, NB, NB, BSTR>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h,
                                        [&](float2 v) { return part_of(v, group); }, [&](float2 v) { return part_of(conj_of<C_::CONJ>(v), group); });
     unscale = 1.f;
   }
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(NTS) void so3_block_mm_slices_kernel(MmParams p) {
   if (!__all(s2cnn::finite(part_sums))) {
     v16f p1[1][1], p2[1][1], p3[1][1];
     const auto contract_kind = [&](int kind, v16f (&acc)[1][1]) {
-      contract_float32<C_, 1, 1, 32, 32>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + r32, tile_n + r32, h, [&](float2 v) { return part_of(v, kind); },
+      contract_float32<C_, 1, 1, 32>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + r32, tile_n + r32, h, [&](float2 v) { return part_of(v, kind); },
                                      [&](float2 v) { return part_of(conj_of<C_::CONJ>(v), kind); });
     };
     contract_kind(RE, p1);

@@ -1,5 +1,5 @@
 // Block-diagonal REAL products over the (2l+1)x(2l+1) blocks of an SO(3) spectrum held in the real
-// basis (see so3_real_basis.hip), on the f16 and bf16 matrix cores of gfx950 with float32 operands and results.
+// basis (see so3_real_basis.hip), on the bf16 matrix cores of gfx950 with float32 operands and results.
 //
 // The spectrum of a real signal on SO(3) obeys x[l,-m,-n] = (-1)^(m-n) conj(x[l,m,n]); a fixed unitary
 // change of basis per degree turns every such block into a real matrix, and the complex product
@@ -14,7 +14,7 @@
 // blocks in which either the contraction index ("K-contiguous") or the free index ("MN-contiguous") is
 // the fast one.
 //
-// Arithmetic of forward products with long contractions: two f16 parts (so3_mm_real_half.h).  Of the others: every operand value is cut into three bf16 parts and six of the nine part products are summed in float32
+// Arithmetic: every operand value is cut into three bf16 parts and six of the nine part products are summed in float32
 // (split_bf16.h).  At nl = 32, batch 16, 64 -> 64 features a product took 2.25 .. 2.35 ms with v_mfma_f32_32x32x2_f32 (77 % of
 // the float32 matrix peak) and takes 1.42 / 1.46 / 1.51 ms now (gradx, fwd, grady): 1.1 PFLOP/s of bf16 instructions, the
 // rate that a large library product in bf16 reaches on this card (its clock falls with the power the matrix cores draw), so
@@ -31,18 +31,14 @@
 // Tried and not kept: three workgroups per CU (168 registers): 0 to 2 % slower.
 #include "common.h"
 #include "split_bf16.h"
-#include "split_f16.h"
 #include "block_loader.h"
 #include "block_float32.h"
-#include <type_traits>
 
 namespace {
 
 using namespace s2cnn::block;
 using s2cnn::v16f;
 using s2cnn::SplitTile;
-using s2cnn::HalfTile;
-using s2cnn::RowScales;
 
 constexpr int NRB = 2;            // 32-row blocks per wave
 constexpr int TM = 64 * NRB;
@@ -197,7 +193,7 @@ __global__ __launch_bounds__(NT, 2) void so3_block_mm_real_kernel(MmParams p) {
   const auto same = [](float v) { return v; };
   float unscale = s2cnn::UNSCALE;
   if (!__all(finite)) {
-    contract_float32<C_, NRB, NCB, BSTR, BSTR>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h, same, same);
+    contract_float32<C_, NRB, NCB, BSTR>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + wrow + r32, tile_n + wcol + r32, h, same, same);
     unscale = 1.f;
   }
 
@@ -227,8 +223,6 @@ __global__ __launch_bounds__(NT, 2) void so3_block_mm_real_kernel(MmParams p) {
     }
   }
 }
-
-#include "so3_mm_real_half.h"
 
 // Small problems: too few 128 x 64 tiles to fill the chip, so that what counts is how many loads are in flight and how few
 // steps follow one another.  A workgroup owns 32 x (32 NJ) outputs and its four waves take every
@@ -311,7 +305,7 @@ __global__ __launch_bounds__(NT) void so3_block_mm_real_slices_kernel(MmParams p
   float unscale = s2cnn::UNSCALE;
   if (!__all(finite)) {
     const auto same = [](float v) { return v; };
-    contract_float32<C_, 1, NJ, 32, 32>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + r32, tile_n + r32, h, same, same);
+    contract_float32<C_, 1, NJ, 32>(A, B, p.RI, p.CI, p.KI, acc, L, tile_m + r32, tile_n + r32, h, same, same);
     unscale = 1.f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
@@ -484,13 +478,6 @@ int run(const float* a, const float* b, float* c, int nl, int RI, int CI, int KI
     else S2CNN_SLICES(1, 1);
 #undef S2CNN_SLICES
     return s2cnn::launch_status();
-  }
-  if constexpr (MODE == FWD) {
-    if (near && !narrow && wa == 4 && wb == 4 && Lmax * KI >= HALF_STEPS && Lmax * KI <= HALF_MOST && Lmax <= HALF_BLOCKS) {
-      if (divides) hipLaunchKernelGGL((so3_block_mm_real_half_kernel<MODE, 4, 4, DIVIDES, 8>), dim3(grid), dim3(NT), 0, st, p);
-      else hipLaunchKernelGGL((so3_block_mm_real_half_kernel<MODE, 4, 4, WALK, 4>), dim3(grid), dim3(NT), 0, st, p);
-      return s2cnn::launch_status();
-    }
   }
   // a 64-column tile of an MN-contiguous operand has one column per thread
 #define S2CNN_LAUNCH(VA, VB, HOW, GR)                                                                                                    \

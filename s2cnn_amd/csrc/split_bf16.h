@@ -62,14 +62,14 @@ __device__ __forceinline__ SplitFragment split_octet(const float (&x)[8]) {
 }
 
 // The parts of EXT rows x TK contraction steps in LDS: per part and octet of steps one 16-byte slot per row.  A lane's operand
-// of the matrix instruction is one slot.  Two slots of padding per octet and an order of the slots that changes with every eight
-// rows keep the stores (four octets of neighbouring rows, or every second or fourth row of one octet) and the loads (neighbouring
-// rows of one octet) of eight lanes in different banks; with two octets (TK = 16: four rows of both) four.
+// of the matrix instruction is one slot.  Two slots of padding per octet and the exchange of neighbouring slots in every
+// other group of eight rows keep the stores (four octets of neighbouring rows, or every other row of one octet) and the
+// loads (neighbouring rows of one octet) of eight lanes in different banks; with two octets (TK = 16: four rows of both) four.
 template <int EXT, int TK> struct SplitTile {
   static constexpr int LD = EXT + (TK == 16 ? 4 : 2);
   uint4 part[3][TK / 8][LD];
 
-  static __device__ __forceinline__ int slot(int row) { return row ^ ((row >> 3) & 3); }
+  static __device__ __forceinline__ int slot(int row) { return row ^ ((row >> 3) & 1); }
 
   template <bool SCALED = false> __device__ __forceinline__ void put(int row, int octet, const float (&x)[8]) {
     uint4 h, m, l;
@@ -78,17 +78,6 @@ template <int EXT, int TK> struct SplitTile {
     part[0][octet][s] = h;
     part[1][octet][s] = m;
     part[2][octet][s] = l;
-  }
-
-  // four values: half an octet
-  __device__ __forceinline__ void put_half(int row, int octet, int half, const float (&x)[4]) {
-    uint2 h, m, l;
-    split_pair(x[0], x[1], h.x, m.x, l.x);
-    split_pair(x[2], x[3], h.y, m.y, l.y);
-    const int s = slot(row);
-    reinterpret_cast<uint2*>(&part[0][octet][s])[half] = h;
-    reinterpret_cast<uint2*>(&part[1][octet][s])[half] = m;
-    reinterpret_cast<uint2*>(&part[2][octet][s])[half] = l;
   }
 
   __device__ __forceinline__ SplitFragment get(int row, int octet) const {
