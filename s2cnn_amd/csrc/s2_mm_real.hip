@@ -14,10 +14,11 @@
 // consecutive output features (16-byte accesses when F_out is a multiple of 4), the small operands come from L1/L2,
 // input features are taken KC at a time in registers.
 #include "common.h"
+#include "s2_mm_real_tiles.h"
 
 namespace {
 
-constexpr int KC = 8;       // input features per register pass (grad y: two loads of four)
+constexpr int KC = s2cnn::GRADY_KC;       // input features per register pass (grad y: two loads of four)
 constexpr int NSPLIT = 8;   // forward: workgroups along n per (l, r)
 constexpr int IPT = 2;      // forward: batch items per thread
 constexpr int IB = 4;       // grad x: batch items per workgroup
@@ -297,12 +298,7 @@ extern "C" int s2cnn_s2_mm_real_grady(const float* gz, const float* x, float* gy
   if (int rc = check(gz, x, gy, nl, nbatch, f_in, f_out)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int vec = vec4(gz, gz, gy, f_out) ? 4 : vec2(gz, gz, gy, f_out) ? 2 : 1;
-  // slices of up to 64 lanes, as even as they come, and of 16 where there would be fewer workgroups than four for each CU: 16 degrees, batch
-  // 32, 6 -> 100 with 256 workgroups 59 us, with 512 40 (before 47)
-  const int fov = f_out / vec;
-  int tiles = (fov + 63) / 64;
-  while (nl * nl * tiles < 1024 && fov > 16 * tiles) tiles *= 2;
-  const int even = (fov + tiles - 1) / tiles, jt = even < 4 ? 4 : even;      // at most 64 slices: with 256 of one lane 13 degrees, batch 7, 8 -> 4 took 14 us (before 9)
+  const int fov = f_out / vec, jt = s2cnn::grady_lanes(nl, f_in, fov);
   const dim3 grid(nl * nl, (fov + jt - 1) / jt, (f_in + KC - 1) / KC);
   if (vec == 4) hipLaunchKernelGGL(s2_mm_real_grady_kernel<4>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
   else if (vec == 2) hipLaunchKernelGGL(s2_mm_real_grady_kernel<2>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);

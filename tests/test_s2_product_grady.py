@@ -1,6 +1,40 @@
 """The kernel gradient of the product on the sphere in the real basis: slices of every width, full and ragged tiles and passes."""
+import ctypes
+import os
+import shutil
+import subprocess
+
 import pytest
 import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def split(tmp_path_factory):
+    """The rule of the launch, compiled for the host: lanes(nl, f_in, groups of features in a row)."""
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not found")
+    d = tmp_path_factory.mktemp("split")
+    (d / "split.cpp").write_text('#include "s2_mm_real_tiles.h"\n'
+                                 'extern "C" int lanes(int nl, int f_in, int fov) { return s2cnn::grady_lanes(nl, f_in, fov); }\n')
+    subprocess.run([gxx, "-shared", "-fPIC", "-I", os.path.join(ROOT, "s2cnn_amd", "csrc"), str(d / "split.cpp"), "-o", str(d / "split.so")], check=True)
+    return ctypes.CDLL(str(d / "split.so"))
+
+
+def test_rows_are_cut_only_where_workgroups_are_few(split):
+    for nl, Fi, fov, want in [(16, 6, 25, 13), (16, 25, 25, 25), (16, 32, 25, 25), (24, 32, 25, 25), (12, 64, 64, 64), (32, 6, 25, 25), (10, 1, 5, 5), (5, 8, 1, 4)]:
+        assert split.lanes(nl, Fi, fov) == want, (nl, Fi, fov)
+    for nl in range(1, 40):
+        for Fi in (1, 8, 9, 16, 17, 64):
+            passes = (Fi + 7) // 8
+            for fov in range(1, 400):
+                jt = split.lanes(nl, Fi, fov)
+                tiles = -(-fov // jt)
+                assert 4 <= jt <= 64
+                if tiles > -(-fov // 64):                       # cut further: too few workgroups with half the tiles, and no slice under 9 lanes
+                    assert nl * nl * passes * ((tiles + 1) // 2) < 1024 and jt >= 9
 
 
 @pytest.mark.gpu
