@@ -11,8 +11,8 @@
 //
 // x [nl^2, B, F_in], y [nl^2, F_in, F_out], z [nspec(nl), B, F_out]: half the bytes of the complex product, and all
 // three kernels are bound by streaming z / gz once (4 nspec B F_out bytes).  Lanes run along j in groups of VEC
-// consecutive output features (16-byte accesses when F_out is a multiple of 4), the small operands come from L1/L2,
-// input features are taken KC at a time in registers.
+// consecutive output features (16-byte accesses when F_out is a multiple of 4), the small operands come from L1/L2
+// (grad y: x through LDS), input features are taken KC at a time in registers.
 #include "common.h"
 #include "s2_mm_real_tiles.h"
 
@@ -157,89 +157,109 @@ __global__ __launch_bounds__(256) void s2_mm_real_gradx_kernel(const float* __re
   }
 }
 
-// ---- grad y.  grid.x = nl^2 (l, s), grid.y = tile of JT j groups, grid.z = feature pass.  The threads form
-// SL = 256 / JT slices of JT lanes; slice q takes the (r, i) pairs q, q + SL, ...: where one tile holds all j groups, the slices read
-// gz[l,r,s] row after row without gaps.  A lane accumulates KC pieces in two sums each, four pairs in flight; the values of x come
-// through LDS, PAIRS pairs at a time; the slices are reduced through LDS.
-// What bounds it is the stream of gz.  us before -> now (a slice's values of x from memory, KC loads beside one of gz, and 16, 32 or 64 lanes
-// a slice whatever F_out): 32 degrees, batch 32, 6 -> 100: 266 -> 188, 3.0 TB/s; 32 degrees, batch 16, 6 -> 50: 96 -> 62; 20 degrees, batch 9,
-// 3 -> 26: 19 -> 11; 16 degrees, batch 20, 3 -> 45: 61 -> 17; 10 degrees, batch 32, 1 -> 20: 13 -> 12.  Errors against 64 bits fall (1.9e-7 ->
-// 1.7e-7 at the first size): shorter chains.
+// ---- grad y.  grid.x = nl^2 (l, s), grid.y = tile of jt j groups, grid.z = feature pass.  The threads form nslice slices of jt lanes; slice
+// q takes the (r, i) pairs q, q + nslice, ...: where one tile holds all j groups, the slices read gz[l,r,s] row after row without gaps.  A
+// lane sums AHEAD pairs at a time for KC input features, their loads issued together; the values of x come through LDS, PAIRS pairs at a
+// time; the slices are reduced through LDS.
+// What bounds it: the stream of gz at large sizes, the chain from the loads to the stores where a slice has few pairs.  So the loads of gz stand
+// behind no branch (into registers that an earlier trip filled, each such load waits for all before it), those of x are all issued before the
+// first value is stored, pointers are stepped, and the divisors come from the host.
+// us: slices of 16, 32 or 64 lanes whatever F_out, x from memory -> slices as wide as the row, but a wait before each load -> now:
+//   32 degrees, batch 32, 6 -> 100: 266, 187, 118 (4.7 TB/s); 32 degrees, batch 16, 6 -> 50: 94, 61, 34; 16 degrees, batch 32, 32 -> 100: 121, 63, 40;
+//   20 degrees, batch 9, 3 -> 26: 19, 11, 7; 16 degrees, batch 20, 3 -> 45: 61, 17, 12; 10 degrees, batch 32, 1 -> 20: 14, 12, 9; few pairs:
+//   16 degrees, batch 1, 6 -> 100: 4.8, 6.2, 4.7; 18 degrees, batch 2, 7 -> 148: 7.2, 12.2, 5.9; 9 degrees, batch 1, 20 -> 193: 6.3, 11.2, 5.2.
+// Error against 64 bits at the first size 1.9e-7, 1.7e-7, 1.4e-7.  Two sums a lane that take every second pair instead of one that takes four at a
+// time: 106 us, and 1.7e-7.
 template <int VEC>
 __global__ __launch_bounds__(256) void s2_mm_real_grady_kernel(const float* __restrict__ gz, const float* __restrict__ x,
-                                                               float* __restrict__ gy, int nl, int nbatch, int fi, int fo, int jt) {
+                                                               float* __restrict__ gy, int nl, int nbatch, int fi, int fo, int jt,
+                                                               int nslice, int dr, int di, float rjt) {
   typedef typename Pack<VEC>::type vec_t;
   constexpr int PAIRS = 256, AHEAD = 4;
-  __shared__ __attribute__((aligned(16))) float part[256 * KC * VEC];      // [slice][u][jt * VEC]
+  __shared__ __attribute__((aligned(16))) float part[256 * KC * VEC];
   __shared__ __attribute__((aligned(16))) float xs[PAIRS][KC];
   const int ls = blockIdx.x, k0 = blockIdx.z * KC;
   const int l = isqrt_floor(ls), sn = ls - l * l - l;
   const int L = 2 * l + 1;
-  const size_t zcol = (size_t)l * (4 * l * l - 1) / 3 + (size_t)(l + sn);
-  const int fov = fo / VEC, nslice = 256 / jt;
-  const int slice = threadIdx.x / jt, jl = threadIdx.x - slice * jt;
+  const int fov = fo / VEC;
+  // threadIdx.x / jt; rjt = 1 / jt.  The half keeps the product 1 / 128 and more away from the next whole number, its error is below 2^-15
+  const int slice = (int)((threadIdx.x + 0.5f) * rjt), jl = threadIdx.x - slice * jt;
   const int jv = blockIdx.y * jt + jl;
   const bool active = slice < nslice && jv < fov;
-  vec_t acc[2][KC];
+  vec_t acc[KC];
 #pragma unroll
-  for (int u = 0; u < KC; ++u) acc[0][u] = acc[1][u] = Pack<VEC>::zero();
+  for (int u = 0; u < KC; ++u) acc[u] = Pack<VEC>::zero();
   const int total = L * nbatch;                                    // (r, i) pairs
-  const int dr = nslice / nbatch, di = nslice - dr * nbatch;
+  // nslice = dr * nbatch + di: the way from a pair of the slice to its next, and what is added where i starts again
+  const long row = (long)L * nbatch * fov, step = dr * row + (long)di * fov, wrap = row - (long)nbatch * fov;
+  const vec_t* column = reinterpret_cast<const vec_t*>(gz) + ((size_t)l * (4 * l * l - 1) / 3 + (size_t)(l + sn)) * nbatch * fov + jv;
+  const int u0 = threadIdx.x % KC, p0 = threadIdx.x / KC;          // this thread's values of x
   for (int c0 = 0; c0 < total; c0 += PAIRS) {
     const int n = total - c0 < PAIRS ? total - c0 : PAIRS;
+    const float* xp = x + ((size_t)l * l * nbatch + c0 + p0) * fi + k0 + u0;
+    float xv[KC];
+#pragma unroll
+    for (int w = 0; w < KC; ++w) xv[w] = p0 + w * (256 / KC) < n && k0 + u0 < fi ? xp[(size_t)w * (256 / KC) * fi] : 0.f;
     if (c0) __syncthreads();
-    for (int e = threadIdx.x; e < n * KC; e += 256) {
-      const int p = e / KC, u = e - p * KC;
-      xs[p][u] = k0 + u < fi ? x[((size_t)l * l * nbatch + c0 + p) * fi + k0 + u] : 0.f;
-    }
+#pragma unroll
+    for (int w = 0; w < KC; ++w) xs[p0 + w * (256 / KC)][u0] = xv[w];
     __syncthreads();
     if (!active) continue;
-    int rr = (c0 + slice) / nbatch, i = c0 + slice - rr * nbatch;  // walks the pairs with stride nslice
+    const int r0 = (c0 + slice) / nbatch;
+    int i = c0 + slice - r0 * nbatch;
+    const vec_t* g = column + r0 * row + (long)i * fov;
     for (int p = slice; p < n; p += AHEAD * nslice) {
+      const vec_t* first = g;
       vec_t a[AHEAD];
 #pragma unroll
       for (int q = 0; q < AHEAD; ++q) {
-        if (p + q * nslice < n) a[q] = reinterpret_cast<const vec_t*>(gz + ((zcol + (size_t)rr * L) * nbatch + i) * fo)[jv];
-        rr += dr; i += di;
-        if (i >= nbatch) { i -= nbatch; ++rr; }
+        a[q] = *(p + q * nslice < n ? g : first);                  // beyond the end the first pair again, which nobody adds
+        g += step; i += di;
+        if (i >= nbatch) { i -= nbatch; g += wrap; }
       }
+      vec_t t[KC];
+#pragma unroll
+      for (int u = 0; u < KC; ++u) t[u] = Pack<VEC>::zero();
 #pragma unroll
       for (int q = 0; q < AHEAD; ++q)
-        if (p + q * nslice < n) {
+        if (q == 0 || p + q * nslice < n) {
           const float4 lo = *reinterpret_cast<const float4*>(&xs[p + q * nslice][0]), hi = *reinterpret_cast<const float4*>(&xs[p + q * nslice][4]);
           const float xx[KC] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
-          for (int u = 0; u < KC; ++u)
-            if (k0 + u < fi) Pack<VEC>::fma(xx[u], a[q], acc[q & 1][u]);
+          for (int u = 0; u < KC; ++u) Pack<VEC>::fma(xx[u], a[q], t[u]);      // features beyond f_in end in sums that nobody reads
         }
+#pragma unroll
+      for (int u = 0; u < KC; ++u) Pack<VEC>::fma(1.f, t[u], acc[u]);
     }
   }
-  if (slice < nslice) {
+  const int used = total < nslice ? total : nslice;                // slices that had pairs
+  vec_t* sums = reinterpret_cast<vec_t*>(part);                    // [slice][u][jt]
+  if (slice < used) {
 #pragma unroll
-    for (int u = 0; u < KC; ++u) {
-      Pack<VEC>::fma(1.f, acc[1][u], acc[0][u]);
-      reinterpret_cast<vec_t*>(part + ((size_t)slice * KC + u) * jt * VEC)[jl] = acc[0][u];
-    }
+    for (int u = 0; u < KC; ++u) sums[(slice * KC + u) * jt + jl] = acc[u];
   }
   __syncthreads();
-  const int row = jt * VEC;
-  for (int o = threadIdx.x; o < KC * row; o += 256) {
-    const int u = o / row, jj = o - u * row;
-    const int j = blockIdx.y * row + jj;
-    if (k0 + u < fi && j < fo) {
-      float v[16];                 // sixteen short sums, then their tree
+  const int nu = fi - k0 < KC ? fi - k0 : KC;
+  for (int o = threadIdx.x; o < nu * jt; o += 256) {
+    const int u = (int)((o + 0.5f) * rjt), jo = blockIdx.y * jt + o - u * jt;
+    if (jo >= fov) continue;
+    vec_t v[16];                   // sixteen short sums, then their tree
 #pragma unroll
-      for (int w = 0; w < 16; ++w) v[w] = 0.f;
-      for (int q = 0; q < nslice; q += 16)
+    for (int w = 0; w < 16; ++w) v[w] = Pack<VEC>::zero();
+    for (int q = 0; q < used; q += 16)
 #pragma unroll
-        for (int w = 0; w < 16; ++w)
-          if (q + w < nslice) v[w] += part[((q + w) * KC + u) * row + jj];
+      for (int h = 0; h < 16; h += 4)
+        if (q + h < used)
 #pragma unroll
-      for (int h = 8; h > 0; h >>= 1)
+          for (int w = h; w < h + 4; ++w) {
+            const vec_t t = sums[(q + w < used ? q + w : q) * KC * jt + o];
+            Pack<VEC>::fma(1.f, q + w < used ? t : Pack<VEC>::zero(), v[w]);
+          }
 #pragma unroll
-        for (int w = 0; w < h; ++w) v[w] += v[w + h];
-      gy[((size_t)ls * fi + k0 + u) * fo + j] = v[0];
-    }
+    for (int h = 8; h > 0; h >>= 1)
+#pragma unroll
+      for (int w = 0; w < h; ++w) Pack<VEC>::fma(1.f, v[w + h], v[w]);
+    reinterpret_cast<vec_t*>(gy + ((size_t)ls * fi + k0 + u) * fo)[jo] = v[0];
   }
 }
 
@@ -298,10 +318,16 @@ extern "C" int s2cnn_s2_mm_real_grady(const float* gz, const float* x, float* gy
   if (int rc = check(gz, x, gy, nl, nbatch, f_in, f_out)) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int vec = vec4(gz, gz, gy, f_out) ? 4 : vec2(gz, gz, gy, f_out) ? 2 : 1;
-  const int fov = f_out / vec, jt = s2cnn::grady_lanes(nl, f_in, fov);
+  const int fov = f_out / vec;
+  const s2cnn::GradySplit split = s2cnn::grady_split(nl, nbatch, f_in, fov);
+  const int jt = split.lanes, nslice = split.slices, dr = nslice / nbatch, di = nslice % nbatch;
+  const float rjt = 1.f / jt;
   const dim3 grid(nl * nl, (fov + jt - 1) / jt, (f_in + KC - 1) / KC);
-  if (vec == 4) hipLaunchKernelGGL(s2_mm_real_grady_kernel<4>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
-  else if (vec == 2) hipLaunchKernelGGL(s2_mm_real_grady_kernel<2>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
-  else hipLaunchKernelGGL(s2_mm_real_grady_kernel<1>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt);
+  if (vec == 4)
+    hipLaunchKernelGGL(s2_mm_real_grady_kernel<4>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt, nslice, dr, di, rjt);
+  else if (vec == 2)
+    hipLaunchKernelGGL(s2_mm_real_grady_kernel<2>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt, nslice, dr, di, rjt);
+  else
+    hipLaunchKernelGGL(s2_mm_real_grady_kernel<1>, grid, dim3(256), 0, st, gz, x, gy, nl, nbatch, f_in, f_out, jt, nslice, dr, di, rjt);
   return s2cnn::launch_status();
 }

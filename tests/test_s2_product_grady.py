@@ -12,29 +12,36 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 @pytest.fixture(scope="module")
 def split(tmp_path_factory):
-    """The rule of the launch, compiled for the host: lanes(nl, f_in, groups of features in a row)."""
+    """The rule of the launch, compiled for the host: split(nl, batch, f_in, groups of features in a row) -> (lanes, slices)."""
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not found")
     d = tmp_path_factory.mktemp("split")
     (d / "split.cpp").write_text('#include "s2_mm_real_tiles.h"\n'
-                                 'extern "C" int lanes(int nl, int f_in, int fov) { return s2cnn::grady_lanes(nl, f_in, fov); }\n')
+                                 'extern "C" int lanes(int nl, int b, int f, int v) { return s2cnn::grady_split(nl, b, f, v).lanes; }\n'
+                                 'extern "C" int slices(int nl, int b, int f, int v) { return s2cnn::grady_split(nl, b, f, v).slices; }\n')
     subprocess.run([gxx, "-shared", "-fPIC", "-I", os.path.join(ROOT, "s2cnn_amd", "csrc"), str(d / "split.cpp"), "-o", str(d / "split.so")], check=True)
-    return ctypes.CDLL(str(d / "split.so"))
+    lib = ctypes.CDLL(str(d / "split.so"))
+    return lambda *size: (lib.lanes(*size), lib.slices(*size))
 
 
 def test_rows_are_cut_only_where_workgroups_are_few(split):
-    for nl, Fi, fov, want in [(16, 6, 25, 13), (16, 25, 25, 25), (16, 32, 25, 25), (24, 32, 25, 25), (12, 64, 64, 64), (32, 6, 25, 25), (10, 1, 5, 5), (5, 8, 1, 4)]:
-        assert split.lanes(nl, Fi, fov) == want, (nl, Fi, fov)
+    for nl, B, Fi, fov, want in [(16, 32, 6, 25, 13), (16, 32, 25, 25, 25), (16, 32, 32, 25, 25), (24, 16, 32, 25, 25), (12, 4, 64, 64, 64), (32, 32, 6, 25, 25),
+                                 (10, 32, 1, 5, 5), (5, 7, 8, 1, 4),
+                                 # few pairs for each slice
+                                 (18, 2, 7, 37, 19), (9, 1, 20, 193, 49), (16, 1, 6, 25, 25), (22, 2, 4, 23, 23)]:
+        assert split(nl, B, Fi, fov)[0] == want, (nl, B, Fi, fov)
     for nl in range(1, 40):
-        for Fi in (1, 8, 9, 16, 17, 64):
-            passes = (Fi + 7) // 8
-            for fov in range(1, 400):
-                jt = split.lanes(nl, Fi, fov)
-                tiles = -(-fov // jt)
-                assert 4 <= jt <= 64
-                if tiles > -(-fov // 64):                       # cut further: too few workgroups with half the tiles, and no slice under 9 lanes
-                    assert nl * nl * passes * ((tiles + 1) // 2) < 1024 and jt >= 9
+        for B in (1, 2, 9, 32, 1000):
+            for Fi in (1, 8, 9, 64):
+                passes, pairs = (Fi + 7) // 8, (2 * nl - 1) * B
+                for fov in range(1, 300):
+                    lanes, slices = split(nl, B, Fi, fov)
+                    tiles = -(-fov // lanes)
+                    assert 4 <= lanes <= 64 and 1 <= slices and lanes * slices <= 256
+                    assert slices == min(256 // lanes, -(-pairs // 4))              # four pairs for each
+                    if tiles > -(-fov // 64):             # cut further: too few workgroups with half the tiles, no slice under 9 lanes or five pairs
+                        assert nl * nl * passes * ((tiles + 1) // 2) < 1024 and lanes >= 9 and pairs // (256 // lanes) >= 5
 
 
 @pytest.mark.gpu
@@ -58,3 +65,29 @@ def test_kernel_gradient(hip, nl, B, Fi, Fo):
         got = gy[l * l:l * l + L].double()
         # sums of L B products, at most one rounding of 2^-24 each on partial sums that grow with the root of their number
         assert ((got - want).norm() / want.norm()).item() <= 2.0 ** -24 * (1 + (L * B) ** 0.5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo", [(5, 7, 9, 8), (6, 3, 3, 63), (4, 80, 1, 6), (3, 1, 17, 4)])
+def test_values_that_are_not_finite_stay_where_they_are(hip, nl, B, Fi, Fo):
+    """Pairs beyond a slice's end and features beyond the last pass are loaded or multiplied, and must reach no result."""
+    from s2cnn_amd.s2_real import s2_mm_real
+    print(f"s2 kernel gradient, infinities, nl={nl} B={B} Fi={Fi} Fo={Fo}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(nl)
+    x = torch.randn(nl * nl, B, Fi, device="cuda", generator=g)
+    y = torch.randn(nl * nl, Fi, Fo, device="cuda", generator=g).requires_grad_()
+    z = s2_mm_real(x, y)
+    gz = torch.randn(z.shape, device="cuda", generator=g)
+    for l in range(1, nl):                                       # one value in the first pair of a row, one in its last
+        L, first = 2 * l + 1, l * (4 * l * l - 1) // 3
+        gz[first, 0, 0] = float("inf")
+        gz[first + L * (L - 1) + 1, B - 1, Fo - 1] = float("nan")
+    (gy,) = torch.autograd.grad(z, y, gz)
+    for l in range(nl):
+        L, first = 2 * l + 1, l * (4 * l * l - 1) // 3
+        want = (gz[first:first + L * L].view(L, L, B, 1, Fo).double() * x[l * l:l * l + L].view(L, 1, B, Fi, 1).double()).sum((0, 2))
+        got = gy[l * l:l * l + L].double()
+        finite = want.isfinite()
+        assert torch.equal(got.isfinite(), finite) and torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isposinf(), want.isposinf())
+        err = (got - want)[finite].norm() / want[finite].norm()
+        assert err.item() <= 2.0 ** -24 * (1 + (L * B) ** 0.5)
