@@ -44,20 +44,50 @@ def test_rows_are_cut_only_where_workgroups_are_few(split):
                         assert nl * nl * passes * ((tiles + 1) // 2) < 1024 and lanes >= 9 and pairs // (256 // lanes) >= 5
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("nl,B,Fi,Fo", [
-    # one lane to sixty-four per slice and one more; loads of four, two and one
-    (3, 1, 1, 4), (5, 7, 8, 4), (7, 3, 9, 1), (6, 40, 6, 20), (9, 5, 6, 100), (8, 2, 3, 256), (8, 3, 2, 260), (5, 4, 7, 26), (6, 3, 8, 63), (4, 6, 17, 65),
+# (nl, B, Fi, Fo, elements by which gz starts beyond a boundary of 16 bytes)
+SIZES = [
+    # narrow slices, loads of four, two and one
+    (3, 1, 1, 4, 0), (5, 7, 8, 4, 0), (7, 3, 9, 1, 0), (6, 40, 6, 20, 0), (9, 5, 6, 100, 0), (8, 2, 3, 256, 0), (8, 3, 2, 260, 0), (5, 4, 7, 26, 0), (6, 3, 8, 63, 0), (4, 6, 17, 65, 0),
     # fewer pairs than slices, whole chunks of 256 pairs and one more, few and many workgroups
-    (1, 1, 6, 8), (1, 256, 6, 8), (1, 257, 6, 8), (16, 32, 6, 100), (32, 9, 6, 100), (16, 20, 3, 45)])
-def test_kernel_gradient(hip, nl, B, Fi, Fo):
+    (1, 1, 6, 8, 0), (1, 256, 6, 8, 0), (1, 257, 6, 8, 0), (16, 32, 6, 100, 0), (32, 9, 6, 100, 0), (16, 20, 3, 45, 0),
+    # wide slices: one tile of 49 to 64 lanes, two of 49 and of 33 with a ragged second, four of 64; the same through many passes
+    (32, 3, 3, 63, 0), (32, 2, 3, 64, 0), (32, 2, 3, 97, 0), (32, 2, 3, 256, 0), (32, 2, 3, 126, 0), (32, 2, 3, 196, 0), (32, 2, 3, 260, 0), (32, 1, 2, 1024, 0), (12, 9, 57, 57, 0),
+    # gz at a boundary of 8 and of 4 bytes with rows of whole groups of four
+    (5, 6, 7, 100, 2), (5, 6, 7, 100, 1), (32, 2, 3, 64, 2), (32, 2, 3, 64, 1), (6, 40, 9, 4, 3)]
+
+
+def vector_width(Fo, offset):
+    return 4 if Fo % 4 == 0 and offset % 4 == 0 else 2 if Fo % 2 == 0 and offset % 2 == 0 else 1
+
+
+def test_sizes_reach_the_splits_they_are_meant_for(split):
+    seen = {}
+    for nl, B, Fi, Fo, offset in SIZES:
+        vec = vector_width(Fo, offset)
+        lanes, slices = split(nl, B, Fi, Fo // vec)
+        seen.setdefault(vec, []).append((lanes, slices, -(-(Fo // vec) // lanes), (Fo // vec) % lanes, (2 * nl - 1) * B))
+    for vec in (1, 2, 4):
+        lanes = {s[0] for s in seen[vec]}
+        assert any(v == 4 for v in lanes) or vec == 2
+        assert any(9 <= v <= 16 for v in lanes) and any(v > 48 for v in lanes), (vec, lanes)
+        assert any(s[2] > 1 and s[3] for s in seen[vec]) or vec == 2                            # a ragged last tile
+    every = [s for v in seen.values() for s in v]
+    assert {4, 64} <= {s[0] for s in every} and any(17 <= s[0] <= 32 for s in every) and any(33 <= s[0] <= 48 for s in every)
+    assert {1, 4, 51, 64} <= {s[1] for s in every}                                              # slices
+    assert any(s[4] < 256 for s in every) and any(s[4] == 256 for s in every) and any(s[4] == 257 for s in every) and any(s[4] > 512 for s in every)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nl,B,Fi,Fo,offset", SIZES)
+def test_kernel_gradient(hip, nl, B, Fi, Fo, offset):
     from s2cnn_amd.s2_real import s2_mm_real
-    print(f"s2 kernel gradient nl={nl} B={B} Fi={Fi} Fo={Fo}", flush=True)
+    print(f"s2 kernel gradient nl={nl} B={B} Fi={Fi} Fo={Fo} offset={offset}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(nl)
     x = torch.randn(nl * nl, B, Fi, device="cuda", generator=g)
     y = torch.randn(nl * nl, Fi, Fo, device="cuda", generator=g).requires_grad_()
     z = s2_mm_real(x, y)
-    gz = torch.randn(z.shape, device="cuda", generator=g)
+    gz = torch.randn(z.numel() + offset, device="cuda", generator=g)[offset:].view(z.shape)
+    assert gz.is_contiguous() and gz.data_ptr() % 16 == 4 * offset
     (gy,) = torch.autograd.grad(z, y, gz)
     for l in range(nl):
         L, first = 2 * l + 1, l * (4 * l * l - 1) // 3
