@@ -29,7 +29,9 @@ def test_rows_are_cut_only_where_workgroups_are_few(split):
     for nl, B, Fi, fov, want in [(16, 32, 6, 25, 13), (16, 32, 25, 25, 25), (16, 32, 32, 25, 25), (24, 16, 32, 25, 25), (12, 4, 64, 64, 64), (32, 32, 6, 25, 25),
                                  (10, 32, 1, 5, 5), (5, 7, 8, 1, 4),
                                  # few pairs for each slice
-                                 (18, 2, 7, 37, 19), (9, 1, 20, 193, 49), (16, 1, 6, 25, 25), (22, 2, 4, 23, 23)]:
+                                 (18, 2, 7, 37, 19), (9, 1, 20, 193, 49), (16, 1, 6, 25, 25), (22, 2, 4, 23, 23),
+                                 # few pairs, but fewer workgroups than CUs
+                                 (3, 7, 5, 56, 14), (5, 3, 60, 51, 26)]:
         assert split(nl, B, Fi, fov)[0] == want, (nl, B, Fi, fov)
     for nl in range(1, 40):
         for B in (1, 2, 9, 32, 1000):
@@ -40,8 +42,9 @@ def test_rows_are_cut_only_where_workgroups_are_few(split):
                     tiles = -(-fov // lanes)
                     assert 4 <= lanes <= 64 and 1 <= slices and lanes * slices <= 256
                     assert slices == min(256 // lanes, -(-pairs // 4))              # four pairs for each
-                    if tiles > -(-fov // 64):             # cut further: too few workgroups with half the tiles, no slice under 9 lanes or five pairs
-                        assert nl * nl * passes * ((tiles + 1) // 2) < 1024 and lanes >= 9 and pairs // (256 // lanes) >= 5
+                    if tiles > -(-fov // 64):             # cut further: too few workgroups with half the tiles, no slice under 9 lanes, five pairs or idle CUs
+                        before = nl * nl * passes * ((tiles + 1) // 2)
+                        assert before < 1024 and lanes >= 9 and (before < 256 or pairs // (256 // lanes) >= 5)
 
 
 # (nl, B, Fi, Fo, elements by which gz starts beyond a boundary of 16 bytes)
